@@ -1,13 +1,13 @@
 // Direct-summation kernels for gfx950.
 //
-//  k_direct_f64   IEEE FP64, one target per lane, sources in ascending index order,
-//                 the operation order of gravhopper/_jbgrav.c:140-193 (self) and
-//                 :299-353 (targets), so the result is bit-identical to the reference.
-//                 Built with -ffp-contract=off; double '/' and sqrt are the compiler's
-//                 correctly rounded expansions.
-//  k_direct_f64_chain, k_direct_f64_spread  the same sums for up to 65536 targets:
-//                 a target's terms are computed by several lanes, then added in the
-//                 same order, so the results are the same bits.
+//  k_direct_f64_relay, k_direct_f64_ring  IEEE FP64, the operation order of
+//                 gravhopper/_jbgrav.c:140-193 (self) and :299-353 (targets) with every
+//                 sum formed in ascending source order, so the result is bit-identical to
+//                 the reference.  Built with -ffp-contract=off; the pair factor comes from
+//                 gh_pairf64.h, correctly rounded like the compiler's division and square
+//                 root.  The terms are computed by many wavefronts and added in order by
+//                 one: a wavefront of its own (relay, few targets) or each in its turn
+//                 (ring).
 //  k_direct_f32   FP32 pair forces with v_rsq_f32, IPT targets per lane, 256-source
 //                 tiles staged in LDS as float4 (x, y, z, m) and read as wave-wide
 //                 broadcasts, FP32 sums per tile and an FP32 two-sum (hi, lo) across
@@ -20,6 +20,7 @@
 #include <cmath>
 
 #include "gh_internal.h"
+#include "gh_pairf64.h"
 
 namespace gh {
 
@@ -28,247 +29,342 @@ int64_t pad_to(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 // ------------------------------------------------------------------------------
 // FP64, reference operation order
 // ------------------------------------------------------------------------------
-template <bool SELF>
-__global__ __launch_bounds__(kBlock) void k_direct_f64(const double4* __restrict__ src,
-                                                       int64_t np,
-                                                       const double* __restrict__ tgt,
-                                                       int64_t nt, double eps2,
-                                                       double* __restrict__ acc)
+// inv[u] = 1/d[u]/sqrt(d[u]) as the reference rounds it (:167; :327-331 with 0 for d = 0
+// when !SELF).  One range check covers the U values: a lane with any value outside
+// pair_factor's range takes the plain expressions for all of its own.
+template <bool SELF, int U>
+__device__ __forceinline__ void pair_factors(const double (&d)[U], double (&inv)[U])
 {
-    __shared__ double4 tile[kBlock];
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const bool live = i < nt;
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    if (live) {
-        xi = tgt[3 * i];
-        yi = tgt[3 * i + 1];
-        zi = tgt[3 * i + 2];
+    u32 hi = 0u, lo = 0u;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        hi = max(hi, (u32)__double2hiint(d[u]) - kPairLoHi);
+        lo = max(lo, (u32)__double2loint(d[u]));
+        inv[u] = pair_factor(d[u], __builtin_amdgcn_rsq(d[u]));
     }
-    double f0 = 0.0, f1 = 0.0, f2 = 0.0;
-    for (int64_t base = 0; base < np; base += kBlock) {
-        __syncthreads();
-        if (base + threadIdx.x < np) tile[threadIdx.x] = src[base + threadIdx.x];
-        __syncthreads();
-        const int cnt = (int)((np - base) < kBlock ? (np - base) : kBlock);
-        if (!live) continue;
-        for (int jj = 0; jj < cnt; jj++) {
-            const double4 s = tile[jj];
-            // dpos[i][j] = x_j - x_i (the reference stores -(x_i - x_j) or (x_j - x_i),
-            // which are the same IEEE value); d2 = ((0 + dx^2) + dy^2) + dz^2.
-            const double dx = s.x - xi, dy = s.y - yi, dz = s.z - zi;
-            double d2 = dx * dx;
-            d2 = d2 + dy * dy;
-            d2 = d2 + dz * dz;
-            const double d = d2 + eps2;
-            double inv;
-            if (SELF) {
-                inv = 1.0 / d / sqrt(d);
-            } else {
-                inv = (d == 0.0) ? 0.0 : 1.0 / d / sqrt(d);
-            }
-            const double c0 = s.w * dx * inv;
-            const double c1 = s.w * dy * inv;
-            const double c2 = s.w * dz * inv;
-            if (!SELF || base + jj != i) {
-                f0 = f0 + c0;
-                f1 = f1 + c1;
-                f2 = f2 + c2;
-            }
-        }
-    }
-    if (live) {
-        acc[3 * i] = f0;
-        acc[3 * i + 1] = f1;
-        acc[3 * i + 2] = f2;
+    if (__builtin_expect(hi >= kPairSpan || lo == kPairLowOnes, 0)) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            inv[u] = (!SELF && d[u] == 0.0) ? 0.0 : 1.0 / d[u] / sqrt(d[u]);
     }
 }
 
-// The same sums for few targets, when one lane per target would leave most of the GPU
-// idle (each lane's serial loop over all sources, with an IEEE division and square root
-// per pair, is then the whole run time).  TPW targets per wavefront, P = 64 / TPW lanes
-// per target: per chunk of P sources, the P lanes of a target compute one term each
-// (the same expressions as k_direct_f64), and the lanes then add the P terms in
-// ascending source order.  Every target's sum is formed term by term in the reference's
-// order, so the results are bit-identical to k_direct_f64's.
-template <bool SELF, int TPW>
-__global__ __launch_bounds__(kBlock) void k_direct_f64_spread(const double4* __restrict__ src,
-                                                              int64_t np,
-                                                              const double* __restrict__ tgt,
-                                                              int64_t nt, double eps2,
-                                                              double* __restrict__ acc)
+// A workgroup barrier that orders LDS accesses only: loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier()
 {
-    constexpr int P = 64 / TPW;
-    __shared__ double terms[kBlock / 64][3][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane / P, q = lane % P;  // target of this lane in the wave, source slot
-    const int64_t i = ((int64_t)blockIdx.x * (kBlock / 64) + wave) * TPW + g;
-    const bool live = i < nt;
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    if (live) {
-        xi = tgt[3 * i];
-        yi = tgt[3 * i + 1];
-        zi = tgt[3 * i + 2];
-    }
-    // one term of source j, computed without branches (the source index is clamped, and
-    // the term is +0.0 for a source past np or for the target itself); adding +0.0 to a
-    // sum that starts at +0.0 never changes it, so these terms leave the reference's
-    // sums untouched
-    auto term = [&](int64_t j, double& c0, double& c1, double& c2) {
-        const double4 s = src[j < np ? j : np - 1];
-        const double dx = s.x - xi, dy = s.y - yi, dz = s.z - zi;
-        double d2 = dx * dx;
-        d2 = d2 + dy * dy;
-        d2 = d2 + dz * dz;
-        const double d = d2 + eps2;
-        double inv;
-        if (SELF) {
-            inv = 1.0 / d / sqrt(d);
-        } else {
-            inv = (d == 0.0) ? 0.0 : 1.0 / d / sqrt(d);
-        }
-        const bool use = j < np && !(SELF && j == i);
-        c0 = use ? s.w * dx * inv : 0.0;
-        c1 = use ? s.w * dy * inv : 0.0;
-        c2 = use ? s.w * dz * inv : 0.0;
-    };
-    // Software pipelined: while a group adds the P terms of one chunk in source order,
-    // its lanes already compute the terms of the next chunk; both are in one branch-free
-    // block, so their dependent chains interleave.
-    double c0, c1, c2;
-    term(q, c0, c1, c2);
-    double f0 = 0.0, f1 = 0.0, f2 = 0.0;  // the sums (every lane of a group holds them)
-    const double* r0 = &terms[wave][0][g * P];
-    const double* r1 = &terms[wave][1][g * P];
-    const double* r2 = &terms[wave][2][g * P];
-    for (int64_t base = 0; base < np; base += P) {
-        terms[wave][0][lane] = c0;
-        terms[wave][1][lane] = c1;
-        terms[wave][2][lane] = c2;
-        __syncthreads();
-        term(base + P + q, c0, c1, c2);
-#pragma unroll
-        for (int k = 0; k < P; k++) {
-            f0 = f0 + r0[k];
-            f1 = f1 + r1[k];
-            f2 = f2 + r2[k];
-        }
-        __syncthreads();
-    }
-    if (live && q == 0) {
-        acc[3 * i] = f0;
-        acc[3 * i + 1] = f1;
-        acc[3 * i + 2] = f2;
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The same sums with a lane of its own for each sum.  A one-wavefront workgroup takes
-// TPW targets, whose 3 TPW component sums are held by lanes 0 .. 3 TPW - 1.  Per chunk
-// of 64 sources, lane l computes the terms of source base + l for every target (the
-// same expressions as k_direct_f64, +0.0 for the target itself and for sources past
-// np) into LDS; lane L then adds the 64 terms of its sum in source order.  Each pass
-// stores one chunk's terms, computes the next chunk's and adds the stored ones (two
-// LDS buffers; a single wavefront reads and writes LDS in program order, so one
-// barrier per chunk orders each buffer's writes after the reads two chunks earlier).
-template <bool SELF, int TPW>
-__global__ __launch_bounds__(64) void k_direct_f64_chain(const double* __restrict__ pos,
-                                                         const double* __restrict__ mass,
-                                                         int64_t np,
-                                                         const double* __restrict__ tgt,
-                                                         int64_t nt, double eps2,
-                                                         double* __restrict__ acc)
+// The same sums with the terms and the additions on different wavefronts.  A workgroup
+// takes T = P K targets: wavefronts 0 .. P - 1 compute the terms of chunks of 128 sources
+// (lane l sources 2l and 2l + 1 of the chunk, K targets each) into LDS, and wavefront P adds
+// them, lane L < 3 T holding one sum (a target's x, y or z) and adding its 128 terms in
+// source order.  While a chunk is added the next one's terms are computed (two LDS buffers,
+// one barrier per chunk), so a chunk costs the longer of the two, not both: the ordered
+// chain of additions (dependent FP64 adds, 9.8 cycles each) is the floor at few targets,
+// the FP64 issue rate of the terms at many.  The adding wavefront gets priority on its
+// SIMD, since the others wait for it.
+template <bool SELF, int P, int K>
+__global__ __launch_bounds__((P + 1) * 64) void k_direct_f64_relay(
+    const double* __restrict__ pos, const double* __restrict__ mass, int64_t np,
+    const double* __restrict__ tgt, int64_t nt, double eps2, double* __restrict__ acc)
 {
-    constexpr int NS = 3 * TPW;  // sums per wavefront
-    // T[b][k][L]: terms 2k and 2k + 1 of sum L in chunk buffer b
-    __shared__ double2 T[2][32][NS];
-    const int lane = threadIdx.x;
-    const int64_t i0 = (int64_t)blockIdx.x * TPW;
-    double xt[TPW], yt[TPW], zt[TPW];
+    constexpr int T = P * K, NS = 3 * T, CH = 128;
+    static_assert(NS <= 64, "one lane per sum");
+    // terms[b][l][L]: terms 2l and 2l + 1 of sum L in chunk buffer b; an odd row length
+    // spreads the rows over the LDS banks
+    constexpr int ROW = NS | 1;
+    __shared__ double2 terms[2][CH / 2][ROW];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t i0 = (int64_t)blockIdx.x * T;
+    // chunks are taken in pairs; one past the last adds zeros
+    const int64_t chunks = (np + 2 * CH - 1) / (2 * CH) * 2;
+    if (wave == P) {
+        __builtin_amdgcn_s_setprio(3);
+        const int L = lane < NS ? lane : NS - 1;
+        // a chunk's terms are read Q rows at a time into one of two sets of registers while
+        // the rows before are added from the other
+        constexpr int Q = 8;
+        double2 v[2][Q];
+        double f = 0.0;
 #pragma unroll
-    for (int t = 0; t < TPW; t++) {
+        for (int k = 0; k < Q; k++) v[1][k] = make_double2(0.0, 0.0);
+        for (int64_t c = 0; c < chunks; c++) {
+            lds_barrier();  // chunk c is in buffer c & 1
+            const double2* t = &terms[c & 1][0][L];
+#pragma unroll
+            for (int q = 0; q < CH / 2 / Q; q++) {
+#pragma unroll
+                for (int k = 0; k < Q; k++) v[q & 1][k] = t[(q * Q + k) * ROW];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < Q; k++) {
+                    f = f + v[(q + 1) & 1][k].x;
+                    f = f + v[(q + 1) & 1][k].y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < Q; k++) {
+            f = f + v[1][k].x;
+            f = f + v[1][k].y;
+        }
+        if (lane < NS && i0 + lane / 3 < nt) acc[3 * i0 + lane] = f;
+        return;
+    }
+    double xt[K], yt[K], zt[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
         // a target past nt takes the last target's position; its sums are not stored
-        const int64_t i = i0 + t < nt ? i0 + t : nt - 1;
-        xt[t] = tgt[3 * i];
-        yt[t] = tgt[3 * i + 1];
-        zt[t] = tgt[3 * i + 2];
+        const int64_t i = i0 + wave * K + k < nt ? i0 + wave * K + k : nt - 1;
+        xt[k] = tgt[3 * i];
+        yt[k] = tgt[3 * i + 1];
+        zt[k] = tgt[3 * i + 2];
     }
-    double c[TPW][3];
-    // sources are read in place from the (n,3) positions and the masses: the chunks
-    // are small, and a packing pass would cost a launch per force evaluation
-    auto terms = [&](int64_t base) {
-        const int64_t j = base + lane;
-        const int64_t jc = j < np ? j : np - 1;
-        const double sx = pos[3 * jc], sy = pos[3 * jc + 1], sz = pos[3 * jc + 2];
-        const double sw = mass[jc];
-#pragma unroll
-        for (int t = 0; t < TPW; t++) {
-            const double dx = sx - xt[t], dy = sy - yt[t], dz = sz - zt[t];
-            double d2 = dx * dx;
-            d2 = d2 + dy * dy;
-            d2 = d2 + dz * dz;
-            const double d = d2 + eps2;
-            double inv;
-            if (SELF) {
-                inv = 1.0 / d / sqrt(d);
-            } else {
-                inv = (d == 0.0) ? 0.0 : 1.0 / d / sqrt(d);
-            }
-            const bool use = j < np && !(SELF && j == i0 + t);
-            c[t][0] = use ? sw * dx * inv : 0.0;
-            c[t][1] = use ? sw * dy * inv : 0.0;
-            c[t][2] = use ? sw * dz * inv : 0.0;
-        }
+    // sources are read in place from the (n,3) positions and the masses, one chunk ahead
+    // (in two sets of registers, so that no copy waits for the loads)
+    struct Source {
+        double x[2], y[2], z[2], w[2];
     };
-    terms(0);
-    const int L = lane < NS ? lane : NS - 1;
-    double f = 0.0;
-    int b = 0;
-    for (int64_t base = 0; base < np; base += 64) {
-        double* w = reinterpret_cast<double*>(&T[b][lane >> 1][0]) + (lane & 1);
+    auto load = [&](int64_t base) {
+        const int64_t at = min(base, np - 1);
+        const int last = (int)min(np - 1 - at, (int64_t)(CH - 1));
+        const double* p = pos + 3 * at;
+        Source s;
 #pragma unroll
-        for (int t = 0; t < TPW; t++) {
-            w[2 * (3 * t)] = c[t][0];
-            w[2 * (3 * t + 1)] = c[t][1];
-            w[2 * (3 * t + 2)] = c[t][2];
+        for (int h = 0; h < 2; h++) {
+            const int l = min(2 * lane + h, last);
+            s.x[h] = p[3 * l];
+            s.y[h] = p[3 * l + 1];
+            s.z[h] = p[3 * l + 2];
+            s.w[h] = mass[at + l];
         }
-        __syncthreads();
-        terms(base + 64);
+        return s;
+    };
+    auto chunk = [&](int64_t base, const Source& s, int buf) {
+        double dx[2 * K], dy[2 * K], dz[2 * K], d[2 * K], inv[2 * K];
 #pragma unroll
-        for (int k = 0; k < 32; k++) {
-            const double2 v = T[b][k][L];
-            f = f + v.x;
-            f = f + v.y;
+        for (int k = 0; k < 2 * K; k++) {
+            dx[k] = s.x[k & 1] - xt[k >> 1];
+            dy[k] = s.y[k & 1] - yt[k >> 1];
+            dz[k] = s.z[k & 1] - zt[k >> 1];
+            double d2 = dx[k] * dx[k];
+            d2 = d2 + dy[k] * dy[k];
+            d2 = d2 + dz[k] * dz[k];
+            d[k] = d2 + eps2;
         }
-        b ^= 1;
+        pair_factors<SELF, 2 * K>(d, inv);
+        double2* o = &terms[buf][lane][3 * K * wave];
+        // the chunk holding the workgroup's own particles, and chunks past np
+        const bool masked = base + CH > np || (SELF && base < i0 + T && base + CH > i0);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            double c[3][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                c[0][h] = s.w[h] * dx[2 * k + h] * inv[2 * k + h];
+                c[1][h] = s.w[h] * dy[2 * k + h] * inv[2 * k + h];
+                c[2][h] = s.w[h] * dz[2 * k + h] * inv[2 * k + h];
+            }
+            if (masked) {
+                // +0.0 for the target itself and for sources past np: adding it leaves a
+                // sum that starts at +0.0 unchanged
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int64_t j = base + 2 * lane + h;
+                    const bool use = j < np && !(SELF && j == i0 + wave * K + k);
+#pragma unroll
+                    for (int a = 0; a < 3; a++) c[a][h] = use ? c[a][h] : 0.0;
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 3; a++) o[3 * k + a] = make_double2(c[a][0], c[a][1]);
+        }
+        lds_barrier();
+    };
+    Source a = load(0);
+    for (int64_t c = 0; c < chunks; c += 2) {
+        const Source b = load(CH * (c + 1));
+        chunk(CH * c, a, 0);
+        a = load(CH * (c + 2));
+        chunk(CH * (c + 1), b, 1);
     }
-    if (lane < NS && i0 + lane / 3 < nt) acc[3 * i0 + lane] = f;
 }
 
-// Kernel shape for the FP64 sums, as targets per wavefront: negative -v selects
-// k_direct_f64_chain with v targets, positive v k_direct_f64_spread with v targets
-// (64: k_direct_f64, one target per lane).  Automatic: the chain kernel up to
-// kF64ChainMax targets (1, 2 or 4 per wavefront by target count), then the spread
-// kernel up to kF64SpreadMax (2 to 16 targets, so that at most about kF64Waves
-// wavefronts run), then one target per lane.  Measured on Plummer spheres (kernel ms):
-//   targets per wavefront    chain 1/2/4/8/16          spread 1/2/4/8/16/32, plain
-//   N=2000                   0.034/0.032/0.040/0.062/0.14  0.071/0.064/0.086/0.13/0.25/0.43, 0.41
-//   N=16384                  1.31/1.02/0.99/1.52/2.23      3.43/1.95/1.36/1.26/1.99/3.50, 3.42
-//   N=65536                  18.6/14.4/13.8/17.0/26.9      48.3/27.8/19.0/15.7/13.6/16.5, 13.8
-//   N=262144                 -/-/208/254/393               plain 141
-constexpr int64_t kF64Waves = 2048;
-constexpr int64_t kF64ChainMax = 32768;
-constexpr int64_t kF64SpreadMax = 65536;
-static int f64_targets_per_wave(const gh_ctx* c, int64_t nt)
+// The value of lane l - 32 in lanes 32 .. 63 (lanes 0 .. 31 keep theirs).
+__device__ __forceinline__ double from_lower_half(double v)
 {
-    const int t = c->tune[GH_TUNE_DIRECT_F64_TPW];
-    if (t == 1 || t == 2 || t == 4 || t == 8 || t == 16 || t == 32 || t == 64) return t;
-    if (t == -1 || t == -2 || t == -4 || t == -8 || t == -16) return t;
-    if (nt <= 1024) return -1;
-    if (nt <= 4096) return -2;
-    if (nt <= kF64ChainMax) return -4;
-    if (nt > kF64SpreadMax) return 64;
-    int tpw = 2;
-    while (tpw < 16 && (int64_t)tpw * kF64Waves < nt) tpw *= 2;
-    return tpw;
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double(hi[0], lo[0]);
+}
+
+// The sources of each target spread over the wavefronts of a workgroup in turns.  A
+// workgroup takes 64 / H targets (H = 1 or 2 lanes per target); per turn a wavefront takes
+// the next H C sources, C per lane, computes their terms in registers, waits until the
+// sources before are added, adds its own in source order to the sums in LDS and passes the
+// turn on.  So every sum is formed in the reference's order while W wavefronts share its
+// arithmetic: W times as many wavefronts as one lane per target gives, which fills the
+// chip and evens out its last round.  The sources of a wavefront's next 64 / (H C) turns
+// are staged in LDS, loaded that many turns ahead.
+template <bool SELF, int W, int C, int H>
+__global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __restrict__ pos,
+                                                            const double* __restrict__ mass,
+                                                            int64_t np,
+                                                            const double* __restrict__ tgt,
+                                                            int64_t nt, double eps2,
+                                                            double* __restrict__ acc)
+{
+    constexpr int T = 64 / H, G = H * C, TURNS = 64 / G;
+    __shared__ double sums[3][T];
+    __shared__ int turn;
+    __shared__ double4 stage[W][2][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int t = lane % T, h = lane / T;
+    const int64_t i0 = (int64_t)blockIdx.x * T;
+    const int64_t i = i0 + t < nt ? i0 + t : nt - 1;  // past nt: computed, not stored
+    const double xi = tgt[3 * i], yi = tgt[3 * i + 1], zi = tgt[3 * i + 2];
+    if (threadIdx.x < T) sums[0][t] = sums[1][t] = sums[2][t] = 0.0;
+    if (threadIdx.x == 0) turn = 0;
+    __syncthreads();
+    // group g (G sources from g G on) is wavefront (g mod W)'s; its turns come in blocks of
+    // TURNS, lane l loading source l % G of turn l / G
+    const int groups = (int)((np + G - 1) / G);
+    auto load = [&](int g) {
+        const int64_t at = ((int64_t)g + (int64_t)(lane / G) * W) * G + lane % G;
+        const int64_t j = at < np ? at : np - 1;
+        return make_double4(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], mass[j]);
+    };
+    double4 next = load(wave);
+    int buf = 0;
+    for (int g0 = wave; g0 < groups; g0 += W * TURNS, buf ^= 1) {
+        stage[wave][buf][lane] = next;
+        next = load(g0 + W * TURNS);
+        __builtin_amdgcn_wave_barrier();
+        for (int k = 0; k < TURNS; k++) {
+            const int g = g0 + k * W;
+            if (g >= groups) break;
+            const int64_t base = (int64_t)g * G;
+            const double4* s = &stage[wave][buf][k * G + h * C];
+            double dx[C], dy[C], dz[C];
+            // four sources at a time keep the FP64 pipe full; more only cost registers
+#pragma unroll
+            for (int u0 = 0; u0 < C; u0 += 4) {
+                double w[4], d[4], inv[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const double4 q = s[u0 + u];
+                    dx[u0 + u] = q.x - xi;
+                    dy[u0 + u] = q.y - yi;
+                    dz[u0 + u] = q.z - zi;
+                    w[u] = q.w;
+                    double d2 = dx[u0 + u] * dx[u0 + u];
+                    d2 = d2 + dy[u0 + u] * dy[u0 + u];
+                    d2 = d2 + dz[u0 + u] * dz[u0 + u];
+                    d[u] = d2 + eps2;
+                }
+                pair_factors<SELF, 4>(d, inv);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    dx[u0 + u] = w[u] * dx[u0 + u] * inv[u];
+                    dy[u0 + u] = w[u] * dy[u0 + u] * inv[u];
+                    dz[u0 + u] = w[u] * dz[u0 + u] * inv[u];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (base + G > np || (SELF && base < i0 + T && base + G > i0)) {
+                // +0.0 for the target itself and for sources past np: adding it leaves a
+                // sum that starts at +0.0 unchanged
+#pragma unroll
+                for (int u = 0; u < C; u++) {
+                    const int64_t j = base + h * C + u;
+                    const bool use = j < np && !(SELF && j == i0 + t);
+                    dx[u] = use ? dx[u] : 0.0;
+                    dy[u] = use ? dy[u] : 0.0;
+                    dz[u] = use ? dz[u] : 0.0;
+                }
+            }
+            // every wavefront of the workgroup is resident and passes each of its turns on,
+            // so this ends
+            while (__hip_atomic_load(&turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != g)
+                __builtin_amdgcn_s_sleep(1);
+            __builtin_amdgcn_s_setprio(3);
+            double f0 = sums[0][t], f1 = sums[1][t], f2 = sums[2][t];
+#pragma unroll
+            for (int p = 0; p < H; p++) {
+                if (p > 0) {
+                    f0 = from_lower_half(f0);
+                    f1 = from_lower_half(f1);
+                    f2 = from_lower_half(f2);
+                }
+#pragma unroll
+                for (int u = 0; u < C; u++) {
+                    f0 = f0 + dx[u];
+                    f1 = f1 + dy[u];
+                    f2 = f2 + dz[u];
+                }
+            }
+            if (h == H - 1) {
+                sums[0][t] = f0;
+                sums[1][t] = f1;
+                sums[2][t] = f2;
+            }
+            asm volatile("" ::: "memory");
+            if (lane == 0)
+                __hip_atomic_store(&turn, g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __builtin_amdgcn_s_setprio(0);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < T && i0 + t < nt) {
+        acc[3 * i] = sums[0][t];
+        acc[3 * i + 1] = sums[1][t];
+        acc[3 * i + 2] = sums[2][t];
+    }
+}
+
+// Kernel shape for the FP64 sums.  Up to kF64RelayMax targets k_direct_f64_relay: the chain
+// of ordered additions is what bounds it, so the fewest wavefronts that keep up with it, and
+// as many targets per workgroup as give each CU one workgroup.  Beyond, k_direct_f64_ring:
+// the issue rate of the terms bounds it, and the shape decides how evenly the wavefronts
+// fill the CUs: two lanes per target (32 targets per workgroup) until 64 targets per
+// workgroup give every CU one, eight wavefronts per workgroup until there are two
+// workgroups per CU.  Measured on Plummer spheres, us per evaluation (the best of the other
+// family beside it; "before" is one or few targets per wavefront, with the compiler's
+// division and square root):
+//   N        500  1000  2000  4000  6000 | 8000  12000  16384  20000  32768  65536  100003  262144
+//   relay    7.3  10.0  17.9  41.2  80.7 |  141    289    529    817   2063
+//   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   91367
+//   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
+// 3001 targets of 65536 sources: 468 (before 1300); 200 of 100000: 393 (1062).
+constexpr int64_t kF64RelayMax = 6500;
+
+enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
+struct F64Shape {
+    int targets;  // relay: per workgroup
+    F64Ring ring;
+};
+static F64Shape f64_shape(const gh_ctx* c, int64_t nt)
+{
+    const int tune = c->tune[GH_TUNE_DIRECT_F64_TPW];
+    const bool relay = tune < 0 || (tune == 0 && nt <= kF64RelayMax);
+    if (relay) {
+        int64_t t = tune < 0 ? -(int64_t)tune : 0;
+        if (tune == 0)
+            t = nt <= 256 ? 1 : nt <= 768 ? 3 : nt <= 1024 ? 4 : nt <= 2048 ? 8
+                : nt <= 3072 ? 12 : nt <= 4096 ? 16 : 6;
+        for (int has : {1, 3, 4, 6, 8, 12})
+            if (t <= has) return {has, F64Ring::none};
+        return {16, F64Ring::none};
+    }
+    const bool one_lane = tune ? tune >= 64 : (nt > 8192 && nt <= 16384) || nt > 24576;
+    if (nt <= 16384) return {0, one_lane ? F64Ring::w8_h1 : F64Ring::w8_h2};
+    return {0, one_lane ? F64Ring::w4_h1 : F64Ring::w4_h2};
 }
 
 // ------------------------------------------------------------------------------
@@ -819,6 +915,35 @@ F32Shape pick_shape(gh_ctx* c, int64_t nt, int64_t np_pad)
     return sh;
 }
 
+template <int P, int K>
+void launch_relay(bool self, const double* pos, const double* mass, int64_t np, const double* tgt,
+                  int64_t nt, double eps2, double* acc, hipStream_t s)
+{
+    const dim3 grid((unsigned)((nt + P * K - 1) / (P * K))), block((P + 1) * 64);
+    if (self)
+        hipLaunchKernelGGL((k_direct_f64_relay<true, P, K>), grid, block, 0, s, pos, mass, np,
+                           tgt, nt, eps2, acc);
+    else
+        hipLaunchKernelGGL((k_direct_f64_relay<false, P, K>), grid, block, 0, s, pos, mass, np,
+                           tgt, nt, eps2, acc);
+}
+
+template <int W, int H>
+void launch_ring(bool self, const double* pos, const double* mass, int64_t np, const double* tgt,
+                 int64_t nt, double eps2, double* acc, hipStream_t s)
+{
+    // 16 sources per lane and turn: passing the turn on takes about 390 cycles, the terms
+    // of 8 sources 1900 (N = 16384: 433 us with 8, 398 with 16)
+    constexpr int C = 16;
+    const dim3 grid(blocks_for(nt, 64 / H)), block(64 * W);
+    if (self)
+        hipLaunchKernelGGL((k_direct_f64_ring<true, W, C, H>), grid, block, 0, s, pos, mass, np,
+                           tgt, nt, eps2, acc);
+    else
+        hipLaunchKernelGGL((k_direct_f64_ring<false, W, C, H>), grid, block, 0, s, pos, mass, np,
+                           tgt, nt, eps2, acc);
+}
+
 template <int IPT, bool DS>
 void launch_f32(bool guard, dim3 grid, hipStream_t s, const double4* src64, int64_t np_pad,
                 int64_t jps, const OrderBufs& t, int64_t nt, float eps2, double* out)
@@ -1074,65 +1199,34 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     }
     if (precision == GH_FP64) {
         const double eps2 = eps * eps;
-        const int tpw = f64_targets_per_wave(c, nt);
-        if (tpw < 0) {
+        const F64Shape sh = f64_shape(c, nt);
+        if (sh.ring == F64Ring::none) {
             TimedScope ts(c, s, GH_T_DIRECT_F64);
-            const int tc = -tpw;
-            const dim3 gc((unsigned)((nt + tc - 1) / tc));
-#define GH_CHAIN(T)                                                                       \
-    do {                                                                                  \
-        if (self)                                                                         \
-            hipLaunchKernelGGL((k_direct_f64_chain<true, T>), gc, dim3(64), 0, s,         \
-                               d_pos, d_mass, np, tgt, nt, eps2, d_acc);                  \
-        else                                                                              \
-            hipLaunchKernelGGL((k_direct_f64_chain<false, T>), gc, dim3(64), 0, s,        \
-                               d_pos, d_mass, np, tgt, nt, eps2, d_acc);                  \
-    } while (0)
-            switch (tc) {
-            case 1: GH_CHAIN(1); break;
-            case 2: GH_CHAIN(2); break;
-            case 4: GH_CHAIN(4); break;
-            case 8: GH_CHAIN(8); break;
-            default: GH_CHAIN(16); break;
+            switch (sh.targets) {
+            case 1: launch_relay<1, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 3: launch_relay<3, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 4: launch_relay<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 6: launch_relay<3, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 8: launch_relay<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 12: launch_relay<6, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            default: launch_relay<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
             }
-#undef GH_CHAIN
-            return check_launch(c, "k_direct_f64_chain");
+            return check_launch(c, "k_direct_f64_relay");
         }
-        GH_TRY(ensure(c, c->src64, sizeof(double4) * (size_t)np));
-        double4* src = c->src64.as<double4>();
-        hipLaunchKernelGGL(k_pack_src64, dim3(blocks_for(np, kBlock)), dim3(kBlock), 0, s,
-                           d_pos, d_mass, np, np, src);
-        GH_TRY(check_launch(c, "k_pack_src64"));
         TimedScope ts(c, s, GH_T_DIRECT_F64);
-        if (tpw == 64) {
-            if (self)
-                hipLaunchKernelGGL(k_direct_f64<true>, dim3(blocks_for(nt, kBlock)),
-                                   dim3(kBlock), 0, s, src, np, tgt, nt, eps2, d_acc);
-            else
-                hipLaunchKernelGGL(k_direct_f64<false>, dim3(blocks_for(nt, kBlock)),
-                                   dim3(kBlock), 0, s, src, np, tgt, nt, eps2, d_acc);
-            return check_launch(c, "k_direct_f64");
+        switch (sh.ring) {
+        case F64Ring::w8_h2:
+            launch_ring<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
+            break;
+        case F64Ring::w8_h1:
+            launch_ring<8, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
+            break;
+        case F64Ring::w4_h2:
+            launch_ring<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
+            break;
+        default: launch_ring<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
         }
-        const dim3 grid(blocks_for((nt + tpw - 1) / tpw, kBlock / 64));
-#define GH_SPREAD(T)                                                                      \
-    do {                                                                                  \
-        if (self)                                                                         \
-            hipLaunchKernelGGL((k_direct_f64_spread<true, T>), grid, dim3(kBlock), 0, s,  \
-                               src, np, tgt, nt, eps2, d_acc);                            \
-        else                                                                              \
-            hipLaunchKernelGGL((k_direct_f64_spread<false, T>), grid, dim3(kBlock), 0, s, \
-                               src, np, tgt, nt, eps2, d_acc);                            \
-    } while (0)
-        switch (tpw) {
-        case 1: GH_SPREAD(1); break;
-        case 2: GH_SPREAD(2); break;
-        case 4: GH_SPREAD(4); break;
-        case 8: GH_SPREAD(8); break;
-        case 16: GH_SPREAD(16); break;
-        default: GH_SPREAD(32); break;
-        }
-#undef GH_SPREAD
-        return check_launch(c, "k_direct_f64_spread");
+        return check_launch(c, "k_direct_f64_ring");
     }
     if (precision != GH_FP32) return fail(c, GH_EARG, "unknown precision %d", precision);
     const int sym = self ? sym_ipt(c, np) : 0;

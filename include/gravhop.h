@@ -227,12 +227,11 @@ int gh_timing_read(gh_ctx *ctx, int kernel_class, double *total_ms, int64_t *lau
  *                        one HIP graph (from 4 steps on), -1 launch every kernel eagerly
  *   GH_TUNE_WALK_F64EVAL FP32 tree walk: 1 evaluates the same interaction lists in FP64
  *                        (a check of the FP32 arithmetic), 0 FP32
- *   GH_TUNE_DIRECT_F64_TPW  FP64 direct sum: 0 automatic, 1/2/4/8/16/32/64 targets per
- *                        wavefront (64: one target per lane; fewer: the terms of a
- *                        target are computed by 64/value lanes and then added in order),
- *                        -1/-2/-4/-8/-16: that many targets per wavefront, every lane
- *                        computing one source's terms for all of them and each of the
- *                        3 x targets sums added in order by a lane of its own
+ *   GH_TUNE_DIRECT_F64_TPW  FP64 direct sum: 0 automatic; v > 0 the wavefronts of a
+ *                        workgroup add their terms to its targets' sums in turns, with
+ *                        64 targets per workgroup for v >= 64 and 32 below; -v < 0 one
+ *                        wavefront adds the others' terms, with v targets per workgroup
+ *                        (rounded up to 1, 3, 4, 6, 8, 12 or 16)
  *   GH_TUNE_ALLOC_LIMIT_MB  cap, in MiB, on the device memory the context's arenas may
  *                        hold (0: no cap); a call that would exceed it fails with
  *                        GH_ENOMEM and leaves the context usable

@@ -208,3 +208,52 @@ def test_fp32_sort_forms_agree(ctx, n):
         ref = ctx.direct(pos, ic["mass"], 1e-5, FP64)
         e = rel_err(got, ref)
         assert np.median(e) <= FP32_MEDIAN and np.percentile(e, 99) <= FP32_P99
+
+
+# either side of every change of kernel shape (f64_shape in gh_direct.hip)
+@pytest.mark.parametrize("nf", [1, 256, 257, 768, 769, 1024, 1025, 2048, 2049, 3072, 3073, 4096,
+                                4097, 6500, 6501, 8192, 8193, 16384, 16385, 24576, 24577])
+def test_fp64_direct_shape_edges_bitwise(ctx, oracle, nf):
+    rng = np.random.default_rng(nf)
+    fpos = rng.standard_cauchy(size=(nf, 3))
+    # source counts around the chunks of 128 and 256 and the turns of 16 and 32
+    for n in (1, 15, 17, 33, 127, 129, 257):
+        pos = rng.standard_cauchy(size=(n, 3))
+        pos[: min(n, nf) // 2] = fpos[: min(n, nf) // 2]  # coincident pairs
+        mass = rng.uniform(0.1, 3.0, size=n)
+        for eps in (0.0, 1e-3):
+            assert_bitwise(ctx.direct(pos, mass, eps, FP64, force_pos=fpos),
+                           oracle.direct_position(pos, mass, fpos, eps), "%d sources" % n)
+
+
+@pytest.mark.parametrize("n", [2049, 6501, 8193, 16385, 24577, 33000])
+def test_fp64_direct_self_shape_edges_bitwise(ctx, oracle, n):
+    rng = np.random.default_rng(n)
+    pos = rng.standard_cauchy(size=(n, 3))
+    mass = rng.uniform(0.1, 3.0, size=n)
+    # with eps > 0 a particle's own term is +-0 and leaves its sum as it is
+    some = np.unique(np.concatenate([[0, 31, 32, 63, 64, n - 2, n - 1],
+                                     rng.integers(0, n, size=300)]))
+    assert_bitwise(ctx.direct(pos, mass, 1e-3, FP64)[some],
+                   oracle.direct_position(pos, mass, pos[some], 1e-3))
+
+
+@pytest.mark.parametrize("nf", [5, 900, 7000, 20000])
+def test_fp64_direct_operand_range_bitwise(ctx, oracle, nf):
+    """Squared separations below, inside and above the pair factor's range (2^-500 to 2^501),
+    zero and overflowing ones among them, mixed in the lanes of a wavefront."""
+    rng = np.random.default_rng(nf)
+    n = 150
+    scale = 10.0 ** rng.choice([-170.0, -76.0, -75.0, -3.0, 0.0, 75.0, 76.0, 150.0, 160.0],
+                               size=n)
+    pos = rng.normal(size=(n, 3)) * scale[:, None]
+    mass = rng.uniform(0.1, 3.0, size=n)
+    fpos = rng.normal(size=(nf, 3)) * 10.0 ** rng.choice([-170.0, -3.0, 76.0], size=nf)[:, None]
+    fpos[::7] = pos[rng.integers(0, n, size=len(fpos[::7]))]
+    for eps in (0.0, 1e-3):
+        with np.errstate(all="ignore"):
+            want = oracle.direct_position(pos, mass, fpos, eps)
+        got = ctx.direct(pos, mass, eps, FP64, force_pos=fpos)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        assert_bitwise(got[ok], want[ok], "eps=%g" % eps)
