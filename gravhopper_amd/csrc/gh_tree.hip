@@ -31,17 +31,15 @@
 //                     end+1
 //   6. moments        node mass and first moment as differences of double-double prefix
 //                     sums over the sorted particles (error far below one FP64 ulp)
-//   7. walks          FP64: stackless pre-order walk with skip pointers.  A wavefront
-//                     walks up to 64 targets in lockstep: the wave visits nodes in
-//                     increasing order (next = n+1 if any waiting lane opened n, else
-//                     skip[n]); a lane waits for every node from the end of the last
-//                     subtree it accepted on, so each lane accepts exactly the nodes the
-//                     reference's recursive walk (:487-541) accepts, while the node index
-//                     stays wave-uniform and node records arrive through scalar loads.
+//   7. walks          FP64: a wavefront walks 1 to 64 targets together, 64 nodes per step
+//                     from an ordered stack that keeps which targets reach each node; each
+//                     target accepts exactly the nodes the reference's recursive walk
+//                     (:487-541) accepts and adds them in its order (k_walk_f64).
 //                     FP32: a group walk with one interaction list per 16 targets whose
 //                     lists refine the reference's accepted nodes (k_walk_group).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "gh_box.h"
 #include "gh_internal.h"
@@ -91,6 +89,7 @@ struct TreeBufs {
     DevBuf tkeys[2], tidx[2];  // Morton order of position targets (tree_force_position)
     long long* readback = nullptr;  // pinned host words: flags[0..1], node count, flags[2]
     long long* readback_dev = nullptr;  // the same words' device address
+    const int* kids_f64 = nullptr;  // children lists of the last FP64 build
     int64_t n_nodes = 0;
     int words = 0;
     int key_sel = 0;  // which of keys[0]/keys[1] holds the sorted keys
@@ -1010,13 +1009,12 @@ __global__ __launch_bounds__(kFillBlock) void k_fill_nodes(FillArgs a, int64_t n
 // Scheduling (both walks).  Workgroups are dealt to the 8 XCDs round-robin (workgroup
 // b runs on XCD b mod 8); xcd_block() renumbers them so that XCD x takes the x-th of 8
 // contiguous, Morton-ordered ranges of walk units, and the L2 of XCD x holds the nodes
-// of one region of the tree.  The FP64 walk runs one wavefront per workgroup, so that the
-// hardware refills a SIMD slot as soon as its walk ends rather than when the slowest of
-// several does; the FP32 group walk runs two independent ones per workgroup (below).
+// of one region of the tree.  Both walks run two independent wavefronts per workgroup, as
+// a CU holds at most 16 workgroups.
 constexpr int kXcds = 8;
-constexpr int64_t kWalkUnits = 4096;  // walks in flight for small target counts
+constexpr int64_t kWalkUnits = 4096;  // FP32 walks in flight for small target counts
+constexpr int64_t kWalks64 = 2560;    // FP64 walks in flight: 10 per CU
 constexpr int64_t kSortTargetsMin = 4096;  // position targets sorted from this many on
-constexpr int kWalkBlock = 64;
 __device__ __forceinline__ int64_t xcd_block(int64_t per_xcd)
 {
     return (int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
@@ -1682,106 +1680,395 @@ __global__ __launch_bounds__(kBlock) void k_kids(const int* __restrict__ skip, i
 //    theta <= 0: nothing is accepted, as size/dist < theta never holds).
 //  - Leaves are accepted without the test (:502).
 //  - Monopole (:506-524): inv = (1/d)/sqrt(d), d = |com - x|^2 + eps^2, 0 if d == 0, here
-//    as r^3 with r = 1/sqrt(d) from v_rsq_f64 and one Newton step.  Measured on gfx950
-//    over 2^20 values of d in [1e-30, 1e30] and [1, 4): v_rsq_f64 alone is within
-//    2.5e8 ulp, one step within 19.4 ulp (4e-15), two within 1.7 ulp.  One step is far
-//    inside the FP64 walk's tolerance against the reference (1e-10), which moment
-//    rounding and summation order set anyway, and 4 % faster than two.
+//    as r^3 (1 - e)^(-3/2) with r = v_rsq_f64(d), e = 1 - d r^2 and the power to second
+//    order.  v_rsq_f64 is within a relative 2^-24.6 (measured over 2^20 values of d in
+//    [1e-30, 1e30] and [1, 4)), so the third order is below 2^-69 and what is left are the
+//    few roundings, far inside the walk's tolerance against the reference (1e-10), which
+//    moment rounding and summation order set anyway.  (One Newton step on r and then its
+//    cube takes as many operations and is off by up to 1.3e-14.)
+//
+// A wavefront walks T consecutive targets (Morton order, T a power of two; lane l holds
+// target l mod T).  Every target accepts exactly the nodes the reference accepts for it
+// and sums them in the reference's (pre-order) order, so its result does not depend on the
+// other targets of its walk.
+//
+// Traversal, in order but 64 nodes at a time: an LDS stack of (node, mask of the targets
+// that reach it), its top the first in pre-order.  A step pops up to 64 entries, one per
+// lane, and tests the pending ones: against the targets' box first (far from all of it:
+// accepted by every target, near to all of it: opened by every one), against each target
+// where that does not decide (S = 64 / T nodes per pass, lane l testing node l / T for its
+// target).  A node some targets accept and others open stays, accepted for the first, with
+// its children behind it for the others.  The leading accepted entries go to the list, and
+// the rest goes back on the stack in order, accepted ones marked as such.  A walk of 64
+// targets of the N = 2^20 galaxy (theta = 0.7) visits 1499 nodes in 51 steps, one of 16
+// visits 1086 in 38; one node at a time, the walk was a chain of 1494 dependent loads (458
+// us for 40001 targets, 700 us for 20011, whatever was left of the GPU idle).
+//
+// Evaluation, 64 list entries at a time: with T = 64 every lane adds the entries to its
+// target's sum in turn; with fewer targets the lanes compute the terms of 64 / T entries at
+// once into LDS, and one lane per sum adds them in order (+0.0 where the target did not
+// accept the entry, which changes no sum, as none is ever -0).
+//
+// A step pops only as many entries as leave room for what goes back; where that is none,
+// the top entry's subtree is walked one node at a time with the skip pointers.
 // COUNT: counts receives the accepted-node count per target.
-__device__ __forceinline__ double rsqrt_f64(double d)
+__device__ __forceinline__ double inv_d15(double d, double c15)
 {
     const double r = __builtin_amdgcn_rsq(d);
-    return r * __builtin_fma(-0.5 * d, r * r, 1.5);
+    const double u = r * r;
+    const double e = __builtin_fma(-d, u, 1.0);  // d = (1 - e) / r^2
+    const double w = r * u;
+    return __builtin_fma(w, e * __builtin_fma(e, 1.875, c15), w);
 }
 
-template <bool COUNT>
-__global__ __launch_bounds__(kBlock) void k_walk_f64(const NodeD* __restrict__ nodes,
-                                                     const int* __restrict__ skip,
-                                                     int64_t n_nodes,
-                                                     const double* __restrict__ tgt,
-                                                     const double4* __restrict__ stgt,
-                                                     const u32* __restrict__ order, int64_t nt,
-                                                     double eps, double theta, double c_lo,
-                                                     double c_hi, double* __restrict__ acc,
-                                                     int* __restrict__ counts,
-                                                     int64_t per_xcd, int lanes)
+// Wavefronts per workgroup, each with a walk of its own.
+constexpr int kWalkWaves = 2;
+constexpr int kWalkDone = (int)0x80000000;  // marks an accepted entry on the stack
+
+template <int T>
+struct WalkMask {
+    typedef u32 M;
+};
+template <>
+struct WalkMask<64> {
+    typedef u64 M;
+};
+
+// CAP: stack entries of a walk.
+template <int T, bool COUNT, int CAP>
+__global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __restrict__ nodes,
+                                                 const int* __restrict__ kids,
+                                                 const int* __restrict__ skip, int n_nodes,
+                                                 const double* __restrict__ tgt,
+                                                 const double4* __restrict__ stgt,
+                                                 const u32* __restrict__ order, int64_t nt,
+                                                 double eps2, double theta, double c_lo,
+                                                 double c_hi, double* __restrict__ acc,
+                                                 int* __restrict__ counts, int64_t per_xcd)
 {
-    // one walk of `lanes` consecutive targets per wavefront (lanes <= 64)
+    typedef typename WalkMask<T>::M Mask;
+    constexpr int S = 64 / T;                  // lanes per target
+    constexpr int U = T < 4 ? T : 4;           // terms per lane and round (T < 64)
+    constexpr int B = S * U;                   // entries per round
+    constexpr int NS = 3 * T, ROW = NS | 1;    // sums; LDS row length of their terms
+    static_assert(T == 64 || NS <= 64, "one lane per sum");
+    struct Shared {
+        double4 stage[64];  // the nodes of the per-target tests; the entries evaluated
+        double2 terms[T < 64 ? B / 2 : 1][T < 64 ? ROW : 1];
+        Mask masks[CAP], lmask[128];
+        int ids[CAP], lid[128];
+    };
+    __shared__ Shared shared[kWalkWaves];
     const int lane = threadIdx.x & 63;
-    const int64_t first = (xcd_block(per_xcd) * (kWalkBlock / 64) + (threadIdx.x >> 6)) * lanes;
-    if (first >= nt) return;  // whole wavefront idle
-    const int64_t k = first + lane;
-    const bool live = lane < lanes && k < nt;
-    int64_t t = 0;
-    double x = 0.0, y = 0.0, z = 0.0;
-    if (live) {
-        t = order ? (int64_t)order[k] : k;
-        if (stgt) {  // self walk: the particles in walk order, read contiguously
-            const double4 q = stgt[k];
-            x = q.x;
-            y = q.y;
-            z = q.z;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    auto& stage = shared[wave].stage;
+    auto& terms = shared[wave].terms;
+    auto& lmask = shared[wave].lmask;
+    auto& lid = shared[wave].lid;
+    auto& masks = shared[wave].masks;
+    auto& ids = shared[wave].ids;
+    const int t = lane % T, slice = lane / T;
+    const int64_t first = (xcd_block(per_xcd) * kWalkWaves + wave) * T;
+    if (first >= nt) return;
+    const int cnt = (int)(nt - first < T ? nt - first : T);
+    const Mask all = (Mask)(cnt == 64 ? ~0ull : (1ull << cnt) - 1ull);
+    const Mask own = (Mask)1 << t;
+    // this lane's target (past the count: the last one, in no mask)
+    const int64_t k = first + (t < cnt ? t : cnt - 1);
+    const int64_t ti = order ? (int64_t)order[k] : k;
+    double x, y, z;
+    if (stgt) {  // self walk: the particles in walk order, read contiguously
+        const double4 q = stgt[k];
+        x = q.x, y = q.y, z = q.z;
+    } else {
+        x = tgt[3 * ti], y = tgt[3 * ti + 1], z = tgt[3 * ti + 2];
+    }
+    // the targets' box; a target that is not finite leaves every node to the per-target tests
+    double lox = x, loy = y, loz = z, hix = x, hiy = y, hiz = z;
+    for (int o = 1; o < T; o <<= 1) {
+        lox = fmin(lox, __shfl_xor(lox, o)), hix = fmax(hix, __shfl_xor(hix, o));
+        loy = fmin(loy, __shfl_xor(loy, o)), hiy = fmax(hiy, __shfl_xor(hiy, o));
+        loz = fmin(loz, __shfl_xor(loz, o)), hiz = fmax(hiz, __shfl_xor(hiz, o));
+    }
+    double bcx = 0.5 * (lox + hix), bcy = 0.5 * (loy + hiy), bcz = 0.5 * (loz + hiz);
+    const double bhx = 0.5 * (hix - lox), bhy = 0.5 * (hiy - loy), bhz = 0.5 * (hiz - loz);
+    if (__ballot(!(isfinite(x) && isfinite(y) && isfinite(z))) != 0) bcx = __builtin_nan("");
+    // bounds on the box's squared distances; the margin covers their rounding
+    const double box_hi = c_hi * (1.0 + 1e-12), box_lo = c_lo * (1.0 - 1e-12);
+
+    double ax = 0.0, ay = 0.0, az = 0.0;  // T = 64: the lane's target's sums
+    double f = 0.0;                       // T < 64: sum lane (3 t + component)
+    int accepted = 0;
+    int held = 0;  // entries in the list
+    double c15 = 1.5;  // in a register: as a literal it would be copied for every entry
+    asm("" : "+v"(c15));
+
+    // m / d^(3/2) of this lane's target and the monopole q, 0 unless use; dx, dy, dz: q - x
+    auto monopole = [&](const double4& q, bool use, bool guard, double& dx, double& dy,
+                        double& dz) {
+        dx = q.x - x, dy = q.y - y, dz = q.z - z;
+        const double d = __builtin_fma(dz, dz, __builtin_fma(dy, dy, __builtin_fma(dx, dx, eps2)));
+        double mi = q.w * inv_d15(d, c15);
+        // opaque, so that it is computed whatever `use` is: a branch around it would keep
+        // the terms of several entries from overlapping
+        asm("" : "+v"(mi));
+        if (guard) use = use && d != 0.0;
+        return use ? mi : 0.0;
+    };
+    // the test of the reference, for this lane's target
+    auto passes = [&](double cx, double cy, double cz, double size) {
+        const double ddx = cx - x, ddy = cy - y, ddz = cz - z;
+        double d2 = ddx * ddx;
+        d2 = d2 + ddy * ddy;
+        d2 = d2 + ddz * ddz;
+        const double s2 = size * size;
+        bool far = d2 > s2 * c_hi;
+        const bool unsure = !far && !(d2 < s2 * c_lo);
+        if (__ballot(unsure) != 0) {
+            if (unsure) far = (size / sqrt(d2)) < theta;
+        }
+        return far;
+    };
+    // Takes the first `have` (<= 64) list entries off the list, lane l entry l, and loads
+    // their monopoles; evaluate() uses them a traversal step later, which hides the loads.
+    int have = 0;
+    Mask m_have = 0;
+    double2 q0, q1;
+    auto fetch = [&]() {
+        have = held < 64 ? held : 64;
+        const bool mine = lane < have;
+        m_have = mine ? lmask[lane] : (Mask)0;
+        const double2* rec = (const double2*)(nodes + (mine ? lid[lane] : 0)) + 2;
+        q0 = rec[0], q1 = rec[1];
+        held -= have;
+        const int id = lid[64 + lane];
+        const Mask m = lmask[64 + lane];
+        wave_sync();
+        if (lane < held) {
+            lid[lane] = id;
+            lmask[lane] = m;
+        }
+        wave_sync();
+    };
+    auto evaluate_as = [&](auto guarded) {
+        constexpr bool guard = decltype(guarded)::value;
+        stage[lane] = make_double4(q0.x, q0.y, q1.x, q1.y);
+        wave_sync();
+        if constexpr (T == 64) {
+            for (int e0 = 0; e0 < have; e0 += 4) {
+                double dx[4], dy[4], dz[4], mi[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const u64 em =
+                        ((u64)(u32)__builtin_amdgcn_readlane((int)(m_have >> 32), e0 + e) << 32) |
+                        (u32)__builtin_amdgcn_readlane((int)m_have, e0 + e);
+                    const bool use = __builtin_amdgcn_inverse_ballot_w64(em);
+                    mi[e] = monopole(stage[e0 + e], use, guard, dx[e], dy[e], dz[e]);
+                    if (COUNT) accepted += use ? 1 : 0;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    // product and sum rounded apart, as with fewer targets (below)
+                    ax = ax + dx[e] * mi[e];
+                    ay = ay + dy[e] * mi[e];
+                    az = az + dz[e] * mi[e];
+                }
+            }
         } else {
-            x = tgt[3 * t];
-            y = tgt[3 * t + 1];
-            z = tgt[3 * t + 2];
-        }
-    }
-    const double eps2 = eps * eps;
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    int cnt = 0;
-    int my_skip = live ? 0 : 0x7fffffff;  // waiting iff node >= my_skip
-    const int n_nodes32 = (int)n_nodes;  // below 2^31 (checked by the build)
-    int node = 0;
-    while (node < n_nodes32) {
-        // the whole record (one 64-byte scalar load) and the skip pointer, issued
-        // together; a leaf's size has its sign bit set
-        const f64x8 nd = *(const f64x8*)(nodes + node);
-        const int sk = skip[node];
-        const bool is_leaf = __double_as_longlong(nd[3]) < 0;
-        const bool active = (u32)my_skip <= (u32)node;
-        bool take = active;
-        int next = node + 1;
-        if (!is_leaf) {  // internal node (a uniform test): opening test
-            const double ddx = nd[0] - x, ddy = nd[1] - y, ddz = nd[2] - z;
-            double d2 = ddx * ddx;
-            d2 = d2 + ddy * ddy;
-            d2 = d2 + ddz * ddz;
-            const double s2 = nd[3] * nd[3];
-            bool far = d2 > s2 * c_hi;
-            const bool unsure = active && !far && !(d2 < s2 * c_lo);
-            if (__builtin_amdgcn_uicmp((u32)unsure, 0u, 33) != 0ull) {
-                if (unsure) far = (nd[3] / sqrt(d2)) < theta;
+            for (int e0 = 0; e0 < have; e0 += B) {
+                double dx[U], dy[U], dz[U], mi[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int j = e0 + u * S + slice;
+                    const bool use = (__shfl(m_have, j) & own) != 0;
+                    mi[u] = monopole(stage[j], use, guard, dx[u], dy[u], dz[u]);
+                    if (COUNT) accepted += use ? 1 : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int j = u * S + slice;
+                    double* o = (double*)&terms[j >> 1][3 * t] + (j & 1);
+                    o[0] = dx[u] * mi[u];
+                    o[2] = dy[u] * mi[u];
+                    o[4] = dz[u] * mi[u];
+                }
+                wave_sync();
+                const int L = lane < NS ? lane : NS - 1;
+#pragma unroll 8
+                for (int r = 0; r < B / 2; r++) {
+                    const double2 v = terms[r][L];
+                    f = f + v.x;
+                    f = f + v.y;
+                }
+                wave_sync();
             }
-            const bool opens = active && !far;
-            take = active && far;
-            next = (__builtin_amdgcn_uicmp((u32)opens, 0u, 33) != 0ull) ? node + 1 : sk;
         }
-        if (take) {
-            const double dx = nd[4] - x, dy = nd[5] - y, dz = nd[6] - z;
-            double d2 = dx * dx;
-            d2 = d2 + dy * dy;
-            d2 = d2 + dz * dz;
-            const double d = d2 + eps2;
-            double inv = 0.0;
-            if (d != 0.0) {
-                const double r = rsqrt_f64(d);
-                inv = r * r * r;
-            }
-            const double mi = nd[7] * inv;
-            ax = ax + dx * mi;
-            ay = ay + dy * mi;
-            az = az + dz * mi;
-            if (COUNT) cnt++;
-            my_skip = sk;
-        }
-        node = __builtin_amdgcn_readfirstlane(next);
+        have = 0;
+        wave_sync();
+    };
+    // a separation of 0 counts as 0; only without softening is there one
+    auto evaluate = [&]() {
+        if (eps2 > 0.0)
+            evaluate_as(std::false_type());
+        else
+            evaluate_as(std::true_type());
+    };
+
+    if (lane == 0) {
+        ids[0] = 0;
+        masks[0] = all;
     }
-    if (live) {
-        acc[3 * t] = ax;
-        acc[3 * t + 1] = ay;
-        acc[3 * t + 2] = az;
-        if (COUNT) counts[t] = cnt;
+    int top = n_nodes > 0 ? 1 : 0;
+    int sub = 0, sub_end = 0, my_skip = 0;  // the subtree walked one node at a time
+    wave_sync();
+    for (;;) {
+        const bool walked = top == 0 && sub == sub_end;
+        if (held >= 64 || (walked && held > 0)) fetch();
+        if (walked) {
+            if (have == 0) break;
+            evaluate();
+            continue;
+        }
+        if (sub != sub_end) {
+            const NodeD nd = nodes[sub];
+            const bool active = my_skip <= sub;
+            const bool far = __double_as_longlong(nd.size) < 0 ||
+                             passes(nd.cx, nd.cy, nd.cz, nd.size);
+            const int sk = skip[sub];
+            const Mask am = (Mask)__ballot(active && far) & all;
+            const bool opens = __ballot(active && !far) != 0;
+            if (active && far) my_skip = sk;
+            if (am != 0) {
+                if (lane == 0) {
+                    lid[held] = sub;
+                    lmask[held] = am;
+                }
+                held += 1;
+                wave_sync();
+            }
+            sub = opens ? sub + 1 : sk;
+            if (have > 0) evaluate();
+            continue;
+        }
+        int n_pop = top < 64 ? top : 64;
+        bool popped = lane < n_pop;
+        const int entry = popped ? ids[top - 1 - lane] : kWalkDone;
+        const Mask m = popped ? masks[top - 1 - lane] : (Mask)0;
+        const bool pending = entry >= 0;
+        const int node = entry & ~kWalkDone;
+        // (lanes without a pending entry load the root's record and ignore it)
+        const double2* rec = (const double2*)(nodes + (pending ? node : 0));
+        const double2 c01 = rec[0], c2s = rec[1];
+        // The children are loaded with the record where latency bounds the walk, and only
+        // where the node is opened where many wavefronts hide it.
+        constexpr bool kAhead = T < 64;
+        int4 ka = make_int4(-1, -1, -1, -1), kb = ka;
+        auto load_kids = [&]() {
+            ka = *(const int4*)(kids + 8 * (int64_t)node);
+            kb = *(const int4*)(kids + 8 * (int64_t)node + 4);
+        };
+        if (kAhead && pending) load_kids();
+        // the box test
+        const bool leaf = __double_as_longlong(c2s.y) < 0;
+        const double s2 = c2s.y * c2s.y;
+        const double gx = fabs(c01.x - bcx), gy = fabs(c01.y - bcy), gz = fabs(c2s.x - bcz);
+        const double nx = fmax(0.0, gx - bhx), ny = fmax(0.0, gy - bhy), nz = fmax(0.0, gz - bhz);
+        const double fx = gx + bhx, fy = gy + bhy, fz = gz + bhz;
+        // (gx is NaN for a box that decides nothing, and nx then 0: hence the third test)
+        const bool clear = leaf || (nx * nx + ny * ny + nz * nz > s2 * box_hi && gx == gx);
+        const bool inside = fx * fx + fy * fy + fz * fz < s2 * box_lo;
+        Mask am = clear ? m : (Mask)0;
+        const bool need = pending && !clear && !inside;
+        const u64 needm = __ballot(need);
+        if (needm != 0) {
+            const int rank = lanes_below(needm);
+            if (need) stage[rank] = make_double4(c01.x, c01.y, c2s.x, c2s.y);
+            wave_sync();
+            const int n_need = (int)__popcll(needm);
+            for (int base = 0, pass = 0; base < n_need; base += S, pass++) {
+                const int j = base + slice < n_need ? base + slice : n_need - 1;
+                const double4 q = stage[j];
+                const u64 far = __ballot(passes(q.x, q.y, q.z, q.w));
+                if (need && rank / S == pass) am = (Mask)(far >> (rank % S * T)) & m;
+            }
+            wave_sync();
+        }
+        const Mask om = pending ? m & ~am : (Mask)0;
+        if (!kAhead && om != 0) load_kids();
+        // children come first in kids[8 n ..], then -1s: 8 plus the sign bits
+        const int nk = om == 0 ? 0 : 8 + (ka.x >> 31) + (ka.y >> 31) + (ka.z >> 31) + (ka.w >> 31) +
+                       (kb.x >> 31) + (kb.y >> 31) + (kb.z >> 31) + (kb.w >> 31);
+        const Mask take = pending ? am : m;  // the targets that accept this entry
+        const u64 opened = __ballot(om != 0);
+        // the first opened entry: what is accepted up to it goes to the list
+        const int stop = opened ? (int)__builtin_ctzll(opened) : 64;
+        // what goes back: the accepted entries after it, and children
+        const bool back = popped && lane > stop && take != 0;
+        const int slots = (back ? 1 : 0) + nk;
+        int total;
+        const int before = wave_excl_count(slots, total);
+        // entries from the first one whose slots do not fit on stay on the stack as they are
+        const u64 over = __ballot(popped && top - 1 - lane + before + slots > CAP);
+        if (over != 0) {
+            n_pop = (int)__builtin_ctzll(over);
+            if (n_pop == 0) {
+                // the top entry (always a pending one: accepted ones at the top have gone to
+                // the list) is walked with its subtree, one node at a time
+                sub = ids[top - 1];
+                sub_end = skip[sub];
+                my_skip = (masks[top - 1] & own) != 0 ? 0 : 0x7fffffff;  // waits below it
+                top -= 1;
+                wave_sync();
+                if (have > 0) evaluate();
+                continue;
+            }
+            total = __builtin_amdgcn_readlane(before, n_pop);
+            popped = lane < n_pop;
+        }
+        const bool out = popped && lane <= stop && take != 0;
+        const int n_out = (int)__popcll(__ballot(out));
+        wave_sync();  // every lane has read its entry
+        if (out) {
+            lid[held + lane] = node;
+            lmask[held + lane] = take;
+        }
+        const int new_top = top - n_pop + total;
+        int w = new_top - 1 - before;
+        if (back && popped) {
+            ids[w] = node | kWalkDone;
+            masks[w] = take;
+            w--;
+        }
+        if (nk > 0 && popped) {
+            const int kk[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (q < nk) {
+                    ids[w - q] = kk[q];
+                    masks[w - q] = om;
+                }
+        }
+        top = new_top;
+        held += n_out;
+        wave_sync();
+        if (have > 0) evaluate();
+    }
+    if constexpr (T == 64) {
+        if (lane < cnt) {
+            acc[3 * ti] = ax;
+            acc[3 * ti + 1] = ay;
+            acc[3 * ti + 2] = az;
+            if (COUNT) counts[ti] = accepted;
+        }
+    } else {
+        if (lane < 3 * cnt) {
+            const int64_t kt = first + lane / 3;
+            acc[3 * (order ? (int64_t)order[kt] : kt) + lane % 3] = f;
+        }
+        if (COUNT) {
+            for (int o = T; o < 64; o <<= 1) accepted += __shfl_xor(accepted, o);
+            if (lane < cnt) counts[ti] = accepted;
+        }
     }
 }
 
@@ -2013,7 +2300,11 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
         GH_TRY(ensure(c, tb->nodes64, sizeof(NodeD) * T));
         GH_TRY(ensure(c, tb->leaf, sizeof(int) * T));
     }
-    if (what & kFillKids) GH_TRY(ensure(c, tb->kids, 8 * sizeof(int) * T));
+    // the FP64 walk's children lists take the place of the moment prefix sums once the fill
+    // has read them (they fit unless the tree has more than two nodes per particle)
+    const size_t kids_bytes = 8 * sizeof(int) * T;
+    const bool kids_in_prefix = (what & kFillF64) && kids_bytes <= tb->prefix.cap;
+    if ((what & kFillKids) && !kids_in_prefix) GH_TRY(ensure(c, tb->kids, kids_bytes));
     if (what & kFillW) GH_TRY(ensure(c, tb->nodesw, sizeof(NodeW) * T));
     if (what & kFillDump) {
         GH_TRY(ensure(c, tb->level, sizeof(short) * T));
@@ -2039,12 +2330,44 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
                        n);
     GH_TRY(check_launch(c, "k_fill_nodes"));
     if (what & kFillKids) {
+        int* const kids = kids_in_prefix ? tb->prefix.as<int>() : tb->kids.as<int>();
         hipLaunchKernelGGL(k_kids, dim3(blocks_for(total, kBlock)), dim3(kBlock), 0, s,
-                           tb->skip.as<int>(), (int)total, tb->kids.as<int>());
+                           tb->skip.as<int>(), (int)total, kids);
+        if (what & kFillF64) tb->kids_f64 = kids;
         GH_TRY(check_launch(c, "k_kids"));
     }
     c->last_tree_nodes = total;
     return 0;
+}
+
+template <int T>
+static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4* stgt,
+                            const u32* order, int64_t nt, double eps, double theta, double c_lo,
+                            double c_hi, double* acc, int* counts, hipStream_t s)
+{
+    const int64_t n_blocks = (nt + (int64_t)T * kWalkWaves - 1) / (T * kWalkWaves);
+    const int64_t per = (n_blocks + kXcds - 1) / kXcds;
+    const dim3 grid((unsigned)(per * kXcds));
+#define GH_WALK64(COUNT, CAP)                                                                 \
+    hipLaunchKernelGGL((k_walk_f64<T, COUNT, CAP>), grid, dim3(64 * kWalkWaves), 0, s,        \
+                       tb->nodes64.as<NodeD>(), tb->kids_f64, tb->skip.as<int>(),             \
+                       (int)tb->n_nodes, tgt, stgt, order, nt, eps * eps, theta, c_lo, c_hi,  \
+                       acc, counts, per)
+    // Stack entries: the window of 64 nodes needs more the smaller theta is (at most 484,
+    // 833 and 1702 in walks of 64 targets at theta = 0.7, 0.5 and 0.3), and a full stack
+    // makes steps small, while LDS for it takes walks off the CU.  N = 2^20, 64 targets,
+    // walk ms with 448 / 768 / 1024 entries: theta 0.7 1.88 / 2.17 / -, 0.5 5.74 / 4.60 /
+    // 5.05, 0.3 - / 18.1 / 15.6 (one node at a time: 2.33, 5.63, 18.7).
+    const int cap = theta >= 0.6 ? 448 : theta >= 0.45 ? 768 : 1024;
+    if (counts)
+        GH_WALK64(true, 1024);
+    else if (cap == 448)
+        GH_WALK64(false, 448);
+    else if (cap == 768)
+        GH_WALK64(false, 768);
+    else
+        GH_WALK64(false, 1024);
+#undef GH_WALK64
 }
 
 // Walks nt targets through the tree built last: the particles themselves (self) or the
@@ -2079,29 +2402,45 @@ static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps,
         GH_TRY(radix_sort(c, tb->tkeys, tb->tidx, tb->hist, nt, 1, 24, s, &sel));
         order = tb->tidx[sel].as<u32>();
     }
-    // Targets per walk: 64 (a full wavefront) when there are enough targets to fill the
-    // GPU; fewer targets give each walk fewer lanes, so that about kWalkUnits walks run
-    // side by side (a walk's length grows with the spread of its targets, and a few
-    // long walks would leave most of the GPU idle).
-    const int lanes = (int)std::min<int64_t>(64, std::max<int64_t>(1, (nt + kWalkUnits - 1) /
-                                                                          kWalkUnits));
-    const int waves_per_block = kWalkBlock / 64;
     if (precision == GH_FP64) {
-        const int64_t n_walks = (nt + lanes - 1) / lanes;
-        const int64_t per = (blocks_for(n_walks, waves_per_block) + kXcds - 1) / kXcds;
+        // Targets per walk.  More of them share a walk's nodes, but its list also holds what
+        // only some of them accept (N = 2^20, theta = 0.7: 1438 entries for 64 targets, 1019
+        // for 16, 631 for 1), and few walks leave the GPU idle: as few targets as leave
+        // about kWalks64 walks, at most 16, and 64 where the GPU is full anyway.  Position
+        // targets lie farther apart than particles as a rule, so fewer share a walk.
+        // Measured (walk, us; start: a walk of 10 to 64 targets, one node at a time):
+        //   particles   2000  5000  20000  40001  150000  300000  2^20
+        //   T = 1         35    66    213    407    1468    3054  11500
+        //   4             42    57    116    205     693    1393   5161
+        //   16            69    86    116    135     406     750   2665
+        //   64           166   214    325    301     456     687   1883
+        //   before       144   233    408    448     682     894   2331
+        // and of 20011 targets among 300007 particles with T = 1, 4, 16, 64: 227, 205, 413
+        // and 1426 us (before 772).
+        int T = 1;
+        if (self) {
+            while (T < 16 && nt > T * kWalks64) T *= 2;
+            if (nt > 200000) T = 64;
+        } else if (order) {
+            while (T < 16 && nt > T * 20000) T *= 2;
+            if (nt > 400000) T = 64;
+        }
         const double inf = __builtin_huge_val();
         const double c_lo = theta > 0.0 ? (1.0 - 1e-13) / (theta * theta) : inf;
         const double c_hi = theta > 0.0 ? (1.0 + 1e-13) / (theta * theta) : inf;
-        if (counts)
-            hipLaunchKernelGGL(k_walk_f64<true>, dim3((unsigned)(per * kXcds)), dim3(kWalkBlock),
-                               0, s, tb->nodes64.as<NodeD>(), tb->skip.as<int>(),
-                               tb->n_nodes, tgt, stgt, order, nt, eps, theta,
-                               c_lo, c_hi, d_acc, counts, per, lanes);
-        else
-            hipLaunchKernelGGL(k_walk_f64<false>, dim3((unsigned)(per * kXcds)), dim3(kWalkBlock),
-                               0, s, tb->nodes64.as<NodeD>(), tb->skip.as<int>(),
-                               tb->n_nodes, tgt, stgt, order, nt, eps, theta,
-                               c_lo, c_hi, d_acc, counts, per, lanes);
+#define GH_WALK64(T)                                                                           \
+    case T:                                                                                    \
+        launch_walk_f64<T>(tb, tgt, stgt, order, nt, eps, theta, c_lo, c_hi, d_acc, counts, s); \
+        break
+        switch (T) {
+            GH_WALK64(1);
+            GH_WALK64(2);
+            GH_WALK64(4);
+            GH_WALK64(8);
+            GH_WALK64(16);
+            GH_WALK64(64);
+        }
+#undef GH_WALK64
         return check_launch(c, "k_walk_f64");
     }
     // FP32: the group walk, 16 targets per wavefront, or one target per wavefront when
@@ -2156,7 +2495,7 @@ int tree_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     if (precision != GH_FP64 && precision != GH_FP32)
         return fail(c, GH_EARG, "unknown precision %d", precision);
     GH_TRY(build_tree(c, d_pos, d_mass, np, eps, theta,
-                      precision == GH_FP64 ? kFillF64 : (kFillW | kFillKids), s));
+                      kFillKids | (precision == GH_FP64 ? kFillF64 : kFillW), s));
     return walk(c, self ? d_pos : d_fpos, self, nt, eps, theta, precision, d_acc, nullptr, s);
 }
 
@@ -2257,7 +2596,7 @@ static int tree_counts(gh_ctx* c, const double* pos, const double* mass, int64_t
         tgt = c->fpos64.as<double>();
     }
     GH_TRY(build_tree(c, c->pos64.as<double>(), c->mass64.as<double>(), np, eps, theta,
-                      precision == GH_FP64 ? kFillF64 : (kFillW | kFillKids), s));
+                      kFillKids | (precision == GH_FP64 ? kFillF64 : kFillW), s));
     GH_TRY(walk(c, tgt, self, nt, eps, theta, precision, c->acc64.as<double>(),
                 c->scratch.as<int>(), s));
     std::vector<int> cnt((size_t)(nt > 0 ? nt : 1));

@@ -378,3 +378,71 @@ def test_fp32_walk_list_lengths(ctx, group):
     assert np.all(c32 >= cref)
     assert c32.mean() < 2.5 * cref.mean()
     assert c32.max() < 8 * cref.max()
+
+
+# targets per walk change at these counts (walk() in gh_tree.hip), for particles
+@pytest.mark.parametrize("n", [2560, 2561, 5121, 10241, 20481, 40961, 200000, 200001])
+def test_fp64_walk_shapes_same_bits(ctx, n):
+    # a particle's force is the same bits from the self walk and from a walk of its own
+    # (few position targets: one per walk)
+    rng = np.random.default_rng(n)
+    pos = rng.normal(size=(n, 3)) * np.exp(rng.normal(size=(n, 1)))
+    mass = rng.uniform(0.5, 2.0, size=n)
+    some = np.unique(np.concatenate([[0, n - 1], rng.integers(0, n, size=400)]))
+    for eps, theta in ((0.01, 0.7), (0.0, 0.7), (0.01, 0.5), (0.01, 0.4)):
+        if n > 100000 and theta != 0.7:
+            continue
+        full = ctx.tree(pos, mass, eps, theta, FP64)
+        own = ctx.tree(pos, mass, eps, theta, FP64, force_pos=pos[some])
+        assert_bitwise(full[some], own, "eps=%g theta=%g" % (eps, theta))
+
+
+# ... and for position targets (sorted from 4096 on)
+@pytest.mark.parametrize("nf", [1, 4095, 4096, 20001, 40001, 80001, 160001, 400001])
+def test_fp64_walk_target_shapes_same_bits(ctx, nf):
+    rng = np.random.default_rng(nf)
+    pos = rng.normal(size=(5000, 3))
+    mass = rng.uniform(0.5, 2.0, size=5000)
+    fpos = rng.normal(size=(nf, 3)) * 2
+    fpos[::50] = pos[rng.integers(0, 5000, size=len(fpos[::50]))]
+    some = np.unique(np.concatenate([[0, nf - 1], rng.integers(0, nf, size=300)]))
+    full = ctx.tree(pos, mass, 0.01, 0.7, FP64, force_pos=fpos)
+    own = ctx.tree(pos, mass, 0.01, 0.7, FP64, force_pos=fpos[some])
+    assert_bitwise(full[some], own)
+
+
+@pytest.mark.parametrize("n", [3, 70, 600, 6000, 12000])
+def test_fp64_walk_full_stack(ctx, oracle, n):
+    """Walks that open almost every node (theta 0 to 0.2) of trees of up to 40 levels: the
+    stack fills, steps take few nodes, and subtrees are walked one node at a time."""
+    rng = np.random.default_rng(n)
+    pos = rng.normal(size=(n, 3))
+    tight = n // 3
+    pos[:tight] = pos[0] + rng.normal(size=(tight, 3)) * 10.0 ** rng.uniform(-10, 0, (tight, 1))
+    mass = rng.uniform(0.5, 2.0, size=n)
+    some = np.unique(rng.integers(0, n, size=200))
+    for theta in (0.0, 0.05, 0.2, 0.7):
+        want, cnt = oracle.tree(pos, mass, 0.01, theta, force_pos=pos[some], count=True)
+        got = ctx.tree(pos, mass, 0.01, theta, FP64)
+        np.testing.assert_allclose(got[some], want, rtol=1e-10,
+                                   atol=1e-10 * np.abs(want).max(), err_msg="theta=%g" % theta)
+        _, gcnt = ctx.tree_interactions(pos, mass, 0.01, theta, precision=FP64)
+        assert np.array_equal(gcnt[some], cnt), theta
+
+
+def test_fp64_walk_target_not_finite(ctx, oracle):
+    # such a target gets what the reference gives it and leaves its neighbours alone
+    rng = np.random.default_rng(5)
+    n = 6000
+    pos = rng.normal(size=(n, 3))
+    mass = rng.uniform(0.5, 2.0, size=n)
+    fpos = rng.normal(size=(5000, 3))
+    fpos[1000] = [np.nan, 0, 0]
+    fpos[2000] = [0, np.inf, 0]
+    fpos[3000] = [0, 0, 1e300]
+    some = np.array([0, 999, 1001, 1999, 2001, 2999, 3001, 4999])
+    got = ctx.tree(pos, mass, 0.01, 0.7, FP64, force_pos=fpos)
+    assert_bitwise(got[some], ctx.tree(pos, mass, 0.01, 0.7, FP64, force_pos=fpos[some]))
+    assert np.all(np.isnan(got[1000]))
+    fine = np.delete(np.arange(5000), [1000, 2000, 3000])
+    assert np.all(np.isfinite(got[fine]))
