@@ -559,15 +559,22 @@ struct SymOut {
 // One block pair.  Work item {I, J, slot_i, slot_j}: global block indices I <= J (of
 // one simulation), the partial slot the i-side field goes to (J's index within its
 // simulation) and the slot of the j-side field (I's index within its simulation).
-template <int IPT, bool GUARD, bool DS>
+// UNI: the particles of block I all have mass mI and those of block J mass mJ, so the masses
+// multiply the sums instead of every pair's factor: 15 instead of 17 VALU operations per
+// pair.
+template <int IPT, bool GUARD, bool DS, bool UNI>
 __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
                                          const double4* __restrict__ s64,
                                          const double4* __restrict__ frame, int64_t np_pad,
-                                         int4 it, float eps2, const SymOut out,
-                                         float4* tile, float4* tile_lo, float (*jp)[3][64])
+                                         int4 it, float eps2, float mI, float mJ,
+                                         const SymOut out, float4* tile, float (*jp)[3][64])
 {
     constexpr int BLK = kBlock * IPT;
     constexpr int NCH = BLK / 64;
+    // each 64-particle chunk of block J is stored twice in a row, so that lane l's rotating
+    // index l + s needs no wrap-around; DS stores it once and its low words after all chunks
+    constexpr int ROW = DS ? 64 : 128;
+    float4* const tile_lo = tile + (DS ? BLK : 0);
     const int I = it.x, J = it.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t ibase = (int64_t)I * BLK + wave * 64 * IPT + lane;
@@ -596,8 +603,8 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
         ax[k] = ay[k] = az[k] = 0.f;
     }
     if (DS) {
-        for (int q = threadIdx.x; q < NCH * 128; q += kBlock) {
-            const double4 v = s64[jbase + (q >> 7) * 64 + (q & 63)];
+        for (int q = threadIdx.x; q < BLK; q += kBlock) {
+            const double4 v = s64[jbase + q];
             float4 h, l;
             split_ds(v.x - oI.x, h.x, l.x);
             split_ds(v.y - oI.y, h.y, l.y);
@@ -623,11 +630,11 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
 
     if (I == J) {
         for (int c = 0; c < NCH; c++) {
-#pragma unroll 8
+#pragma unroll(DS ? 1 : 8)
             for (int q = 0; q < 64; q++) {
-                const float4 s = tile[c * 128 + q];
+                const float4 s = tile[c * ROW + q];
                 float4 sl = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (DS) sl = tile_lo[c * 128 + q];
+                if (DS) sl = tile_lo[c * ROW + q];
 #pragma unroll
                 for (int k = 0; k < IPT; k++) {
                     float dx = s.x - xi[k], dy = s.y - yi[k], dz = s.z - zi[k];
@@ -640,7 +647,7 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
                     r2 = __builtin_fmaf(dy, dy, r2);
                     r2 = __builtin_fmaf(dz, dz, r2);
                     const float ri = __builtin_amdgcn_rsqf(r2);
-                    float sc = (s.w * ri) * (ri * ri);
+                    float sc = UNI ? ri * (ri * ri) : (s.w * ri) * (ri * ri);
                     if (GUARD) sc = clamp_finite(sc);
                     ax[k] = __builtin_fmaf(dx, sc, ax[k]);
                     ay[k] = __builtin_fmaf(dy, sc, ay[k]);
@@ -650,15 +657,14 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
         }
     } else {
         for (int c = 0; c < NCH; c++) {
-            const float4* row = &tile[c * 128 + lane];
-            const float4* row_lo = &tile_lo[DS ? c * 128 + lane : 0];
             float fx = 0.f, fy = 0.f, fz = 0.f;
             for (int s0 = 0; s0 < 64; s0 += 8) {
-#pragma unroll
+#pragma unroll(DS ? 1 : 8)
                 for (int s = 0; s < 8; s++) {
-                    const float4 sj = row[s0 + s];
+                    const int q = c * ROW + (DS ? (lane + s0 + s) & 63 : lane + s0 + s);
+                    const float4 sj = tile[q];
                     float4 sl = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (DS) sl = row_lo[s0 + s];
+                    if (DS) sl = tile_lo[q];
 #pragma unroll
                     for (int k = 0; k < IPT; k++) {
                         float dx = sj.x - xi[k], dy = sj.y - yi[k], dz = sj.z - zi[k];
@@ -672,12 +678,12 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
                         r2 = __builtin_fmaf(dz, dz, r2);
                         const float ri = __builtin_amdgcn_rsqf(r2);
                         const float ri3 = ri * ri * ri;
-                        float si = sj.w * ri3;
+                        float si = UNI ? ri3 : sj.w * ri3;
                         if (GUARD) si = clamp_finite(si);
                         ax[k] = __builtin_fmaf(dx, si, ax[k]);
                         ay[k] = __builtin_fmaf(dy, si, ay[k]);
                         az[k] = __builtin_fmaf(dz, si, az[k]);
-                        float sm = mi[k] * ri3;
+                        float sm = UNI ? ri3 : mi[k] * ri3;
                         if (GUARD) sm = clamp_finite(sm);
                         fx = __builtin_fmaf(dx, sm, fx);
                         fy = __builtin_fmaf(dy, sm, fy);
@@ -700,7 +706,7 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
 #pragma unroll
                 for (int w = 1; w < kBlock / 64; w++) sacc += jp[w][comp][t];
                 out.jpart[((int64_t)it.w * out.jstride + (jbase - out.joff) + c * 64 + t) * 3 +
-                          comp] = -sacc;
+                          comp] = UNI ? -sacc * mI : -sacc;
             }
             __syncthreads();
         }
@@ -708,78 +714,72 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
 #pragma unroll
     for (int k = 0; k < IPT; k++) {
         float* o = out.part + ((int64_t)it.z * np_pad + ibase + k * 64) * 3;
-        o[0] = ax[k];
-        o[1] = ay[k];
-        o[2] = az[k];
+        o[0] = UNI ? ax[k] * mJ : ax[k];
+        o[1] = UNI ? ay[k] * mJ : ay[k];
+        o[2] = UNI ? az[k] * mJ : az[k];
     }
 }
 
-// One launch over a list of block pairs; items with a flagged block are skipped (the DS
-// kernel takes them).  queue == nullptr: workgroup b takes item b.  Otherwise the
-// workgroups are persistent and take items from *queue (which must be 0 at launch)
-// until the list is exhausted.
+// One launch over a list of block pairs.  queue == nullptr: workgroup b takes item b.
+// Otherwise the workgroups are persistent and take items from *queue (which must be 0 at
+// launch) until the list is exhausted.
+//  - Items with a flagged block take the DS form, about twice the time of another item; a
+//    persistent launch takes them first, spread over the workgroups, so that none starts
+//    last.  (As a launch of its own after the others the DS form ran at the length of one
+//    item, 190 us in an ensemble of 32 spheres of 1024 to 16384 particles, whose outermost
+//    blocks are flagged, and 4.6 us where no block is.)
+//  - Items whose blocks each have one mass (umass, not NaN) take the UNI form in simulations
+//    of at least kUniMin particles (nb_blk[b] or, where it is null, nb blocks), unless the
+//    guard is needed, which bounds the factors with their masses.  Measured (N = 262144,
+//    equal masses, per launch): 13.33 -> 11.98 ms.  Below kUniMin the sort, the reduction
+//    and the launches are a growing share of a step (N = 16384: 2 % of a gradient gained),
+//    and results keep the bits of the general form.
+constexpr int kUniMin = 131072;
+
 template <int IPT, bool GUARD>
-__global__ __launch_bounds__(kBlock) void k_direct_sym_f32(const float4* __restrict__ src,
-                                                           const double4* __restrict__ frame,
-                                                           const int* __restrict__ flag,
-                                                           int64_t np_pad,
-                                                           const int4* __restrict__ work,
-                                                           int64_t items,
-                                                           const float* __restrict__ eps2_blk,
-                                                           const SymOut out,
-                                                           int* __restrict__ queue)
+__global__ __launch_bounds__(kBlock) void k_direct_sym_f32(
+    const float4* __restrict__ src, const double4* __restrict__ s64,
+    const double4* __restrict__ frame, const int* __restrict__ flag,
+    const int* __restrict__ nflag, const float* __restrict__ umass,
+    const int* __restrict__ nb_blk, int nb, int64_t np_pad, const int4* __restrict__ work,
+    int64_t items, const float* __restrict__ eps2_blk, const SymOut out, int* __restrict__ queue)
 {
     constexpr int NCH = kBlock * IPT / 64;
-    // each 64-particle chunk of block J is stored twice in a row, so that lane l's
-    // rotating index l + s needs no wrap-around
     __shared__ float4 tile[NCH * 128];
     __shared__ float jp[kBlock / 64][3][64];
     __shared__ int next;
-    if (!queue) {
-        const int4 it = work[blockIdx.x];
-        if (flag[it.x] | flag[it.y]) return;
-        sym_item<IPT, GUARD, false>(src, nullptr, frame, np_pad, it, eps2_blk[it.x], out, tile,
-                                    nullptr, jp);
-        return;
-    }
-    for (;;) {
-        if (threadIdx.x == 0) next = atomicAdd(queue, 1);
-        __syncthreads();
-        const int64_t k = next;
-        __syncthreads();
-        if (k >= items) break;
+    // the persistent launch's flagged items; k runs over this workgroup's share of the list
+    const bool first = queue && *nflag != 0;
+    int64_t k = blockIdx.x;
+    for (bool flagged = first;;) {
+        if (queue && !flagged) {
+            if (threadIdx.x == 0) next = atomicAdd(queue, 1);
+            __syncthreads();
+            k = next;
+            __syncthreads();
+        }
+        if (k >= items) {
+            if (!flagged) break;
+            flagged = false;
+            continue;
+        }
         const int4 it = work[k];
-        if (flag[it.x] | flag[it.y]) continue;
-        sym_item<IPT, GUARD, false>(src, nullptr, frame, np_pad, it, eps2_blk[it.x], out, tile,
-                                    nullptr, jp);
+        const bool ds = (flag[it.x] | flag[it.y]) != 0;
+        const float mI = umass[it.x], mJ = umass[it.y], eps2 = eps2_blk[it.x];
+        const int blocks = nb_blk ? nb_blk[it.x] : nb;
+        if (ds && flagged == first)
+            sym_item<IPT, GUARD, true, false>(nullptr, s64, frame, np_pad, it, eps2, 0.f, 0.f,
+                                              out, tile, jp);
+        else if (!ds && !flagged && !GUARD && blocks >= kUniMin / (kBlock * IPT) && mI == mI &&
+                 mJ == mJ)
+            sym_item<IPT, GUARD, false, !GUARD>(src, nullptr, frame, np_pad, it, eps2, mI, mJ,
+                                                out, tile, jp);
+        else if (!ds && !flagged)
+            sym_item<IPT, GUARD, false, false>(src, nullptr, frame, np_pad, it, eps2, 0.f, 0.f,
+                                               out, tile, jp);
+        if (!queue) break;
         __syncthreads();
-    }
-}
-
-// The items the fast kernel skips, in double-single form: a persistent grid strides
-// over the whole list and takes the items with a flagged block.
-template <int IPT, bool GUARD>
-__global__ __launch_bounds__(kBlock) void k_direct_sym_ds(const double4* __restrict__ s64,
-                                                          const double4* __restrict__ frame,
-                                                          const int* __restrict__ flag,
-                                                          const int* __restrict__ nflag,
-                                                          int64_t np_pad,
-                                                          const int4* __restrict__ work,
-                                                          int64_t items,
-                                                          const float* __restrict__ eps2_blk,
-                                                          const SymOut out)
-{
-    constexpr int NCH = kBlock * IPT / 64;
-    __shared__ float4 tile[NCH * 128];
-    __shared__ float4 tile_lo[NCH * 128];
-    __shared__ float jp[kBlock / 64][3][64];
-    if (*nflag == 0) return;  // no flagged block: nothing to do
-    for (int64_t k = blockIdx.x; k < items; k += gridDim.x) {
-        const int4 it = work[k];
-        if (!(flag[it.x] | flag[it.y])) continue;
-        sym_item<IPT, GUARD, true>(nullptr, s64, frame, np_pad, it, eps2_blk[it.x], out, tile,
-                                   tile_lo, jp);
-        __syncthreads();
+        if (flagged) k += gridDim.x;
     }
 }
 
@@ -997,29 +997,11 @@ int sym_ipt(gh_ctx* c, int64_t np)
     return ipt;
 }
 
-template <int IPT>
-static void launch_sym_t(bool guard, unsigned grid, hipStream_t s, const float4* src,
-                         const double4* s64, const double4* frame, const int* flag,
-                         const int* nflag, int64_t np_pad, const int4* work, int64_t items,
-                         const float* eps2_blk, const SymOut out, int* queue, unsigned ds_grid)
-{
-    if (guard) {
-        hipLaunchKernelGGL((k_direct_sym_f32<IPT, true>), dim3(grid), dim3(kBlock), 0, s, src,
-                           frame, flag, np_pad, work, items, eps2_blk, out, queue);
-        hipLaunchKernelGGL((k_direct_sym_ds<IPT, true>), dim3(ds_grid), dim3(kBlock), 0, s, s64,
-                           frame, flag, nflag, np_pad, work, items, eps2_blk, out);
-    } else {
-        hipLaunchKernelGGL((k_direct_sym_f32<IPT, false>), dim3(grid), dim3(kBlock), 0, s, src,
-                           frame, flag, np_pad, work, items, eps2_blk, out, queue);
-        hipLaunchKernelGGL((k_direct_sym_ds<IPT, false>), dim3(ds_grid), dim3(kBlock), 0, s,
-                           s64, frame, flag, nflag, np_pad, work, items, eps2_blk, out);
-    }
-}
-
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,
-               const double4* frame, const int* flag, const int* nflag, int64_t np_pad,
-               const int4* work, int64_t items, const float* eps2_blk, float* part, int* queue,
-               unsigned persistent_grid, hipStream_t s, float* jpart, int64_t jstride,
+               const double4* frame, const int* flag, const int* nflag, const float* umass,
+               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
+               const float* eps2_blk, float* part,
+               int* queue, unsigned persistent_grid, hipStream_t s, float* jpart, int64_t jstride,
                int64_t joff)
 {
     SymOut out;
@@ -1030,13 +1012,24 @@ int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4*
     if (items > 0x7fffffff) return fail(c, GH_EARG, "too many block pairs for one launch");
     const unsigned grid = queue ? persistent_grid : (unsigned)items;
     if (grid == 0) return 0;
-    const unsigned ds_grid = (unsigned)std::min<int64_t>(items, 2 * (int64_t)c->n_cu);
+#define GH_SYM(IPT)                                                                            \
+    case IPT:                                                                                  \
+        if (guard)                                                                             \
+            hipLaunchKernelGGL((k_direct_sym_f32<IPT, true>), dim3(grid), dim3(kBlock), 0, s,  \
+                               src, s64, frame, flag, nflag, umass, nb_blk, nb, np_pad, work,  \
+                               items, eps2_blk, out, queue);                                   \
+        else                                                                                   \
+            hipLaunchKernelGGL((k_direct_sym_f32<IPT, false>), dim3(grid), dim3(kBlock), 0, s, \
+                               src, s64, frame, flag, nflag, umass, nb_blk, nb, np_pad, work,  \
+                               items, eps2_blk, out, queue);                                   \
+        break
     switch (ipt) {
-        case 1: launch_sym_t<1>(guard, grid, s, src, s64, frame, flag, nflag, np_pad, work, items, eps2_blk, out, queue, ds_grid); break;
-        case 2: launch_sym_t<2>(guard, grid, s, src, s64, frame, flag, nflag, np_pad, work, items, eps2_blk, out, queue, ds_grid); break;
-        case 4: launch_sym_t<4>(guard, grid, s, src, s64, frame, flag, nflag, np_pad, work, items, eps2_blk, out, queue, ds_grid); break;
+        GH_SYM(1);
+        GH_SYM(2);
+        GH_SYM(4);
         default: return fail(c, GH_EARG, "unsupported particles-per-lane %d", ipt);
     }
+#undef GH_SYM
     return check_launch(c, "k_direct_sym_f32");
 }
 
@@ -1114,9 +1107,9 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
         {
             TimedScope ts(c, s, GH_T_DIRECT_F32);
             GH_TRY(launch_sym(c, ipt, guard, o.loc.as<float4>(), o.s64.as<double4>(),
-                              o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(), np_pad,
-                              c->work.as<int4>(), items, c->eps_blk.as<float>(), part, nullptr,
-                              0, s));
+                              o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
+                              o.umass.as<float>(), nullptr, nb, np_pad, c->work.as<int4>(), items,
+                              c->eps_blk.as<float>(), part, nullptr, 0, s));
         }
         return reduce_sym(c, part, nb, nullptr, (int)blk, np_pad, np, o.perm(), d_acc, s);
     }
@@ -1127,9 +1120,10 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
         {
             TimedScope ts(c, s, GH_T_DIRECT_F32);
             GH_TRY(launch_sym(c, ipt, guard, o.loc.as<float4>(), o.s64.as<double4>(),
-                              o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(), np_pad,
-                              c->work.as<int4>() + i0, ni, c->eps_blk.as<float>(), part, nullptr,
-                              0, s, partj, (int64_t)w * blk, (int64_t)c0 * blk));
+                              o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
+                              o.umass.as<float>(), nullptr, nb, np_pad, c->work.as<int4>() + i0, ni,
+                              c->eps_blk.as<float>(), part, nullptr, 0, s, partj,
+                              (int64_t)w * blk, (int64_t)c0 * blk));
         }
         hipLaunchKernelGGL(k_reduce_band, dim3(blocks_for(3 * np, kBlock)), dim3(kBlock), 0, s,
                            part, partj, (int)blk, c0, wb, w, np_pad, 3 * np, o.perm(), b == 0,

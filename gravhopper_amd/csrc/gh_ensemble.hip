@@ -94,9 +94,8 @@ static int ens_step(gh_ensemble* e, hipStream_t s)
     {
         TimedScope ts(c, s, GH_T_DIRECT_F32);
         GH_TRY(launch_sym(c, e->ipt, e->guard, o.loc.as<float4>(), o.s64.as<double4>(),
-                          o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(), e->n_pad,
-                          e->work.as<int4>(),
-                          e->items, e->eps_blk.as<float>(), e->part.as<float>(),
+                          o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
+                          o.umass.as<float>(), e->nb_blk.as<int>(), 0, e->n_pad, e->work.as<int4>(), e->items, e->eps_blk.as<float>(), e->part.as<float>(),
                           e->persistent ? e->queue.as<int>() : nullptr, e->grid, s));
     }
     GH_TRY(reduce_sym(c, e->part.as<float>(), 0, e->nb_blk.as<int>(), e->blk, e->n_pad,
@@ -120,7 +119,7 @@ static void ens_free(gh_ensemble* e)
                       &e->dt_blk,    &e->queue,     &e->seg_blk,  &e->seg_start, &e->seg_count,
                       &o.keys[0],    &o.keys[1],    &o.idx[0],    &o.idx[1],     &o.hist,
                       &o.box,        &o.boxpart,    &o.loc,       &o.s64,        &o.frame,
-                      &o.flag,       &o.nflag};
+                      &o.flag,       &o.nflag,     &o.umass};
     for (DevBuf* b : bufs) release(c, *b);
 }
 

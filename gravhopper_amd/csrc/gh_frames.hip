@@ -273,7 +273,8 @@ __device__ __forceinline__ long long wave_sum(long long v)
 // One workgroup per group of G consecutive sorted points.  Origin: the group's point at
 // offset min(G/2, count-1) (a point of the group's majority part, so that a group with a
 // few strays keeps a useful frame).  Writes loc / s64 for the group's G slots (padding:
-// massless at the origin), frame = (origin, R) and the compactness flag.
+// massless at the origin), frame = (origin, R), the compactness flag, and the FP32 mass all
+// points of the group share (NaN where they do not, or where the group is padded).
 template <int G>
 __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ pos,
                                                    const double* __restrict__ mass,
@@ -283,8 +284,10 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
                                                    double4* __restrict__ s64,
                                                    double4* __restrict__ frame,
                                                    int* __restrict__ flag,
-                                                   int* __restrict__ nflag)
+                                                   int* __restrict__ nflag,
+                                                   float* __restrict__ umass)
 {
+    __shared__ float sLo[kBlock / 64], sHi[kBlock / 64];
     __shared__ double sR[kBlock / 64];
     __shared__ long long sE[kBlock / 64], sC[kBlock / 64];
     const int64_t p0 = (int64_t)blockIdx.x * G;
@@ -300,6 +303,8 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
     }
     double R = 0.0;
     long long esum = 0, gcnt = 0;
+    float mlo = HUGE_VALF, mhi = -HUGE_VALF;
+    bool same = cnt == G;  // no padding, and no mass that is not a number
     for (int k = threadIdx.x; k < G; k += kBlock) {
         const int64_t p = p0 + k;
         if (k < cnt) {
@@ -309,6 +314,9 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
             const double dx = x - ox, dy = y - oy, dz = z - oz;
             R = fmax(R, fmax(fabs(dx), fmax(fabs(dy), fabs(dz))));
             loc[p] = make_float4((float)dx, (float)dy, (float)dz, (float)m);
+            mlo = fminf(mlo, (float)m);
+            mhi = fmaxf(mhi, (float)m);
+            same = same && m == m;
             if (s64) s64[p] = make_double4(x, y, z, m);
             if (k + 1 < cnt) {
                 const int64_t j2 = perm ? (int64_t)perm[p + 1] : p + 1;
@@ -325,11 +333,18 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
     R = wave_max(R);
     esum = wave_sum(esum);
     gcnt = wave_sum(gcnt);
+    for (int o = 32; o > 0; o >>= 1) {
+        mlo = fminf(mlo, __shfl_xor(mlo, o));
+        mhi = fmaxf(mhi, __shfl_xor(mhi, o));
+    }
+    if (__ballot(!same) != 0) mlo = -HUGE_VALF;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) {
         sR[wave] = R;
         sE[wave] = esum;
         sC[wave] = gcnt;
+        sLo[wave] = mlo;
+        sHi[wave] = mhi;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -337,7 +352,10 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
             R = fmax(R, sR[w]);
             esum += sE[w];
             gcnt += sC[w];
+            mlo = fminf(mlo, sLo[w]);
+            mhi = fmaxf(mhi, sHi[w]);
         }
+        umass[blockIdx.x] = mlo == mhi ? mlo : __builtin_nanf("");
         // log2 R - mean log2 gap > kFrameLog2, in integer exponents
         const long long eR = exponent_of(R);
         const bool loose = gcnt > 0 && eR * gcnt - esum > (long long)kFrameLog2 * gcnt;
@@ -359,11 +377,12 @@ int gather_frames(gh_ctx* c, OrderBufs& o, const double* d_pos, const double* d_
     GH_TRY(ensure(c, o.frame, sizeof(double4) * (size_t)ng));
     GH_TRY(ensure(c, o.flag, sizeof(int) * (size_t)ng));
     GH_TRY(ensure(c, o.nflag, 256));
+    GH_TRY(ensure(c, o.umass, sizeof(float) * (size_t)ng));
     double4* s64 = want_s64 ? o.s64.as<double4>() : nullptr;
 #define GH_FRAMES(GG)                                                                       \
     hipLaunchKernelGGL(k_frames<GG>, dim3((unsigned)ng), dim3(kBlock), 0, s, d_pos, d_mass,  \
                        perm, n, valid, o.loc.as<float4>(), s64, o.frame.as<double4>(),       \
-                       o.flag.as<int>(), o.nflag.as<int>())
+                       o.flag.as<int>(), o.nflag.as<int>(), o.umass.as<float>())
     switch (group) {
         case 256: GH_FRAMES(256); break;
         case 512: GH_FRAMES(512); break;

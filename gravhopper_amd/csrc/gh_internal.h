@@ -49,6 +49,7 @@ struct OrderBufs {
     DevBuf frame;  // double4 per group: origin (x, y, z), largest |x - o| (max norm)
     DevBuf flag;   // int per group: 1 if the group is not compact (see k_frames)
     DevBuf nflag;  // int: number of flagged groups (cleared by the key kernels)
+    DevBuf umass;  // float per group: the mass all its points share, else NaN
     int sel = 0;   // which of idx[0] / idx[1] holds the order
     const double* sorted = nullptr;  // positions spatial_order last ordered (n of them)
     int64_t sorted_n = 0;
@@ -186,13 +187,13 @@ bool fp32_guard(double eps);
 int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np, int ipt,
                double eps, double* d_acc, hipStream_t s);
 // The pair-once kernel over a block-pair list (src: local FP32 coordinates per sorted
-// particle, s64: the same particles in FP64, frame/flag: per block), followed by its
+// particle, s64: the same particles in FP64, frame/flag/umass: per block), followed by its
 // double-single instance for the items with a flagged block.
 // jpart (nullable): the j-side partials go to jpart[slot_j][p - joff] with a stride of
 // jstride particles instead of part.
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,
-               const double4* frame, const int* flag, const int* nflag, int64_t np_pad,
-               const int4* work, int64_t items, const float* eps2_blk, float* part, int* queue,
+               const double4* frame, const int* flag, const int* nflag, const float* umass,
+               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items, const float* eps2_blk, float* part, int* queue,
                unsigned persistent_grid, hipStream_t s, float* jpart = nullptr,
                int64_t jstride = 0, int64_t joff = 0);
 // acc[perm[p]] (perm nullable) = the FP64 sum of particle p's partial slots

@@ -257,3 +257,21 @@ def test_fp64_direct_operand_range_bitwise(ctx, oracle, nf):
         assert np.array_equal(np.isnan(got), np.isnan(want))
         ok = ~np.isnan(want)
         assert_bitwise(got[ok], want[ok], "eps=%g" % eps)
+
+
+@pytest.mark.parametrize("n", [131071, 131072, 131072 + 300, 140000])
+def test_fp32_direct_block_masses(ctx, n):
+    """Either side of the size from which blocks of one mass take it out of their pairs'
+    factors, with blocks of one mass, of mixed masses and a padded one: as accurate
+    against FP64 as the general form (the direct sum's FP32 tolerance)."""
+    ic = workloads.plummer(n, seed=n % 1000)
+    rng = np.random.default_rng(n)
+    mass = ic["mass"].copy()
+    mass[ic["pos"][:, 0] > 2e-3] *= 3.0          # a region of another mass
+    odd = rng.integers(0, n, size=20)
+    mass[odd] *= rng.uniform(0.5, 2.0, size=20)  # and single particles of their own
+    got = ctx.direct(ic["pos"], mass, 2e-5, FP32)
+    some = np.unique(np.concatenate([odd, rng.integers(0, n, size=2000)]))
+    want = ctx.direct(ic["pos"], mass, 2e-5, FP64)[some]
+    e = rel_err(got[some], want)
+    assert np.median(e) <= 1e-6 and np.percentile(e, 99) <= 1e-4, (np.median(e), e.max())
