@@ -27,6 +27,7 @@ struct gh_ensemble {
     bool persistent = false;
     int64_t n_pad = 0, nb_total = 0, items = 0;
     int nb_max = 0;
+    int64_t n_max = 0;  // particles of the largest simulation
     unsigned grid = 0;
     std::vector<int64_t> start, count;
     gh::DevBuf x, v, xh, m, acc, part, work, eps_blk, nb_blk, valid_blk, dt_blk, queue;
@@ -84,7 +85,7 @@ static int ens_step(gh_ensemble* e, hipStream_t s)
     OrderBufs& o = e->ord;
     GH_TRY(spatial_order_seg(c, o, e->xh.as<double>(), e->n_pad, e->blk, e->nsims,
                              e->seg_blk.as<int>(), e->seg_start.as<int64_t>(),
-                             e->seg_count.as<int64_t>(), s));
+                             e->seg_count.as<int64_t>(), e->n_max, s));
     GH_TRY(gather_frames(c, o, e->xh.as<double>(), e->m.as<double>(), o.perm(), e->n_pad,
                          e->n_pad, e->blk, e->valid_blk.as<int>(), true, s));
     if (e->persistent) {
@@ -173,6 +174,7 @@ int gh_ensemble_create(gh_ctx* c, int n_sims, const int64_t* counts, const doubl
         }
         if (fp32_guard(eps[s])) e->guard = true;
         e->nb_max = std::max<int>(e->nb_max, (int)nb);
+        e->n_max = std::max(e->n_max, n);
         pad += nb * e->blk;
         total += n;
     }
@@ -238,7 +240,7 @@ int gh_ensemble_create(gh_ctx* c, int n_sims, const int64_t* counts, const doubl
     if (!rc)
         rc = spatial_order_seg(c, e->ord, e->xh.as<double>(), e->n_pad, e->blk, e->nsims,
                                e->seg_blk.as<int>(), e->seg_start.as<int64_t>(),
-                               e->seg_count.as<int64_t>(), s);
+                               e->seg_count.as<int64_t>(), e->n_max, s);
     if (!rc)
         rc = gather_frames(c, e->ord, e->xh.as<double>(), e->m.as<double>(), e->ord.perm(),
                            e->n_pad, e->n_pad, e->blk, e->valid_blk.as<int>(), true, s);

@@ -219,10 +219,11 @@ int spatial_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, hipSt
 // The same order for a padded layout of nseg segments (segment g: positions
 // [start[g], start[g] + count[g]) of pos (n_pad,3), blocks of blk positions, seg[b] the
 // segment of block b, all device arrays): each segment sorted in its own box exactly as
-// spatial_order sorts it alone, segments in place, padding last in its segment.
+// spatial_order sorts it alone, segments in place, padding last in its segment.  most: the
+// largest segment's count.
 int spatial_order_seg(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n_pad, int blk,
                       int nseg, const int* seg, const int64_t* start, const int64_t* count,
-                      hipStream_t s);
+                      int64_t most, hipStream_t s);
 // Fills o.loc, o.s64 (nullable output: skipped if want_s64 is false), o.frame and
 // o.flag for n_pad / group points in groups of `group` (256, 512 or 1024) consecutive
 // sorted points; perm == nullptr means the points are already in order.  valid
@@ -235,23 +236,12 @@ int gather_frames(gh_ctx* c, OrderBufs& o, const double* d_pos, const double* d_
 // tree helpers shared with the spatial order (gh_tree.hip)
 constexpr int kRsItems = 8;
 constexpr int kRsChunk = kBlock * kRsItems;  // elements per radix-sort workgroup
-// Sorts of at most this many chunks may take radix_sort_direct.
-constexpr int kRsDirectChunks = 32;
 // have_hist0: hist already holds the first pass's digit counts (k_rs_hist's layout).
 int radix_sort(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n, int words,
                int lo_shift, hipStream_t s, int* sel_out, int hi_shift = 64,
                bool have_hist0 = false);
-// One-word stable LSD sort of (keys[0], idx[0]) by bits [lo_shift, hi_shift), 8 per pass,
-// one kernel per pass, for at most kRsDirectChunks chunks.  hist holds, per pass p, the
-// digit counts of each chunk of that pass's input at hist + p * 256 * nb (digit d, chunk
-// b at d * nb + b, nb = the chunk count): pass 0's counted by the caller, the later ones
-// zero on entry (each pass counts the next pass's).
-int radix_sort_direct(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n,
-                      int lo_shift, int hi_shift, hipStream_t s, int* sel_out);
 int bbox_dev(gh_ctx* c, const double* d_pos, int64_t n, double eps, DevBuf& part, double* box,
              hipStream_t s);
-int bbox_partial_dev(gh_ctx* c, const double* d_pos, int64_t n, DevBuf& part, u32* zero,
-                     int64_t nzero, hipStream_t s, int* nparts);
 
 // tree (gh_tree.hip)
 int tree_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,

@@ -99,16 +99,11 @@ struct TreeBufs {
 // ------------------------------------------------------------------------------
 // 1. bounding box
 // ------------------------------------------------------------------------------
-// Extent of each workgroup's share of the points: part[6 b ..] = (min, max).  The
-// workgroups also clear zero[0 .. nzero) (the small sort's digit counts; may be null).
+// Extent of each workgroup's share of the points: part[6 b ..] = (min, max).
 __global__ __launch_bounds__(kBlock) void k_bbox_partial(const double* __restrict__ pos,
-                                                         int64_t n, double* __restrict__ part,
-                                                         u32* __restrict__ zero, int64_t nzero)
+                                                         int64_t n, double* __restrict__ part)
 {
     __shared__ double smin[3][kBlock], smax[3][kBlock];
-    for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < nzero;
-         j += (int64_t)gridDim.x * kBlock)
-        zero[j] = 0u;
     double mn[3], mx[3];
     for (int k = 0; k < 3; k++) mn[k] = mx[k] = pos[k];  // particle 0 seeds, as :747-750
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
@@ -285,25 +280,18 @@ __global__ __launch_bounds__(kBlock) void k_rs_scan(u32* __restrict__ hist, int 
 // wavefronts.  STAGE (one key word only): the block's elements are first placed in LDS
 // in output order and then written out by consecutive threads, so each digit's run of
 // the block leaves as contiguous stores; otherwise every element is stored directly.
-// DIRECT (STAGE only, at most kRsDirectChunks blocks): hist holds the unscanned digit
-// counts of every block, and each block forms its bases from them itself (totals is
-// unused); when hnext is not null the block also counts, per output chunk, the digits
-// of the next pass (bits shift + 8 ..) into hnext, which must be zero beforehand.
-template <bool STAGE, bool DIRECT>
+template <bool STAGE>
 __global__ __launch_bounds__(kBlock) void k_rs_scatter(
     const u64* __restrict__ kin, u64* __restrict__ kout, const u32* __restrict__ iin,
     u32* __restrict__ iout, int64_t n, int words, int wsel, int shift,
-    const u32* __restrict__ hist, int nblocks, const u32* __restrict__ totals,
-    u32* __restrict__ hnext)
+    const u32* __restrict__ hist, int nblocks, const u32* __restrict__ totals)
 {
-    static_assert(!DIRECT || STAGE, "the direct form stages its output");
     constexpr int kWaves = kBlock / 64;
     __shared__ u32 gbase0[256];          // this block's first output position per digit
     __shared__ u32 lstart[256];          // this block's first LDS slot per digit (STAGE)
     __shared__ u32 wcount[kWaves][256];  // per-wave running counts, then wave offsets
     __shared__ u64 stage_k[STAGE ? kRsChunk : 1];
     __shared__ u32 stage_i[STAGE ? kRsChunk : 1];
-    __shared__ u32 next_cnt[DIRECT ? kRsDirectChunks * 256 : 1];  // [output chunk][digit]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dd = threadIdx.x;  // one digit per thread in the per-digit steps
     const int64_t base = (int64_t)blockIdx.x * kRsChunk;
@@ -318,30 +306,6 @@ __global__ __launch_bounds__(kBlock) void k_rs_scatter(
         kw[it] = i < n ? kin[(int64_t)wsel * n + i] : 0ull;
         id[it] = i < n ? iin[i] : 0u;
     }
-    if (DIRECT) {
-        // this digit's count in every block: total, earlier blocks, this block
-        u32 tot = 0u, before = 0u, mine = 0u;
-        for (int b = 0; b < nblocks; b++) {
-            const u32 h = hist[dd * nblocks + b];
-            tot += h;
-            if (b < (int)blockIdx.x) before += h;
-            if (b == (int)blockIdx.x) mine = h;
-        }
-        gbase0[dd] = tot;
-        lstart[dd] = mine;
-        for (int j = threadIdx.x; j < kRsDirectChunks * 256; j += kBlock) next_cnt[j] = 0u;
-        __syncthreads();
-        for (int off = 1; off < 256; off <<= 1) {
-            const u32 t = dd >= off ? gbase0[dd - off] : 0u;
-            const u32 m = dd >= off ? lstart[dd - off] : 0u;
-            __syncthreads();
-            gbase0[dd] += t;
-            lstart[dd] += m;
-            __syncthreads();
-        }
-        gbase0[dd] += before - tot;  // exclusive base plus earlier blocks
-        lstart[dd] -= mine;
-    } else {
     // digit bases: exclusive scan of the 256 digit totals, plus earlier blocks
     {
         const u32 tot = totals[dd];
@@ -373,7 +337,6 @@ __global__ __launch_bounds__(kBlock) void k_rs_scatter(
             __syncthreads();
         }
         lstart[dd] -= cnt;
-    }
     }
     for (int w = 0; w < kWaves; w++) wcount[w][dd] = 0u;
     __syncthreads();
@@ -434,16 +397,6 @@ __global__ __launch_bounds__(kBlock) void k_rs_scatter(
             const u32 dst = gbase0[d] + (u32)(e - lstart[d]);
             kout[dst] = k;
             iout[dst] = stage_i[e];
-            if (DIRECT && hnext)
-                atomicAdd(&next_cnt[(dst / kRsChunk) * 256 + (u32)((k >> (shift + 8)) & 255u)],
-                          1u);
-        }
-        if (DIRECT && hnext) {
-            __syncthreads();
-            for (int j = threadIdx.x; j < nblocks * 256; j += kBlock) {
-                const u32 v = next_cnt[j];
-                if (v) atomicAdd(&hnext[(j & 255) * nblocks + (j >> 8)], v);
-            }
         }
     }
 }
@@ -2097,15 +2050,15 @@ int radix_sort(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n, in
                                hist.as<u32>() + (int64_t)256 * nblocks);
             GH_TRY(check_launch(c, "k_rs_scan"));
             if (words == 1)
-                hipLaunchKernelGGL((k_rs_scatter<true, false>), dim3(nblocks), dim3(kBlock), 0,
+                hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nblocks), dim3(kBlock), 0,
                                    s, kin, keys[sel ^ 1].as<u64>(), idx[sel].as<u32>(),
                                    idx[sel ^ 1].as<u32>(), n, words, w, shift, hist.as<u32>(),
-                                   nblocks, hist.as<u32>() + (int64_t)256 * nblocks, nullptr);
+                                   nblocks, hist.as<u32>() + (int64_t)256 * nblocks);
             else
-                hipLaunchKernelGGL((k_rs_scatter<false, false>), dim3(nblocks), dim3(kBlock), 0,
+                hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nblocks), dim3(kBlock), 0,
                                    s, kin, keys[sel ^ 1].as<u64>(), idx[sel].as<u32>(),
                                    idx[sel ^ 1].as<u32>(), n, words, w, shift, hist.as<u32>(),
-                                   nblocks, hist.as<u32>() + (int64_t)256 * nblocks, nullptr);
+                                   nblocks, hist.as<u32>() + (int64_t)256 * nblocks);
             GH_TRY(check_launch(c, "k_rs_scatter"));
             sel ^= 1;
         }
@@ -2114,46 +2067,16 @@ int radix_sort(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n, in
     return 0;
 }
 
-int radix_sort_direct(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n,
-                      int lo_shift, int hi_shift, hipStream_t s, int* sel_out)
-{
-    const int nblocks = (int)((n + kRsChunk - 1) / kRsChunk);
-    if (nblocks > kRsDirectChunks) return fail(c, GH_EARG, "internal: direct sort of %d chunks", nblocks);
-    int sel = 0;
-    u32* h = hist.as<u32>();
-    for (int shift = lo_shift; shift < hi_shift; shift += 8) {
-        u32* hn = shift + 8 < hi_shift ? h + (int64_t)256 * nblocks : nullptr;
-        hipLaunchKernelGGL((k_rs_scatter<true, true>), dim3(nblocks), dim3(kBlock), 0, s,
-                           keys[sel].as<u64>(), keys[sel ^ 1].as<u64>(), idx[sel].as<u32>(),
-                           idx[sel ^ 1].as<u32>(), n, 1, 0, shift, h, nblocks, nullptr, hn);
-        GH_TRY(check_launch(c, "k_rs_scatter"));
-        h += (int64_t)256 * nblocks;
-        sel ^= 1;
-    }
-    *sel_out = sel;
-    return 0;
-}
-
-// Extents of n points per workgroup into part (*nparts of them), clearing zero[0 ..
-// nzero) on the way.
-int bbox_partial_dev(gh_ctx* c, const double* d_pos, int64_t n, DevBuf& part, u32* zero,
-                     int64_t nzero, hipStream_t s, int* nparts)
-{
-    const int np = (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
-    GH_TRY(ensure(c, part, sizeof(double) * 6 * (size_t)np));
-    hipLaunchKernelGGL(k_bbox_partial, dim3(np), dim3(kBlock), 0, s, d_pos, n,
-                       part.as<double>(), zero, nzero);
-    *nparts = np;
-    return check_launch(c, "k_bbox_partial");
-}
-
 // Root box of the reference (centre box[0..2], size box[3], gravhopper/_jbgrav.c:747-772)
 // of n points, written to the device array box; part holds the partial extents.
 int bbox_dev(gh_ctx* c, const double* d_pos, int64_t n, double eps, DevBuf& part, double* box,
              hipStream_t s)
 {
-    int nparts = 0;
-    GH_TRY(bbox_partial_dev(c, d_pos, n, part, nullptr, 0, s, &nparts));
+    const int nparts = (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
+    GH_TRY(ensure(c, part, sizeof(double) * 6 * (size_t)nparts));
+    hipLaunchKernelGGL(k_bbox_partial, dim3(nparts), dim3(kBlock), 0, s, d_pos, n,
+                       part.as<double>());
+    GH_TRY(check_launch(c, "k_bbox_partial"));
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, s, part.as<double>(), nparts,
                        eps, box);
     return check_launch(c, "k_bbox_final");

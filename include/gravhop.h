@@ -239,9 +239,9 @@ int gh_timing_read(gh_ctx *ctx, int kernel_class, double *total_ms, int64_t *lau
  *                        partial per particle and block fits 13 GiB, else bands of
  *                        block columns, one pass each, whose partials fit it), n > 0
  *                        bands of n block columns
- *   GH_TUNE_SORT_DIRECT  spatial order of the FP32 direct sum: 0 automatic (up to 32
- *                        chunks of 2048 points, one kernel per radix pass), -1 always
- *                        the histogram, scan and scatter kernels per pass
+ *   GH_TUNE_SORT_DIRECT  spatial order of the FP32 direct sum: 0 automatic (two launches
+ *                        while points times points of the largest simulation stay within
+ *                        2^33, else radix passes), -1 always radix passes
  *   GH_TUNE_TREE_SORT    octree key sort: 0 automatic (radix passes over the digits of
  *                        levels 0-12, then each run of keys equal there sorted on its
  *                        own; a run of more than 64 keys makes the build sort over all

@@ -210,6 +210,49 @@ def test_fp32_sort_forms_agree(ctx, n):
         assert np.median(e) <= FP32_MEDIAN and np.percentile(e, 99) <= FP32_P99
 
 
+# edges of the 64-point lists, the runs of 1024 and the part one wavefront searches
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 16385, 92681, 92682])
+def test_fp32_run_sort(ctx, n):
+    # points on a coarse lattice, so that many keys are equal: ties go by index in both forms
+    rng = np.random.default_rng(n)
+    pos = rng.integers(0, 6, size=(n, 3)).astype(np.float64)
+    mass = rng.uniform(0.5, 1.0, size=n)
+    fpos = rng.normal(size=(77, 3))
+    got = ctx.direct(pos, mass, 0.1, FP32), ctx.direct(pos, mass, 0.1, FP32, force_pos=fpos)
+    ctx.set_tuning(_native.TUNE_SORT_DIRECT, -1)
+    try:
+        want = ctx.direct(pos, mass, 0.1, FP32), ctx.direct(pos, mass, 0.1, FP32, force_pos=fpos)
+    finally:
+        ctx.set_tuning(_native.TUNE_SORT_DIRECT, 0)
+    for g, w in zip(got, want):
+        assert_bitwise(g, w, "n=%d" % n)
+
+
+@pytest.mark.parametrize("ipt", [1, 2, 4])  # runs of 256, 512 and 1024 places
+def test_fp32_run_sort_of_segments(ctx, ipt):
+    sims = []
+    for k, n in enumerate([1, 255, 256, 257, 513, 1024, 1025, 5000]):
+        ic = workloads.plummer(n, seed=k) if n > 1 else {"pos": np.ones((1, 3)),
+                                                         "vel": np.zeros((1, 3)),
+                                                         "mass": np.ones(1)}
+        ic["eps"], ic["dt"] = 1e-5, 1e-4
+        sims.append(ic)
+
+    def run(form):
+        ctx.set_tuning(_native.TUNE_SORT_DIRECT, form)
+        try:
+            ens = _native.Ensemble(ctx, sims, ipt=ipt)
+            ens.run(3)
+            state = [np.concatenate(a) for a in ens.state()]
+            ens.close()
+            return state
+        finally:
+            ctx.set_tuning(_native.TUNE_SORT_DIRECT, 0)
+
+    for k, (got, want) in enumerate(zip(run(0), run(-1))):
+        assert_bitwise(got, want, "array %d" % k)
+
+
 # either side of every change of kernel shape (f64_shape in gh_direct.hip)
 @pytest.mark.parametrize("nf", [1, 256, 257, 768, 769, 1024, 1025, 2048, 2049, 3072, 3073, 4096,
                                 4097, 6500, 6501, 8192, 8193, 16384, 16385, 24576, 24577])
