@@ -8,7 +8,6 @@
 
 namespace gh {
 
-int set_slot(gh_ctx* c, long long* slot, long long value, int add, hipStream_t s);
 int energy_dev(gh_ctx* c, const double* d_pos, const double* d_vel, const double* d_mass,
                int64_t n, double eps, double* d_out5, hipStream_t s);
 
@@ -160,13 +159,11 @@ static int check_common(gh_ctx* c, int64_t np, int64_t nf, double eps, int preci
     return 0;
 }
 
-// One step: force at xh, then the fused kick/drift/half-drift.  slot != nullptr: the
-// history slot is read on the device (graph replay), and *slot_next becomes *slot + 1;
-// otherwise hp/hv point at the step's snapshot.
+// One step: force at xh, then the fused kick/drift/half-drift; hp / hv (nullable) receive the
+// step's snapshot.
 static int one_step(gh_ctx* c, double* x, double* v, const double* m, int64_t np,
                     double dt, double eps, int algorithm, double theta, int precision,
-                    double* hp, double* hv, const long long* slot, hipStream_t s,
-                    long long* slot_next = nullptr)
+                    double* hp, double* hv, hipStream_t s)
 {
     const int64_t n3 = 3 * np;
     double* xh = c->xh.as<double>();
@@ -181,7 +178,7 @@ static int one_step(gh_ctx* c, double* x, double* v, const double* m, int64_t np
         GH_TRY(zero_dev(c, acc, n3, s));
     }
     TimedScope ts(c, s, GH_T_UPDATE);
-    return kick_drift(c, acc, np, dt, xh, v, x, hp, hv, s, slot, nullptr, slot_next);
+    return kick_drift(c, acc, np, dt, xh, v, x, hp, hv, s);
 }
 
 // Copies a run's device history to host memory in slices of steps, on the copy stream,
@@ -250,18 +247,17 @@ struct HistCopier {
     bool complete() const { return on && marked == nsteps && issued == slices.size(); }
 };
 
-// nsteps DKD steps on device state; d_hist_* (nullable) receive (nsteps, n, 3).
-// Direct-sum runs replay two captured steps as one HIP graph after a first eager step
-// (which sizes every buffer); an odd last step runs eagerly.  In the graph the history
-// slot comes from two device counters that the steps' update kernels advance in turn
-// (step A reads slot[0] and writes slot[1] = slot[0] + 1, step B the reverse), so a step
-// is two launches.  The tree's build reads its node count back to the host, so tree
-// runs stay eager.
+// nsteps DKD steps on device state; d_hist_* (nullable) receive (nsteps, n, 3).  Every kernel
+// is launched on its own: the host queues one in 2.6 us, and the shortest kernel takes 4, so
+// the queue runs ahead of the device.  (Direct-sum runs replayed graphs of two steps before.
+// Between two replays the device stood still for 8 to 13 us: 50 steps took 8.6 us each at 100
+// particles in FP64, 20.0 at 2000 and 41.8 at 3000 in FP32, and take 5.6, 17.4 and 39.7.)
 // out_p / out_v (nullable, host memory; needs the context's copy stream): the run copies
 // its history there itself while later steps still run, and sets *copied; otherwise the
-// caller copies the device history afterwards.  Replayed runs queue every step first and
-// then copy slices of at least 8 steps (at most about 16); eager runs copy slices of
-// about 16 MiB, each after the next step has been queued.
+// caller copies the device history afterwards.  Direct-sum runs queue every step first and
+// then copy slices of at least 8 steps (at most about 16).  The tree's build reads its node
+// count back to the host, so a tree run copies slices of about 16 MiB, each after the next
+// step has been queued.
 static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t np, double dt,
                      double eps, int algorithm, double theta, int precision, int64_t nsteps,
                      double* hist_p, double* hist_v, hipStream_t s, double* out_p = nullptr,
@@ -270,75 +266,38 @@ static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t n
     if (copied) *copied = false;
     if (np == 0 || nsteps == 0) return 0;
     const int64_t n3 = 3 * np;
+    const bool ahead = algorithm == GH_DIRECT;
+    if (ahead && nsteps >= 4) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        GH_HIP(c, hipStreamIsCapturing(s, &cap));
+        if (cap != hipStreamCaptureStatusNone)
+            return fail(c, GH_EHIP, "a direct-sum run of %lld steps cannot be captured",
+                        (long long)nsteps);
+    }
     GH_TRY(ensure(c, c->xh, sizeof(double) * (size_t)n3));
     GH_TRY(ensure(c, c->acc64, sizeof(double) * (size_t)n3));
     GH_TRY(half_drift(c, x, v, np, dt, c->xh.as<double>(), s));
-    GH_TRY(one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision, hist_p, hist_v,
-                    nullptr, s));
-    const bool graph = algorithm == GH_DIRECT && !c->timing && nsteps >= 4 &&
-                       c->tune[GH_TUNE_RUN_GRAPH] >= 0;
-    if (!graph) {
-        const int64_t step_bytes = (int64_t)sizeof(double) * n3 * 2;
-        HistCopier hc(c, s, n3, nsteps, std::max<int64_t>(1, ((int64_t)16 << 20) / step_bytes),
-                      hist_p, hist_v, out_p, out_v);
-        GH_TRY(hc.mark(1));
-        for (int64_t st = 1; st < nsteps; st++) {
-            GH_TRY(one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision,
-                            hist_p ? hist_p + st * n3 : nullptr,
-                            hist_v ? hist_v + st * n3 : nullptr, nullptr, s));
-            // step st is queued: copy every slice recorded before it
-            GH_TRY(hc.issue(hc.slices.size()));
-            GH_TRY(hc.mark(st + 1));
-        }
-        GH_TRY(hc.finish());
-        if (copied) *copied = hc.complete();
-        return 0;
+    const int64_t step_bytes = (int64_t)sizeof(double) * n3 * 2;
+    HistCopier hc(c, s, n3, nsteps,
+                  ahead ? std::max<int64_t>(8, (nsteps + 15) / 16)
+                        : std::max<int64_t>(1, ((int64_t)16 << 20) / step_bytes),
+                  hist_p, hist_v, out_p, out_v);
+    for (int64_t st = 0; st < nsteps; st++) {
+        GH_TRY(one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision,
+                        hist_p ? hist_p + st * n3 : nullptr, hist_v ? hist_v + st * n3 : nullptr,
+                        s));
+        // step st is queued: copy every slice recorded before it
+        if (!ahead) GH_TRY(hc.issue(hc.slices.size()));
+        GH_TRY(hc.mark(st + 1));
     }
-    GH_TRY(ensure(c, c->slot, 256));
-    long long* slot = c->slot.as<long long>();
-    GH_TRY(set_slot(c, slot, 1, 0, s));
-    GH_HIP(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int rc = one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision, hist_p, hist_v,
-                      slot, s, slot + 1);
-    if (!rc)
-        rc = one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision, hist_p, hist_v,
-                      slot + 1, s, slot);
-    hipGraph_t g = nullptr;
-    const hipError_t ee = hipStreamEndCapture(s, &g);
-    if (rc) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-    }
-    if (ee != hipSuccess)
-        return fail(c, GH_EHIP, "step capture failed: %s", hipGetErrorString(ee));
-    hipGraphExec_t ex = nullptr;
-    const hipError_t ie = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (ie != hipSuccess)
-        return fail(c, GH_EHIP, "step graph instantiation failed: %s", hipGetErrorString(ie));
-    {
-        HistCopier hc(c, s, n3, nsteps, std::max<int64_t>(8, (nsteps + 15) / 16), hist_p,
-                      hist_v, out_p, out_v);
-        if (!rc) rc = hc.mark(1);
-        int64_t st = 1;
-        for (; st + 1 < nsteps && !rc; st += 2) {
-            if (hipGraphLaunch(ex, s) != hipSuccess) rc = fail(c, GH_EHIP, "graph launch failed");
-            if (!rc) rc = hc.mark(st + 2);
-        }
-        if (!rc && st < nsteps) {
-            rc = one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision,
-                          hist_p ? hist_p + st * n3 : nullptr,
-                          hist_v ? hist_v + st * n3 : nullptr, nullptr, s);
-            if (!rc) rc = hc.mark(nsteps);
-        }
-        // every step is queued: copy the slices out as they complete
-        if (!rc) rc = hc.finish();
-        if (!rc && copied) *copied = hc.complete();
-    }
-    // the executable graph may be destroyed once its launches are enqueued
-    (void)hipStreamSynchronize(s);
-    (void)hipGraphExecDestroy(ex);
-    return rc;
+    GH_TRY(hc.finish());
+    if (copied) *copied = hc.complete();
+    // A long queue is drained here, as a replayed run's was.  A later call on another stream
+    // would have to wait for it on the device, and there the switch takes 115 us longer (16
+    // steps of 3000 particles in FP32 on three streams in turn: 672 us a run, 745 without
+    // this; on one stream 672 and 632).
+    if (ahead && nsteps >= 4) GH_HIP(c, hipStreamSynchronize(s));
+    return 0;
 }
 
 // nsteps DKD steps on device state with external accelerations from a host callback
@@ -396,7 +355,7 @@ static int run_ext_steps(gh_ctx* c, double* x, double* v, const double* m, int64
         {
             TimedScope ts(c, s, GH_T_UPDATE);
             GH_TRY(kick_drift(c, acc, np, dt, xh, v, x, hist_p ? hist_p + st * n3 : nullptr,
-                              hist_v ? hist_v + st * n3 : nullptr, s, nullptr, ext));
+                              hist_v ? hist_v + st * n3 : nullptr, s, ext));
         }
         *t = *t + dt;
         GH_TRY(hc.mark(st + 1));
@@ -453,7 +412,7 @@ void gh_ctx_destroy(gh_ctx* c)
                       &c->src32a, &c->src32b, &c->tgt32,  &c->xs,    &c->vs,
                       &c->xh,     &c->hist_p, &c->hist_v, &c->scratch, &c->counters,
                       &c->work,   &c->eps_blk, &c->adj_work, &c->adj_src, &c->adj_mu,
-                      &c->adj_mv, &c->adj_part, &c->adj_seg, &c->adj_perm, &c->slot};
+                      &c->adj_mv, &c->adj_part, &c->adj_seg, &c->adj_perm};
     for (DevBuf* b : bufs) release(c, *b);
     release(c, c->ext);
     for (OrderBufs* o : {&c->ord_p, &c->ord_t}) {

@@ -77,7 +77,6 @@ struct gh_ctx {
     // adjoint workspaces (gh_adjoint.hip)
     gh::DevBuf adj_work, adj_src, adj_mu, adj_mv, adj_part, adj_seg, adj_perm;
     int adj_nb = -1, adj_ipt = -1;
-    gh::DevBuf slot;  // history slot counter of graph-replayed runs
     gh::OrderBufs ord_p, ord_t;  // spatial order of sources and of targets (FP32 paths)
     // the stream of the last entry-point call and an event recorded at its end: a call
     // on another stream waits for it first (StreamOrder), since all calls share the
@@ -201,15 +200,12 @@ int reduce_sym(gh_ctx* c, const float* part, int nb, const int* nb_blk, int blk,
                int64_t np_pad, int64_t n, const u32* perm, double* acc, hipStream_t s);
 
 // leapfrog update (gh_step.hip).  kick_drift: ext (nullable) is an extra acceleration
-// in km/s/Myr added to the N-body one, as a = acc*A + ext; slot (nullable) is the
-// history slot counter of graph-replayed runs, and slot_next (nullable) receives
-// *slot + 1.
+// in km/s/Myr added to the N-body one, as a = acc*A + ext.
 int half_drift(gh_ctx* c, const double* x, const double* v, int64_t n, double dt, double* xh,
                hipStream_t s);
 int kick_drift(gh_ctx* c, const double* acc, int64_t n, double dt, double* xh, double* v,
                double* x, double* hp, double* hv, hipStream_t s,
-               const long long* slot = nullptr, const double* ext = nullptr,
-               long long* slot_next = nullptr);
+               const double* ext = nullptr);
 
 // spatial order and frames (gh_frames.hip)
 constexpr int kFrameLog2 = 10;  // a group is flagged when R > 2^kFrameLog2 x its mean gap
