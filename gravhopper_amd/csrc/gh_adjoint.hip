@@ -485,20 +485,26 @@ static int forward_segment(gh_ctx* c, double* x, double* v, const double* m, int
     const int64_t n3 = 3 * n;
     GH_TRY(ensure(c, c->xh, sizeof(double) * (size_t)n3));
     GH_TRY(ensure(c, c->acc64, sizeof(double) * (size_t)n3));
-    double* xh = c->xh.as<double>();
     double* acc = c->acc64.as<double>();
     if (have) have->assign((size_t)len, 0);
-    GH_TRY(half_drift(c, x, v, n, dt, xh, s));
+    StepUpdate up;
+    up.xh = up.xh_next = hx ? hx : c->xh.as<double>();
+    up.v = v;
+    up.x = x;
+    up.dt = dt;
+    GH_TRY(half_drift(c, x, v, n, dt, up.xh_next, s));
     for (int64_t st = 0; st < len; st++) {
+        const double* xh = up.xh;
+        bool updated = false;
         if (hx) {
-            GH_TRY(copy_d(c, xh, hx + st * n3, n3, s));
             // the reverse sweep needs only the last step's half-step positions
             if (st == len - 1) break;
+            up.xh_next = hx + (st + 1) * n3;
         }
         if (n > 1) {
             OrderBufs& o = c->ord_p;
             o.sorted = nullptr;
-            GH_TRY(direct_dev(c, xh, m, n, nullptr, n, eps, precision, acc, s));
+            GH_TRY(direct_dev(c, xh, m, n, nullptr, n, eps, precision, acc, s, &up, &updated));
             if (hperm && have && o.sorted == xh && o.sorted_n == n) {
                 hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
                                    o.perm(), hperm + st * n, n);
@@ -508,7 +514,8 @@ static int forward_segment(gh_ctx* c, double* x, double* v, const double* m, int
         } else {
             GH_TRY(zero_dev(c, acc, n3, s));
         }
-        GH_TRY(kick_drift(c, acc, n, dt, xh, v, x, nullptr, nullptr, s));
+        if (!updated) GH_TRY(kick_drift(c, acc, n, up, s));
+        up.xh = up.xh_next;
     }
     return 0;
 }

@@ -159,26 +159,26 @@ static int check_common(gh_ctx* c, int64_t np, int64_t nf, double eps, int preci
     return 0;
 }
 
-// One step: force at xh, then the fused kick/drift/half-drift; hp / hv (nullable) receive the
-// step's snapshot.
-static int one_step(gh_ctx* c, double* x, double* v, const double* m, int64_t np,
-                    double dt, double eps, int algorithm, double theta, int precision,
-                    double* hp, double* hv, hipStream_t s)
+// One step: force at up.xh, then the fused kick/drift/half-drift.
+static int one_step(gh_ctx* c, const double* m, int64_t np, double eps, int algorithm,
+                    double theta, int precision, const StepUpdate& up, hipStream_t s)
 {
     const int64_t n3 = 3 * np;
-    double* xh = c->xh.as<double>();
+    const double* xh = up.xh;
+    bool updated = false;
     double* acc = c->acc64.as<double>();
     if (np > 1) {
         if (algorithm == GH_DIRECT)
-            GH_TRY(direct_dev(c, xh, m, np, nullptr, np, eps, precision, acc, s));
+            GH_TRY(direct_dev(c, xh, m, np, nullptr, np, eps, precision, acc, s, &up, &updated));
         else
             GH_TRY(tree_dev(c, xh, m, np, nullptr, np, eps, theta, precision, acc, s));
     } else {
         // gravhopper.py:442,449-450: a single particle feels no N-body force
         GH_TRY(zero_dev(c, acc, n3, s));
     }
+    if (updated) return 0;
     TimedScope ts(c, s, GH_T_UPDATE);
-    return kick_drift(c, acc, np, dt, xh, v, x, hp, hv, s);
+    return kick_drift(c, acc, np, up, s);
 }
 
 // Copies a run's device history to host memory in slices of steps, on the copy stream,
@@ -274,8 +274,16 @@ static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t n
             return fail(c, GH_EHIP, "a direct-sum run of %lld steps cannot be captured",
                         (long long)nsteps);
     }
-    GH_TRY(ensure(c, c->xh, sizeof(double) * (size_t)n3));
+    // steps take the two halves in turn where the update must not be in place
+    const bool two = ahead && precision == GH_FP64 && np <= kF64RelayMax;
+    GH_TRY(ensure(c, c->xh, sizeof(double) * (two ? 2 : 1) * (size_t)n3));
     GH_TRY(ensure(c, c->acc64, sizeof(double) * (size_t)n3));
+    StepUpdate up;
+    up.xh = c->xh.as<double>();
+    up.xh_next = c->xh.as<double>() + (two ? n3 : 0);
+    up.v = v;
+    up.x = x;
+    up.dt = dt;
     GH_TRY(half_drift(c, x, v, np, dt, c->xh.as<double>(), s));
     const int64_t step_bytes = (int64_t)sizeof(double) * n3 * 2;
     HistCopier hc(c, s, n3, nsteps,
@@ -283,9 +291,12 @@ static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t n
                         : std::max<int64_t>(1, ((int64_t)16 << 20) / step_bytes),
                   hist_p, hist_v, out_p, out_v);
     for (int64_t st = 0; st < nsteps; st++) {
-        GH_TRY(one_step(c, x, v, m, np, dt, eps, algorithm, theta, precision,
-                        hist_p ? hist_p + st * n3 : nullptr, hist_v ? hist_v + st * n3 : nullptr,
-                        s));
+        up.hist_p = hist_p ? hist_p + st * n3 : nullptr;
+        up.hist_v = hist_v ? hist_v + st * n3 : nullptr;
+        GH_TRY(one_step(c, m, np, eps, algorithm, theta, precision, up, s));
+        double* next = up.xh_next;
+        up.xh_next = const_cast<double*>(up.xh);
+        up.xh = next;
         // step st is queued: copy every slice recorded before it
         if (!ahead) GH_TRY(hc.issue(hc.slices.size()));
         GH_TRY(hc.mark(st + 1));
@@ -328,6 +339,11 @@ static int run_ext_steps(gh_ctx* c, double* x, double* v, const double* m, int64
     HistCopier hc(c, s, n3, nsteps,
                   std::max<int64_t>(1, ((int64_t)16 << 20) / (int64_t)(2 * bytes)), hist_p,
                   hist_v, out_p, out_v);
+    StepUpdate up;
+    up.xh = up.xh_next = xh;
+    up.v = v;
+    up.x = x;
+    up.dt = dt;
     GH_TRY(half_drift(c, x, v, np, dt, xh, s));
     for (int64_t st = 0; st < nsteps; st++) {
         GH_HIP(c, hipEventRecord(ready, s));
@@ -354,8 +370,9 @@ static int run_ext_steps(gh_ctx* c, double* x, double* v, const double* m, int64
         GH_HIP(c, hipStreamWaitEvent(s, back, 0));
         {
             TimedScope ts(c, s, GH_T_UPDATE);
-            GH_TRY(kick_drift(c, acc, np, dt, xh, v, x, hist_p ? hist_p + st * n3 : nullptr,
-                              hist_v ? hist_v + st * n3 : nullptr, s, ext));
+            up.hist_p = hist_p ? hist_p + st * n3 : nullptr;
+            up.hist_v = hist_v ? hist_v + st * n3 : nullptr;
+            GH_TRY(kick_drift(c, acc, np, up, s, ext));
         }
         *t = *t + dt;
         GH_TRY(hc.mark(st + 1));

@@ -69,7 +69,8 @@ __device__ __forceinline__ void lds_barrier()
 template <bool SELF, int P, int K>
 __global__ __launch_bounds__((P + 1) * 64) void k_direct_f64_relay(
     const double* __restrict__ pos, const double* __restrict__ mass, int64_t np,
-    const double* __restrict__ tgt, int64_t nt, double eps2, double* __restrict__ acc)
+    const double* __restrict__ tgt, int64_t nt, double eps2, double* __restrict__ acc,
+    StepUpdate up)
 {
     constexpr int T = P * K, NS = 3 * T, CH = 128;
     static_assert(NS <= 64, "one lane per sum");
@@ -113,7 +114,12 @@ __global__ __launch_bounds__((P + 1) * 64) void k_direct_f64_relay(
             f = f + v[1][k].x;
             f = f + v[1][k].y;
         }
-        if (lane < NS && i0 + lane / 3 < nt) acc[3 * i0 + lane] = f;
+        if (lane < NS && i0 + lane / 3 < nt) {
+            if (SELF && up.v)
+                update_one(up, 3 * i0 + lane, f);
+            else
+                acc[3 * i0 + lane] = f;
+        }
         return;
     }
     double xt[K], yt[K], zt[K];
@@ -342,8 +348,6 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
 //   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   91367
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
 // 3001 targets of 65536 sources: 468 (before 1300); 200 of 100000: 393 (1062).
-constexpr int64_t kF64RelayMax = 6500;
-
 enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
 struct F64Shape {
     int targets;  // relay: per workgroup
@@ -398,25 +402,19 @@ __device__ __forceinline__ void split_ds(double d, float& hi, float& lo)
 // wave-wide broadcasts, FP32 sums per tile and an FP32 two-sum (hi, lo) across tiles;
 // FP64 out.  Workgroup b holds the sorted targets of group b (256 IPT of them), whose
 // frame is tframe[b]; every source tile is re-based into that frame from the FP64
-// sources (src64, any order, massless padding).  A workgroup runs only in the
-// instance matching its group's flag (DS = 1: double-single separations).  Sources may
+// sources (src64, any order, massless padding).  DS: the group is flagged, and its
+// separations are double-single.  (A launch of its own for the flagged groups, which are
+// few or none, cost 4 us.)  Sources may
 // be split over grid.y when there are too few targets to fill 256 CUs; the splits are
 // added in split order.  perm (sorted target -> caller's index) places the results;
 // with splits the per-split fields go to out in sorted order instead.
 template <int IPT, bool GUARD, bool DS>
-__global__ __launch_bounds__(kBlock) void k_direct_f32(const double4* __restrict__ src64,
-                                                       int64_t np_pad, int64_t j_per_split,
-                                                       const float4* __restrict__ tloc,
-                                                       const double4* __restrict__ t64,
-                                                       const double4* __restrict__ tframe,
-                                                       const int* __restrict__ tflag,
-                                                       const u32* __restrict__ perm,
-                                                       int64_t nt, float eps2,
-                                                       double* __restrict__ out)
+__device__ __forceinline__ void one_sided_group(
+    float4 (&tile)[kBlock], float4 (&tile_lo)[kBlock], const double4* __restrict__ src64,
+    int64_t np_pad, int64_t j_per_split, const float4* __restrict__ tloc,
+    const double4* __restrict__ t64, const double4* __restrict__ tframe,
+    const u32* __restrict__ perm, int64_t nt, float eps2, double* __restrict__ out)
 {
-    __shared__ float4 tile[kBlock];
-    __shared__ float4 tile_lo[DS ? kBlock : 1];
-    if ((tflag[blockIdx.x] != 0) != DS) return;
     const double4 o = tframe[blockIdx.x];
     const int64_t i0 = (int64_t)blockIdx.x * (kBlock * IPT) + threadIdx.x;
     const int64_t j_begin = (int64_t)blockIdx.y * j_per_split;
@@ -514,6 +512,26 @@ __global__ __launch_bounds__(kBlock) void k_direct_f32(const double4* __restrict
             d[2] = (double)hz[k] + (double)lz[k];
         }
     }
+}
+
+template <int IPT, bool GUARD>
+__global__ __launch_bounds__(kBlock) void k_direct_f32(const double4* __restrict__ src64,
+                                                       int64_t np_pad, int64_t j_per_split,
+                                                       const float4* __restrict__ tloc,
+                                                       const double4* __restrict__ t64,
+                                                       const double4* __restrict__ tframe,
+                                                       const int* __restrict__ tflag,
+                                                       const u32* __restrict__ perm,
+                                                       int64_t nt, float eps2,
+                                                       double* __restrict__ out)
+{
+    __shared__ float4 tile[kBlock], tile_lo[kBlock];
+    if (tflag[blockIdx.x] == 0)
+        one_sided_group<IPT, GUARD, false>(tile, tile_lo, src64, np_pad, j_per_split, tloc, t64,
+                                           tframe, perm, nt, eps2, out);
+    else
+        one_sided_group<IPT, GUARD, true>(tile, tile_lo, src64, np_pad, j_per_split, tloc, t64,
+                                          tframe, perm, nt, eps2, out);
 }
 
 // ------------------------------------------------------------------------------
@@ -793,7 +811,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_sym(const float* __restrict__
                                                        const int* __restrict__ nb_blk,
                                                        int blk, int64_t np_pad, int64_t n3,
                                                        const u32* __restrict__ perm,
-                                                       double* __restrict__ acc)
+                                                       double* __restrict__ acc, StepUpdate up)
 {
     // Each workgroup takes 64 groups of 4 floats, one per lane; its wavefront w adds the
     // slots w, w + kSlotLanes, ... in order (so each load reads 64 consecutive float4),
@@ -823,7 +841,11 @@ __global__ __launch_bounds__(kBlock) void k_reduce_sym(const float* __restrict__
     if (k0 < n3 && k < n3) {
         const double t = (sh[0][w][lane] + sh[1][w][lane]) + (sh[2][w][lane] + sh[3][w][lane]);
         const int64_t q = k / 3;
-        acc[perm ? 3 * (int64_t)perm[q] + (k - 3 * q) : k] = t;
+        const int64_t at = perm ? 3 * (int64_t)perm[q] + (k - 3 * q) : k;
+        if (up.v)
+            update_one(up, at, t);
+        else
+            acc[at] = t;
     }
 }
 
@@ -858,18 +880,29 @@ __global__ __launch_bounds__(kBlock) void k_reduce_band(const float* __restrict_
 }
 
 // Sum of per-split partial fields (sorted target order), in split order, written to
-// acc[perm[i]].
+// acc[perm[i]], or the particles' update with it.
 __global__ __launch_bounds__(kBlock) void k_reduce_splits(const double* __restrict__ part,
                                                           int splits, int64_t n3,
                                                           const u32* __restrict__ perm,
-                                                          double* __restrict__ acc)
+                                                          double* __restrict__ acc,
+                                                          StepUpdate up)
 {
     const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (k >= n3) return;
-    double s = part[k];
-    for (int p = 1; p < splits; p++) s += part[(int64_t)p * n3 + k];
     const int64_t q = k / 3;
-    acc[3 * (int64_t)perm[q] + (k - 3 * q)] = s;
+    const int64_t at = 3 * (int64_t)perm[q] + (k - 3 * q);
+    double s = part[k];
+    int p = 1;
+    for (; p + 4 <= splits; p += 4) {  // four loads in flight
+        const double a = part[(int64_t)p * n3 + k], b = part[(int64_t)(p + 1) * n3 + k];
+        const double d = part[(int64_t)(p + 2) * n3 + k], e = part[(int64_t)(p + 3) * n3 + k];
+        s = (((s + a) + b) + d) + e;
+    }
+    for (; p < splits; p++) s += part[(int64_t)p * n3 + k];
+    if (up.v)
+        update_one(up, at, s);
+    else
+        acc[at] = s;
 }
 
 // (x, y, z, m) in input order, entries n..n_pad-1 massless at the origin
@@ -917,15 +950,15 @@ F32Shape pick_shape(gh_ctx* c, int64_t nt, int64_t np_pad)
 
 template <int P, int K>
 void launch_relay(bool self, const double* pos, const double* mass, int64_t np, const double* tgt,
-                  int64_t nt, double eps2, double* acc, hipStream_t s)
+                  int64_t nt, double eps2, double* acc, const StepUpdate& up, hipStream_t s)
 {
     const dim3 grid((unsigned)((nt + P * K - 1) / (P * K))), block((P + 1) * 64);
     if (self)
         hipLaunchKernelGGL((k_direct_f64_relay<true, P, K>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc);
+                           tgt, nt, eps2, acc, up);
     else
         hipLaunchKernelGGL((k_direct_f64_relay<false, P, K>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc);
+                           tgt, nt, eps2, acc, up);
 }
 
 template <int W, int H>
@@ -944,7 +977,7 @@ void launch_ring(bool self, const double* pos, const double* mass, int64_t np, c
                            tgt, nt, eps2, acc);
 }
 
-template <int IPT, bool DS>
+template <int IPT>
 void launch_f32(bool guard, dim3 grid, hipStream_t s, const double4* src64, int64_t np_pad,
                 int64_t jps, const OrderBufs& t, int64_t nt, float eps2, double* out)
 {
@@ -954,10 +987,10 @@ void launch_f32(bool guard, dim3 grid, hipStream_t s, const double4* src64, int6
     const int* fl = t.flag.as<int>();
     const u32* perm = t.perm();
     if (guard)
-        hipLaunchKernelGGL((k_direct_f32<IPT, true, DS>), grid, dim3(kBlock), 0, s, src64,
+        hipLaunchKernelGGL((k_direct_f32<IPT, true>), grid, dim3(kBlock), 0, s, src64,
                            np_pad, jps, tloc, t64, fr, fl, perm, nt, eps2, out);
     else
-        hipLaunchKernelGGL((k_direct_f32<IPT, false, DS>), grid, dim3(kBlock), 0, s, src64,
+        hipLaunchKernelGGL((k_direct_f32<IPT, false>), grid, dim3(kBlock), 0, s, src64,
                            np_pad, jps, tloc, t64, fr, fl, perm, nt, eps2, out);
 }
 
@@ -1034,13 +1067,14 @@ int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4*
 }
 
 int reduce_sym(gh_ctx* c, const float* part, int nb, const int* nb_blk, int blk,
-               int64_t np_pad, int64_t n, const u32* perm, double* acc, hipStream_t s)
+               int64_t np_pad, int64_t n, const u32* perm, double* acc, hipStream_t s,
+               const StepUpdate* up)
 {
     if (n <= 0) return 0;
     if ((np_pad * 3) % 4 != 0 || (3 * blk) % 4 != 0)
         return fail(c, GH_EARG, "partial slabs are not 16-byte aligned");
     hipLaunchKernelGGL(k_reduce_sym, dim3(blocks_for((3 * n + 3) / 4, 64)), dim3(kBlock), 0, s,
-                       part, nb, nb_blk, blk, np_pad, 3 * n, perm, acc);
+                       part, nb, nb_blk, blk, np_pad, 3 * n, perm, acc, up ? *up : StepUpdate());
     return check_launch(c, "k_reduce_sym");
 }
 
@@ -1051,7 +1085,7 @@ __global__ void k_fill_f32(float* __restrict__ p, int64_t n, float v)
 }
 
 int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np, int ipt,
-               double eps, double* d_acc, hipStream_t s)
+               double eps, double* d_acc, hipStream_t s, const StepUpdate* up, bool* updated)
 {
     const int64_t blk = (int64_t)kBlock * ipt;
     const int64_t np_pad = pad_to(np, blk);
@@ -1111,7 +1145,8 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
                               o.umass.as<float>(), nullptr, nb, np_pad, c->work.as<int4>(), items,
                               c->eps_blk.as<float>(), part, nullptr, 0, s));
         }
-        return reduce_sym(c, part, nb, nullptr, (int)blk, np_pad, np, o.perm(), d_acc, s);
+        if (up) *updated = true;
+        return reduce_sym(c, part, nb, nullptr, (int)blk, np_pad, np, o.perm(), d_acc, s, up);
     }
     float* partj = part + 3 * (size_t)np_pad * w;
     for (int b = 0; b < bands; b++) {
@@ -1138,7 +1173,8 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
 // 256 x the chosen targets per lane.
 static int direct_f32_onesided(gh_ctx* c, const double4* src64, int64_t np_pad, OrderBufs& t,
                                int64_t nt, const F32Shape& sh, double eps, double* d_acc,
-                               hipStream_t s)
+                               hipStream_t s, const StepUpdate* up = nullptr,
+                               bool* updated = nullptr)
 {
     if (nt <= 0) return 0;
     if (np_pad % kBlock != 0) return fail(c, GH_EARG, "internal: source count not padded");
@@ -1156,16 +1192,13 @@ static int direct_f32_onesided(gh_ctx* c, const double4* src64, int64_t np_pad, 
         TimedScope ts(c, s, GH_T_DIRECT_F32);
         switch (sh.ipt) {
             case 1:
-                launch_f32<1, false>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
-                launch_f32<1, true>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
+                launch_f32<1>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
                 break;
             case 2:
-                launch_f32<2, false>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
-                launch_f32<2, true>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
+                launch_f32<2>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
                 break;
             case 4:
-                launch_f32<4, false>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
-                launch_f32<4, true>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
+                launch_f32<4>(guard, grid, s, src64, np_pad, jps, t, nt, eps2, out);
                 break;
             default: return fail(c, GH_EARG, "unsupported targets-per-lane %d", sh.ipt);
         }
@@ -1173,7 +1206,8 @@ static int direct_f32_onesided(gh_ctx* c, const double4* src64, int64_t np_pad, 
     }
     if (splits > 1) {
         hipLaunchKernelGGL(k_reduce_splits, dim3(blocks_for(3 * nt, kBlock)), dim3(kBlock), 0,
-                           s, out, splits, 3 * nt, t.perm(), d_acc);
+                           s, out, splits, 3 * nt, t.perm(), d_acc, up ? *up : StepUpdate());
+        if (up) *updated = true;
         GH_TRY(check_launch(c, "k_reduce_splits"));
     }
     return 0;
@@ -1181,8 +1215,10 @@ static int direct_f32_onesided(gh_ctx* c, const double4* src64, int64_t np_pad, 
 
 int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
                const double* d_fpos, int64_t nf, double eps, int precision, double* d_acc,
-               hipStream_t s)
+               hipStream_t s, const StepUpdate* up, bool* updated)
 {
+    // timed runs keep the update apart, in its own class
+    if (c->timing) up = nullptr;
     const bool self = (d_fpos == nullptr);
     const double* tgt = self ? d_pos : d_fpos;
     const int64_t nt = self ? np : nf;
@@ -1196,14 +1232,17 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
         const F64Shape sh = f64_shape(c, nt);
         if (sh.ring == F64Ring::none) {
             TimedScope ts(c, s, GH_T_DIRECT_F64);
+            const bool fuse = up && up->xh_next != up->xh;  // other workgroups read xh
+            const StepUpdate u = fuse ? *up : StepUpdate();
+            if (fuse) *updated = true;
             switch (sh.targets) {
-            case 1: launch_relay<1, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            case 3: launch_relay<3, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            case 4: launch_relay<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            case 6: launch_relay<3, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            case 8: launch_relay<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            case 12: launch_relay<6, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
-            default: launch_relay<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+            case 1: launch_relay<1, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            case 3: launch_relay<3, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            case 4: launch_relay<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            case 6: launch_relay<3, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            case 8: launch_relay<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            case 12: launch_relay<6, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
+            default: launch_relay<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
             }
             return check_launch(c, "k_direct_f64_relay");
         }
@@ -1224,7 +1263,7 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     }
     if (precision != GH_FP32) return fail(c, GH_EARG, "unknown precision %d", precision);
     const int sym = self ? sym_ipt(c, np) : 0;
-    if (sym > 0) return direct_sym(c, d_pos, d_mass, np, sym, eps, d_acc, s);
+    if (sym > 0) return direct_sym(c, d_pos, d_mass, np, sym, eps, d_acc, s, up, updated);
     F32Shape sh = pick_shape(c, nt, pad_to(np, kBlock));
     const int forced = c->tune[GH_TUNE_DIRECT_IPT];
     if (forced == 1 || forced == 2 || forced == 4) sh.ipt = forced;
@@ -1236,7 +1275,8 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
         OrderBufs& o = c->ord_p;
         GH_TRY(spatial_order(c, o, d_pos, np, s));
         GH_TRY(gather_frames(c, o, d_pos, d_mass, o.perm(), np, nt_pad, group, nullptr, true, s));
-        return direct_f32_onesided(c, o.s64.as<double4>(), nt_pad, o, nt, sh, eps, d_acc, s);
+        return direct_f32_onesided(c, o.s64.as<double4>(), nt_pad, o, nt, sh, eps, d_acc, s, up,
+                                   updated);
     }
     const int64_t np_pad = pad_to(np, kBlock);
     GH_TRY(ensure(c, c->src64, sizeof(double4) * (size_t)np_pad));

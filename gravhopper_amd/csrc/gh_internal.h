@@ -175,16 +175,46 @@ inline unsigned blocks_for(int64_t n, int per_block) {
     return static_cast<unsigned>((n + per_block - 1) / per_block);
 }
 
+// A particle's update by one step: the kick by the accelerations at the half-step positions xh,
+// the drift to x, and the next step's half drift to xh_next (which may be xh).  hist_p /
+// hist_v (nullable): snapshot slot of the step.  v == nullptr: no update.
+struct StepUpdate {
+    const double* xh = nullptr;
+    double *xh_next = nullptr, *v = nullptr, *x = nullptr, *hist_p = nullptr, *hist_v = nullptr;
+    double dt = 0.0;
+};
+// Component k; ext: acceleration in km/s/Myr, added as the reference adds the summed external
+// forces to the N-body acceleration (gravhopper.py:419-459), 0.0 without any.
+__device__ __forceinline__ void update_one(const StepUpdate& u, int64_t k, double acc,
+                                           double ext = 0.0)
+{
+    const double a = acc * kAccelScale + ext;
+    const double vn = u.v[k] + a * u.dt;
+    const double inc = 0.5 * vn * u.dt * kDriftScale;
+    const double xn = u.xh[k] + inc;
+    u.v[k] = vn;
+    u.x[k] = xn;
+    u.xh_next[k] = xn + inc;
+    if (u.hist_p) u.hist_p[k] = xn;
+    if (u.hist_v) u.hist_v[k] = vn;
+}
+
 // direct sum (gh_direct.hip)
+// up (nullable; self field): the particles' update from these accelerations.  Where a kernel
+// that finishes sums can apply it there, it does, sets *updated and leaves d_acc undefined.
 int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
                const double* d_fpos, int64_t nf, double eps, int precision, double* d_acc,
-               hipStream_t s);
+               hipStream_t s, const StepUpdate* up = nullptr, bool* updated = nullptr);
+// FP64 self fields of up to this many particles are updated by the kernel that reads the
+// positions of all, so StepUpdate::xh_next must be another array than xh there.
+constexpr int64_t kF64RelayMax = 6500;
 int64_t pad_to(int64_t n, int64_t m);
 int sym_ipt(gh_ctx* c, int64_t np);
 // true when the FP32 pair kernels need the zero-separation guard for this softening
 bool fp32_guard(double eps);
 int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np, int ipt,
-               double eps, double* d_acc, hipStream_t s);
+               double eps, double* d_acc, hipStream_t s, const StepUpdate* up = nullptr,
+               bool* updated = nullptr);
 // The pair-once kernel over a block-pair list (src: local FP32 coordinates per sorted
 // particle, s64: the same particles in FP64, frame/flag/umass: per block), followed by its
 // double-single instance for the items with a flagged block.
@@ -192,19 +222,19 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
 // jstride particles instead of part.
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,
                const double4* frame, const int* flag, const int* nflag, const float* umass,
-               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items, const float* eps2_blk, float* part, int* queue,
-               unsigned persistent_grid, hipStream_t s, float* jpart = nullptr,
-               int64_t jstride = 0, int64_t joff = 0);
+               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
+               const float* eps2_blk, float* part, int* queue, unsigned persistent_grid,
+               hipStream_t s, float* jpart = nullptr, int64_t jstride = 0, int64_t joff = 0);
 // acc[perm[p]] (perm nullable) = the FP64 sum of particle p's partial slots
 int reduce_sym(gh_ctx* c, const float* part, int nb, const int* nb_blk, int blk,
-               int64_t np_pad, int64_t n, const u32* perm, double* acc, hipStream_t s);
+               int64_t np_pad, int64_t n, const u32* perm, double* acc, hipStream_t s,
+               const StepUpdate* up = nullptr);
 
 // leapfrog update (gh_step.hip).  kick_drift: ext (nullable) is an extra acceleration
 // in km/s/Myr added to the N-body one, as a = acc*A + ext.
 int half_drift(gh_ctx* c, const double* x, const double* v, int64_t n, double dt, double* xh,
                hipStream_t s);
-int kick_drift(gh_ctx* c, const double* acc, int64_t n, double dt, double* xh, double* v,
-               double* x, double* hp, double* hv, hipStream_t s,
+int kick_drift(gh_ctx* c, const double* acc, int64_t n, const StepUpdate& up, hipStream_t s,
                const double* ext = nullptr);
 
 // spatial order and frames (gh_frames.hip)

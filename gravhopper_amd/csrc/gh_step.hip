@@ -7,7 +7,8 @@
 //                                     inc = ((0.5*v')*dt)*D,  x' = xh + inc,
 //                                     xh' = x' + inc  (next step's half drift)
 // so every step is one force evaluation plus one fused elementwise pass, which also
-// writes the snapshot slots of the history when asked to.
+// writes the snapshot slots of the history when asked to.  Where the force's last kernel
+// can, it does the pass itself (StepUpdate): a launch of 4 to 5 us less.
 #include "gh_internal.h"
 
 namespace gh {
@@ -21,30 +22,12 @@ __global__ __launch_bounds__(kBlock) void k_half_drift(const double* __restrict_
     if (k < n3) xh[k] = x[k] + 0.5 * v[k] * dt * kDriftScale;
 }
 
-// hist_p / hist_v (nullable): snapshot slot of this step.
-// ext (nullable): external acceleration in km/s/Myr, added as the reference adds the
-// summed external forces to the N-body acceleration (gravhopper.py:419-459); without
-// external forces the sum is with 0.0, as in the reference.
 __global__ __launch_bounds__(kBlock) void k_kick_drift(const double* __restrict__ acc,
-                                                       int64_t n3, double dt,
-                                                       double* __restrict__ xh,
-                                                       double* __restrict__ v,
-                                                       double* __restrict__ x,
-                                                       double* __restrict__ hist_p,
-                                                       double* __restrict__ hist_v,
+                                                       int64_t n3, StepUpdate up,
                                                        const double* __restrict__ ext)
 {
     const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n3) return;
-    const double a = acc[k] * kAccelScale + (ext ? ext[k] : 0.0);
-    const double vn = v[k] + a * dt;
-    const double inc = 0.5 * vn * dt * kDriftScale;
-    const double xn = xh[k] + inc;
-    v[k] = vn;
-    x[k] = xn;
-    xh[k] = xn + inc;
-    if (hist_p) hist_p[k] = xn;
-    if (hist_v) hist_v[k] = vn;
+    if (k < n3) update_one(up, k, acc[k], ext ? ext[k] : 0.0);
 }
 
 __global__ __launch_bounds__(kBlock) void k_fill_zero(double* __restrict__ p, int64_t n)
@@ -71,12 +54,12 @@ int half_drift(gh_ctx* c, const double* x, const double* v, int64_t n, double dt
     return check_launch(c, "k_half_drift");
 }
 
-int kick_drift(gh_ctx* c, const double* acc, int64_t n, double dt, double* xh, double* v,
-               double* x, double* hp, double* hv, hipStream_t s, const double* ext)
+int kick_drift(gh_ctx* c, const double* acc, int64_t n, const StepUpdate& up, hipStream_t s,
+               const double* ext)
 {
     if (n <= 0) return 0;
     hipLaunchKernelGGL(k_kick_drift, dim3(blocks_for(3 * n, kBlock)), dim3(kBlock), 0, s, acc,
-                       3 * n, dt, xh, v, x, hp, hv, ext);
+                       3 * n, up, ext);
     return check_launch(c, "k_kick_drift");
 }
 

@@ -263,3 +263,21 @@ def test_external_run_history_slices_equal_chained_steps(ctx):
         assert_bitwise(hv[k], vc, "step %d vel" % k)
     assert_bitwise(x, xc, "final pos")
     assert_bitwise(v, vc, "final vel")
+
+
+# FP64: either side of the last size whose force kernel applies the update; FP32: source
+# splits, pair once, and no split (unfused)
+@pytest.mark.parametrize("prec,n", [(_native.GH_FP64, n) for n in (2, 65, 6500, 6501)] +
+                         [(_native.GH_FP32, n) for n in (2, 257, 3000, 16384, 16385)])
+def test_run_update_in_the_force_kernel(ctx, prec, n):
+    # a timed run keeps the update in a kernel of its own: the same bits
+    ic = workloads.plummer(n, seed=n)
+    got = ctx.run(ic["pos"], ic["vel"], ic["mass"], 1e-3, 1e-4, 5, precision=prec, history=True)
+    ctx.timing_enable(True)
+    try:
+        want = ctx.run(ic["pos"], ic["vel"], ic["mass"], 1e-3, 1e-4, 5, precision=prec,
+                       history=True)
+    finally:
+        ctx.timing_enable(False)
+    for k, (g, w) in enumerate(zip(got, want)):
+        assert_bitwise(g, w, "array %d" % k)
