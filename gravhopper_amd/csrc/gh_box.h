@@ -1,6 +1,6 @@
-// Root box of a point set from per-workgroup extents, shared by the box kernel of the
-// tree build (gh_tree.hip) and the key kernel of the small spatial sort (gh_frames.hip),
-// so that both form the same box bit for bit.
+// Root box of a point set from its extents, shared by the box and key kernels of the tree
+// build (gh_tree.hip) and of the spatial order (gh_frames.hip), so that all form the same
+// box bit for bit.
 #pragma once
 
 #include "gh_internal.h"
@@ -24,9 +24,21 @@ __device__ __forceinline__ void block_extent(double (*smin)[kBlock], double (*sm
     }
 }
 
-// The reference's root box (gravhopper/_jbgrav.c:764-772) of the nparts extents
-// part[6 b ..] = (min x, y, z, max x, y, z), returned to every thread of the workgroup:
-// box[0..2] = centre, box[3] = size.  Minima and maxima are exact in any order.
+// The reference's root box (gravhopper/_jbgrav.c:764-772) of the extents mn, mx: box[0..2] =
+// centre, box[3] = size.
+__device__ __forceinline__ void box_of_extents(const double mn[3], const double mx[3],
+                                               double eps, double box[4])
+{
+    double bs = mx[0] - mn[0] + eps;
+    for (int k = 1; k < 3; k++)
+        if ((mx[k] - mn[k]) > bs) bs = mx[k] - mn[k] + eps;
+    for (int k = 0; k < 3; k++) box[k] = 0.5 * (mn[k] + mx[k]);
+    box[3] = bs;
+}
+
+// The root box of the nparts extents
+// part[6 b ..] = (min x, y, z, max x, y, z), returned to every thread of the workgroup.
+// Minima and maxima are exact in any order.
 __device__ __forceinline__ void box_from_parts(const double* __restrict__ part, int nparts,
                                                double eps, double (*smin)[kBlock],
                                                double (*smax)[kBlock], double box[4])
@@ -50,11 +62,7 @@ __device__ __forceinline__ void box_from_parts(const double* __restrict__ part, 
         mn[k] = smin[k][0];
         mx[k] = smax[k][0];
     }
-    double bs = mx[0] - mn[0] + eps;
-    for (int k = 1; k < 3; k++)
-        if ((mx[k] - mn[k]) > bs) bs = mx[k] - mn[k] + eps;
-    for (int k = 0; k < 3; k++) box[k] = 0.5 * (mn[k] + mx[k]);
-    box[3] = bs;
+    box_of_extents(mn, mx, eps, box);
     __syncthreads();  // smin/smax may be reused
 }
 

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "gh_box.h"
+#include "gh_runsort.h"
 #include "gh_internal.h"
 
 namespace gh {
@@ -78,20 +79,8 @@ __global__ __launch_bounds__(kBlock) void k_morton(const double* __restrict__ po
     idx[i] = (u32)i;
 }
 
-// Small sorts: runs of up to 1024 points are sorted where their keys are formed, and a point's
-// place in the order is its place in its run plus what a binary search finds in every other
-// run.  A radix sort of so few points is bound by the latency of its passes; this is two
-// launches with a chain of some 60 dependent LDS reads.  The sort of one call, radix passes of
-// one launch each before: 43 us at N = 3000, now 19; 50 us at 16384, now 18.
-//
-// Every run forms the box of all its segment's points, and every 64 points search all its
-// runs, so the work grows as n^2 (rank_form draws the line).
-//
-// Segments: with seg_start / seg_count, segment g of a padded layout is sorted on its own
-// (run b belongs to segment seg[b]), its padding left in place behind its points.
-constexpr int kRankThreads = 1024;
-constexpr int kRankWaves = kRankThreads / 64;
-
+// Small sorts, in runs of up to 1024 points (gh_runsort.h).  The sort of one call, radix passes
+// of one launch each before: 43 us at N = 3000, now 19; 50 us at 16384, now 18.
 // Bits kKeyShift .. 62 of the Morton key: from bit 0 on y and z of level 10, then x, y, z of
 // levels 11 .. 20 (bit 3 k + a of the key is bit k of axis a).
 static_assert(kKeyShift == 31, "the axes' shares of the 32 key bits");
@@ -103,107 +92,34 @@ __device__ __forceinline__ u32 spread3_11(u32 v)
     return (v | (v << 2)) & 0x49249249u;
 }
 
-// x of another lane, by DPP control CTRL in the rows of ROWS; other rows keep their own.
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ double dpp_f64(double x)
-{
-    const int lo = __double2loint(x), hi = __double2hiint(x);
-    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false),
-                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false));
-}
-
 // Root box (as k_bbox_final with eps = 0) of the n points from pos on, in every thread of the
 // workgroup; minima and maxima are exact in any order.
 __device__ __forceinline__ void points_box(const double* __restrict__ pos, int n, double box[4])
 {
-    __shared__ double ext[6][kRankWaves];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double mn[3], mx[3];
     for (int a = 0; a < 3; a++) mn[a] = mx[a] = pos[a];  // the first point seeds
 #pragma unroll 4
-    for (int i = threadIdx.x; i < n; i += kRankThreads)
+    for (int i = threadIdx.x; i < n; i += kRunThreads)
         for (int a = 0; a < 3; a++) {
             const double q = pos[3 * i + a];
             if (q < mn[a]) mn[a] = q;
             if (q > mx[a]) mx[a] = q;
         }
-    auto fold = [&](auto moved) {
-        for (int a = 0; a < 3; a++) {
-            const double lo = moved(mn[a]), hi = moved(mx[a]);
-            if (lo < mn[a]) mn[a] = lo;
-            if (hi > mx[a]) mx[a] = hi;
-        }
-    };
-    auto over_row = [&] {  // every lane of a row of 16 ends with the row's extremes
-        fold([](double x) { return dpp_f64<0x128>(x); });
-        fold([](double x) { return dpp_f64<0x124>(x); });
-        fold([](double x) { return dpp_f64<0x122>(x); });
-        fold([](double x) { return dpp_f64<0x121>(x); });
-    };
-    over_row();
-    fold([](double x) { return dpp_f64<0x142, 0xa>(x); });  // rows 0 and 2 into 1 and 3
-    fold([](double x) { return dpp_f64<0x143, 0xc>(x); });  // row 1 into 2 and 3
-    if (lane == 63)
-        for (int a = 0; a < 3; a++) {
-            ext[a][wave] = mn[a];
-            ext[3 + a][wave] = mx[a];
-        }
-    __syncthreads();
-    static_assert(kRankWaves == 16, "one value per lane of a row");
-    for (int a = 0; a < 3; a++) {
-        mn[a] = ext[a][lane % kRankWaves];
-        mx[a] = ext[3 + a][lane % kRankWaves];
-    }
-    over_row();
-    box[3] = mx[0] - mn[0];
-    for (int a = 0; a < 3; a++) {
-        if (mx[a] - mn[a] > box[3]) box[3] = mx[a] - mn[a];
-        box[a] = 0.5 * (mn[a] + mx[a]);
-    }
+    run_extents(mn, mx);
+    box_of_extents(mn, mx, 0.0, box);
 }
 
-// How many of the N sorted keys from k on come before key: those smaller, and with `ties` those
-// equal.
-template <int N>
-__device__ __forceinline__ int count_before(const u32* k, u32 key, bool ties)
-{
-    int at = 0;
-#pragma unroll
-    for (int h = N / 2; h > 0; h /= 2) {
-        const u32 q = k[at + h - 1];
-        at += q < key || (ties && q == key) ? h : 0;
-    }
-    const u32 q = k[at];
-    return at + (q < key || (ties && q == key) ? 1 : 0);
-}
-
-// A point's place in the merger of its run of N keys, its place there `at`, with the other
-// three of its group of four (run r of the group; ties: earlier runs first).
-template <int N>
-__device__ __forceinline__ int place_in_four(const u32* group, int r, int at, u32 key)
-{
-    int place = at;
-#pragma unroll
-    for (int o = 1; o < 4; o++) {
-        const int other = r ^ o;
-        place += count_before<N>(group + other * N, key, other < r);
-    }
-    return place;
-}
-
-// Run b of RUN points (RUN of the kRankThreads threads hold one each; all of them form the
-// box of the run's segment): the keys in order, with the points they belong to, ties by index.
-// A wavefront sorts 64 by counting, then four sorted lists become one, twice.  Places behind
-// the segment's points are filled with the largest key.
+// Run b of RUN points (RUN of the kRunThreads threads hold one each; all of them form the box
+// of the run's segment): the keys in order, with the points they belong to.  Places behind the
+// segment's points are filled with the largest key.
 template <int RUN>
-__global__ __launch_bounds__(kRankThreads) void k_rank_runs(
+__global__ __launch_bounds__(kRunThreads) void k_rank_runs(
     const double* __restrict__ pos, int64_t n_all, const int* __restrict__ seg,
     const int64_t* __restrict__ seg_start, const int64_t* __restrict__ seg_count,
     u32* __restrict__ keys, u32* __restrict__ from, u32* __restrict__ perm,
     int* __restrict__ nflag)
 {
-    __shared__ u32 sk[2][RUN], si[2][RUN];
-    const int t = threadIdx.x, lane = t & 63;
+    const int t = threadIdx.x;
     const int g = seg ? seg[blockIdx.x] : 0;
     const int64_t first = seg ? seg_start[g] : 0;
     const int n = (int)(seg ? seg_count[g] : n_all);
@@ -213,104 +129,21 @@ __global__ __launch_bounds__(kRankThreads) void k_rank_runs(
     points_box(p, n, box);
     const bool act = t < RUN;  // whole wavefronts
     const int64_t base = (int64_t)blockIdx.x * RUN;
+    const int i = (int)(base - first) + t;
     u32 key = 0xffffffffu, idx = (u32)(base + t);
-    int at = 0;
-    if (act) {
-        const int i = (int)(base - first) + t;
-        if (i < n) {
-            const double size = box[3], scale = size > 0.0 ? 2097152.0 / size : 0.0;
-            u32 q[3];
-            for (int a = 0; a < 3; a++)
-                q[a] = quantize(p[3 * i + a], box[a] - 0.5 * size, scale);
-            key = spread3_11(q[1] >> 10) | spread3_11(q[2] >> 10) << 1 |
-                  spread3_11(q[0] >> 11) << 2;
-        } else if (seg) {
-            perm[base + t] = idx;
-        }
-#pragma unroll
-        for (int q = 0; q < 64; q++) {
-            const u32 k = (u32)__builtin_amdgcn_readlane((int)key, q);
-            at += k < key || (k == key && q < lane) ? 1 : 0;
-        }
+    if (act && i < n) {
+        const double size = box[3], scale = size > 0.0 ? 2097152.0 / size : 0.0;
+        u32 q[3];
+        for (int a = 0; a < 3; a++) q[a] = quantize(p[3 * i + a], box[a] - 0.5 * size, scale);
+        key = spread3_11(q[1] >> 10) | spread3_11(q[2] >> 10) << 1 | spread3_11(q[0] >> 11) << 2;
+    } else if (act && seg) {
+        perm[base + t] = idx;
     }
-    if (act) {
-        sk[0][t - lane + at] = key;
-        si[0][t - lane + at] = idx;
-    }
-    __syncthreads();
-    if (act) {
-        key = sk[0][t];
-        idx = si[0][t];
-        at = place_in_four<64>(&sk[0][t & ~255], (t >> 6) & 3, lane, key);
-    }
-    if constexpr (RUN > 256) {
-        if (act) {
-            sk[1][(t & ~255) + at] = key;
-            si[1][(t & ~255) + at] = idx;
-        }
-        __syncthreads();
-        if (act) {
-            key = sk[1][t];
-            idx = si[1][t];
-            if constexpr (RUN == 512)
-                at = (t & 255) + count_before<256>(&sk[1][t < 256 ? 256 : 0], key, t >= 256);
-            else
-                at = place_in_four<256>(sk[1], t >> 8, t & 255, key);
-        }
-    }
-    static_assert(RUN == 256 || RUN == 512 || RUN == 1024, "lists merged");
+    const int at = sort_run<RUN>(key, idx, act);
     if (act) {
         keys[base + at] = key;
         from[base + at] = idx;
     }
-}
-
-// perm from the sorted runs of RUN keys: 64 places of one run per workgroup, a lane each.  A
-// wavefront takes 1024 keys of the segment at a time into its part of LDS and searches each
-// run of them.
-template <int RUN>
-__global__ __launch_bounds__(kRankThreads) void k_rank_merge(
-    const u32* __restrict__ keys, const u32* __restrict__ from, int64_t n_all,
-    const int* __restrict__ seg, const int64_t* __restrict__ seg_start,
-    const int64_t* __restrict__ seg_count, u32* __restrict__ perm)
-{
-    constexpr int kRuns = 1024 / RUN;
-    __shared__ u32 part[kRankWaves][1024];
-    __shared__ int below[kRankWaves][64];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t place = (int64_t)blockIdx.x * 64 + lane;
-    const int g = seg ? seg[(int64_t)blockIdx.x * 64 / RUN] : 0;
-    const int64_t first = seg ? seg_start[g] : 0;
-    const int n = (int)(seg ? seg_count[g] : n_all);
-    const int end = (n + RUN - 1) / RUN * RUN;              // keys of the segment's runs
-    const int own = (int)((place - lane - first) / RUN);    // this run in its segment
-    const u32 key = keys[place];
-    int count = 0;
-    for (int k0 = wave * 1024; k0 < end; k0 += kRankWaves * 1024) {
-        uint4* mine = (uint4*)part[wave];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int k = k0 + 4 * (64 * q + lane);
-            mine[64 * q + lane] = k < end ? *(const uint4*)(keys + first + k)
-                                          : make_uint4(~0u, ~0u, ~0u, ~0u);
-        }
-        __builtin_amdgcn_wave_barrier();  // LDS serves a wavefront in order
-#pragma unroll 4
-        for (int r = 0; r < kRuns; r++) {
-            const int run = k0 / RUN + r;
-            const int c = count_before<RUN>(&part[wave][r * RUN], key, run < own);
-            count += run == own ? 0 : c;
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    below[wave][lane] = count;
-    __syncthreads();
-    if (wave != 0) return;
-    const u32 idx = from[place];
-    for (int w = 1; w < kRankWaves; w++) count += below[w][lane];
-    const int at = (int)(place - first) - own * RUN;
-    if ((int64_t)idx - first < n) perm[first + at + count] = idx;
 }
 
 // The order of n points, or of segments of at most `most` points each (runs of `run` places,
@@ -319,15 +152,15 @@ static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, i
                       int run, const int* seg, const int64_t* start, const int64_t* count,
                       hipStream_t s)
 {
-    const dim3 runs((unsigned)(n_pad / run)), blocks((unsigned)(n_pad / 64)), threads(kRankThreads);
+    const dim3 runs((unsigned)(n_pad / run)), blocks((unsigned)(n_pad / 64)), threads(kRunThreads);
     u32 *keys = o.keys[0].as<u32>(), *from = o.keys[1].as<u32>(), *perm = o.idx[0].as<u32>();
 #define GH_RANK(RUN)                                                                          \
     case RUN:                                                                                 \
         hipLaunchKernelGGL(k_rank_runs<RUN>, runs, threads, 0, s, d_pos, n, seg, start, count, \
                            keys, from, perm, o.nflag.as<int>());                              \
         GH_TRY(check_launch(c, "k_rank_runs"));                                               \
-        hipLaunchKernelGGL(k_rank_merge<RUN>, blocks, threads, 0, s, keys, from, n, seg,      \
-                           start, count, perm);                                               \
+        hipLaunchKernelGGL((k_run_merge<RUN, kRunThreads / 64, 1, u32>), blocks, threads, 0,  \
+                           s, keys, from, n, seg, start, count, (u32*)nullptr, perm);         \
         break;
     switch (run) {
         GH_RANK(256)
@@ -337,10 +170,11 @@ static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, i
     }
 #undef GH_RANK
     o.sel = 0;
-    return check_launch(c, "k_rank_merge");
+    return check_launch(c, "k_run_merge");
 }
 
-// Where rank_order is the faster form, of n places in segments of at most `most` points: a
+// Every run forms the box of all its segment's points, and every 64 points search all its runs,
+// so the work grows as n^2.  Where this is the faster form, of n places in segments of at most `most` points: a
 // force of 65536 particles took 1058 us with it and 1080 with the radix passes, of 98304 2083
 // and 2089, of 131072 3158 and 3135; a step of 4 simulations of 32768 1.11 ms and 1.22, of 32
 // of 16384 2.19 and 2.20, of 128 of 16384 7.84 and 7.75.
@@ -355,14 +189,14 @@ int spatial_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, hipSt
     if (n <= 0) return 0;
     for (int k = 0; k < 2; k++) {
         // (512: rank_order pads its 32-bit keys to whole runs)
-        GH_TRY(ensure(c, o.keys[k], sizeof(u64) * (size_t)std::max(n, (int64_t)kRankThreads / 2)));
+        GH_TRY(ensure(c, o.keys[k], sizeof(u64) * (size_t)std::max(n, (int64_t)kRunThreads / 2)));
         GH_TRY(ensure(c, o.idx[k], sizeof(u32) * (size_t)n));
     }
     GH_TRY(ensure(c, o.box, sizeof(double) * 8));
     GH_TRY(ensure(c, o.nflag, 256));
     if (rank_form(c, n, n)) {
-        const int64_t n_pad = (int64_t)blocks_for(n, kRankThreads) * kRankThreads;
-        GH_TRY(rank_order(c, o, d_pos, n, n_pad, kRankThreads, nullptr, nullptr, nullptr, s));
+        const int64_t n_pad = (int64_t)blocks_for(n, kRunThreads) * kRunThreads;
+        GH_TRY(rank_order(c, o, d_pos, n, n_pad, kRunThreads, nullptr, nullptr, nullptr, s));
         o.sorted = d_pos;
         o.sorted_n = n;
         return 0;

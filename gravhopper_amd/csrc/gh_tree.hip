@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "gh_box.h"
+#include "gh_runsort.h"
 #include "gh_internal.h"
 #include "gh_search.h"
 
@@ -152,6 +153,20 @@ __device__ __forceinline__ int descend(double x, double y, double z, double& cx,
     return (int)gx | ((int)gy << 1) | ((int)gz << 2);
 }
 
+// One key word: the octants of x on kLevelsPerWord levels from the node (c, size) down, which
+// become the node below them.
+__device__ __forceinline__ u64 key_word(const double (&x)[3], double (&c)[3], double& size)
+{
+    u64 k = 0;
+    for (int l = 0; l < kLevelsPerWord; l++) {
+        const double h = 0.5 * size;
+        const int d = descend(x[0], x[1], x[2], c[0], c[1], c[2], h);
+        k = (k << 3) | (u64)d;
+        size = h;
+    }
+    return k;
+}
+
 // One workgroup per radix-sort chunk (kRsChunk particles, kKeysItems per thread).
 // packed (nullable) receives (x, y, z, m) of each particle in input order, so that the
 // gather into sorted order after the sort fetches one 32-byte record per particle
@@ -177,18 +192,12 @@ __global__ __launch_bounds__(kKeysBlock) void k_keys(
     for (int it = 0; it < kKeysItems; it++) {
         const int64_t i = (int64_t)blockIdx.x * kRsChunk + (int64_t)it * kKeysBlock + threadIdx.x;
         if (i >= n) break;
-        const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-        if (packed) packed[i] = make_double4(x, y, z, mass[i]);
-        double cx = bx, cy = by, cz = bz;
+        const double x[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+        if (packed) packed[i] = make_double4(x[0], x[1], x[2], mass[i]);
+        double c[3] = {bx, by, bz};
         double size = bs;
         for (int w = 0; w < words; w++) {
-            u64 k = 0;
-            for (int l = 0; l < kLevelsPerWord; l++) {
-                const double hh = 0.5 * size;
-                const int d = descend(x, y, z, cx, cy, cz, hh);
-                k = (k << 3) | (u64)d;
-                size = hh;
-            }
+            const u64 k = key_word(x, c, size);
             keys[(int64_t)w * n + i] = k;
             if (hist && w == hword) atomicAdd(&h[(u32)(k >> hshift) & 255u], 1u);
         }
@@ -198,6 +207,50 @@ __global__ __launch_bounds__(kKeysBlock) void k_keys(
         __syncthreads();
         if (threadIdx.x < 256) hist[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
     }
+}
+
+// The keys of a small tree or target set (one word, without its low `drop` bits), sorted in
+// runs of kRunThreads, and the particles as `packed` (nullable).  part (nullable): the extents
+// to form the root box from, which goes to box; otherwise box holds it.  Places behind the
+// particles get the largest key.
+__global__ __launch_bounds__(kRunThreads) void k_keys_runs(
+    const double* __restrict__ pos, int64_t n, const double* __restrict__ part, int nparts,
+    double eps, double* __restrict__ box, int drop, u64* __restrict__ keys,
+    u32* __restrict__ from, int* __restrict__ flags, const double* __restrict__ mass,
+    double4* __restrict__ packed)
+{
+    double b[4];
+    if (part) {
+        double mn[3], mx[3];
+        for (int a = 0; a < 3; a++) {
+            mn[a] = part[a];
+            mx[a] = part[3 + a];
+        }
+        for (int p = threadIdx.x; p < nparts; p += kRunThreads)
+            for (int a = 0; a < 3; a++) {
+                if (part[6 * p + a] < mn[a]) mn[a] = part[6 * p + a];
+                if (part[6 * p + 3 + a] > mx[a]) mx[a] = part[6 * p + 3 + a];
+            }
+        run_extents(mn, mx);
+        box_of_extents(mn, mx, eps, b);
+        if (blockIdx.x == 0 && threadIdx.x < 4) box[threadIdx.x] = b[threadIdx.x];
+    } else {
+        for (int a = 0; a < 4; a++) b[a] = box[a];
+    }
+    if (flags && blockIdx.x == 0 && threadIdx.x < 4) flags[threadIdx.x] = 0;
+    const int64_t base = (int64_t)blockIdx.x * kRunThreads, i = base + threadIdx.x;
+    u64 key = ~0ull;
+    u32 idx = (u32)i;
+    if (i < n) {
+        const double x[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+        if (packed) packed[i] = make_double4(x[0], x[1], x[2], mass[i]);
+        double c[3] = {b[0], b[1], b[2]};
+        double size = b[3];
+        key = key_word(x, c, size) >> drop;
+    }
+    const int at = sort_run<kRunThreads>(key, idx, true);
+    keys[base + at] = key;
+    from[base + at] = idx;
 }
 
 // ------------------------------------------------------------------------------
@@ -2069,17 +2122,54 @@ int radix_sort(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n, in
 
 // Root box of the reference (centre box[0..2], size box[3], gravhopper/_jbgrav.c:747-772)
 // of n points, written to the device array box; part holds the partial extents.
+static int bbox_parts_dev(gh_ctx* c, const double* d_pos, int64_t n, DevBuf& part, hipStream_t s,
+                          int* nparts)
+{
+    *nparts = (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
+    GH_TRY(ensure(c, part, sizeof(double) * 6 * (size_t)*nparts));
+    hipLaunchKernelGGL(k_bbox_partial, dim3(*nparts), dim3(kBlock), 0, s, d_pos, n,
+                       part.as<double>());
+    return check_launch(c, "k_bbox_partial");
+}
+
 int bbox_dev(gh_ctx* c, const double* d_pos, int64_t n, double eps, DevBuf& part, double* box,
              hipStream_t s)
 {
-    const int nparts = (int)std::min<int64_t>(1024, (n + kBlock - 1) / kBlock);
-    GH_TRY(ensure(c, part, sizeof(double) * 6 * (size_t)nparts));
-    hipLaunchKernelGGL(k_bbox_partial, dim3(nparts), dim3(kBlock), 0, s, d_pos, n,
-                       part.as<double>());
-    GH_TRY(check_launch(c, "k_bbox_partial"));
+    int nparts = 0;
+    GH_TRY(bbox_parts_dev(c, d_pos, n, part, s, &nparts));
     hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, s, part.as<double>(), nparts,
                        eps, box);
     return check_launch(c, "k_bbox_final");
+}
+
+// Sorts of up to this many one-word keys take k_keys_runs and k_run_merge, two launches of 27 us
+// together at 40001 particles; the box's second launch, the keys and the radix passes took 98.
+// The merge's work grows as n^2.  FP64 forces, us with the runs (and with radix passes): 62 (114)
+// for 2 particles, 101 (154) for 2000, 223 (274) for 40001, 308 (351) for 65536, 431 (440) for
+// 100000, 511 (501) for 131072, 837 (715) for 200000; 300007 particles on 20011 targets 331
+// (387), on 65536 474 (515), on 131072 638 (625).
+constexpr int64_t kRunSortMax = 100000;
+
+// Keys of n <= kRunSortMax points in order in keys[1] with the points in idx[1], by the bits
+// from `drop` on.  part / box / flags / mass / packed: k_keys_runs.
+static int run_sort(gh_ctx* c, const double* d_pos, int64_t n, const double* part, int nparts,
+                    double eps, double* box, int drop, DevBuf* keys, DevBuf* idx, int* flags,
+                    const double* mass, double4* packed, hipStream_t s)
+{
+    constexpr int kWaves = 8, kPerLane = 2;
+    const int64_t n_pad = (n + kRunThreads - 1) / kRunThreads * kRunThreads;
+    GH_TRY(ensure(c, keys[0], sizeof(u64) * (size_t)n_pad));
+    GH_TRY(ensure(c, idx[0], sizeof(u32) * (size_t)n_pad));
+    hipLaunchKernelGGL(k_keys_runs, dim3((unsigned)(n_pad / kRunThreads)), dim3(kRunThreads), 0,
+                       s, d_pos, n, part, nparts, eps, box, drop, keys[0].as<u64>(),
+                       idx[0].as<u32>(), flags, mass, packed);
+    GH_TRY(check_launch(c, "k_keys_runs"));
+    hipLaunchKernelGGL((k_run_merge<kRunThreads, kWaves, kPerLane, u64>),
+                       dim3((unsigned)(n_pad / (64 * kPerLane))), dim3(64 * kWaves), 0, s,
+                       keys[0].as<u64>(), idx[0].as<u32>(), n, (const int*)nullptr,
+                       (const int64_t*)nullptr, (const int64_t*)nullptr, keys[1].as<u64>(),
+                       idx[1].as<u32>());
+    return check_launch(c, "k_run_merge");
 }
 
 // Builds the tree of (d_pos, d_mass) into c->tree.  One host synchronisation reads the
@@ -2093,7 +2183,12 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
 
     // 1. box
     GH_TRY(ensure(c, tb->box, sizeof(double) * 8));
-    GH_TRY(bbox_dev(c, d_pos, n, eps, tb->bbox_part, tb->box.as<double>(), s));
+    const bool few = n <= kRunSortMax && c->tune[GH_TUNE_TREE_SORT] == 0;
+    int nparts = 0;
+    if (few)
+        GH_TRY(bbox_parts_dev(c, d_pos, n, tb->bbox_part, s, &nparts));
+    else
+        GH_TRY(bbox_dev(c, d_pos, n, eps, tb->bbox_part, tb->box.as<double>(), s));
 
     GH_TRY(ensure(c, tb->idx[0], sizeof(u32) * (size_t)n));
     GH_TRY(ensure(c, tb->idx[1], sizeof(u32) * (size_t)n));
@@ -2142,19 +2237,26 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
         const bool by_runs = words == 1 && !all_bits;
         const int lo_bits = by_runs ? kSortLowBits : 0;
         GH_TRY(ensure(c, tb->hist, sizeof(u32) * 256 * (size_t)(blocks_for(n, kRsChunk) + 1)));
-        hipLaunchKernelGGL(k_keys, dim3(blocks_for(n, kRsChunk)), dim3(kKeysBlock), 0, s, d_pos,
-                           n, tb->box.as<double>(), words, tb->keys[0].as<u64>(),
-                           tb->idx[0].as<u32>(), tb->flags.as<int>(), d_mass,
-                           tb->packed.as<double4>(), tb->hist.as<u32>(), words - 1, lo_bits);
-        GH_TRY(check_launch(c, "k_keys"));
-        // 3. sort
-        GH_TRY(radix_sort(c, tb->keys, tb->idx, tb->hist, n, words, lo_bits, s, &tb->key_sel,
-                          64, true));
-        if (by_runs) {
-            hipLaunchKernelGGL(k_sort_runs, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
-                               tb->keys[tb->key_sel].as<u64>(), tb->idx[tb->key_sel].as<u32>(),
-                               n, tb->flags.as<int>() + 2);
-            GH_TRY(check_launch(c, "k_sort_runs"));
+        if (few && words == 1) {
+            GH_TRY(run_sort(c, d_pos, n, tb->bbox_part.as<double>(), nparts, eps,
+                            tb->box.as<double>(), 0, tb->keys, tb->idx, tb->flags.as<int>(),
+                            d_mass, tb->packed.as<double4>(), s));
+            tb->key_sel = 1;
+        } else {
+            hipLaunchKernelGGL(k_keys, dim3(blocks_for(n, kRsChunk)), dim3(kKeysBlock), 0, s, d_pos,
+                               n, tb->box.as<double>(), words, tb->keys[0].as<u64>(),
+                               tb->idx[0].as<u32>(), tb->flags.as<int>(), d_mass,
+                               tb->packed.as<double4>(), tb->hist.as<u32>(), words - 1, lo_bits);
+            GH_TRY(check_launch(c, "k_keys"));
+            // 3. sort
+            GH_TRY(radix_sort(c, tb->keys, tb->idx, tb->hist, n, words, lo_bits, s, &tb->key_sel,
+                              64, true));
+            if (by_runs) {
+                hipLaunchKernelGGL(k_sort_runs, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
+                                   tb->keys[tb->key_sel].as<u64>(), tb->idx[tb->key_sel].as<u32>(),
+                                   n, tb->flags.as<int>() + 2);
+                GH_TRY(check_launch(c, "k_sort_runs"));
+            }
         }
         // 4./5. shared levels, end-search levels, node counts, sorted particles
         DeltaArgs da;
@@ -2316,14 +2418,20 @@ static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps,
             GH_TRY(ensure(c, tb->tkeys[k], sizeof(u64) * (size_t)nt));
             GH_TRY(ensure(c, tb->tidx[k], sizeof(u32) * (size_t)nt));
         }
-        hipLaunchKernelGGL(k_keys, dim3(blocks_for(nt, kRsChunk)), dim3(kKeysBlock), 0, s, tgt,
-                           nt, tb->box.as<double>(), 1, tb->tkeys[0].as<u64>(),
-                           tb->tidx[0].as<u32>(), (int*)nullptr, (const double*)nullptr,
-                           (double4*)nullptr, (u32*)nullptr, 0, 0);
-        GH_TRY(check_launch(c, "k_keys"));
-        int sel = 0;
-        GH_TRY(radix_sort(c, tb->tkeys, tb->tidx, tb->hist, nt, 1, 24, s, &sel));
-        order = tb->tidx[sel].as<u32>();
+        if (nt <= kRunSortMax && c->tune[GH_TUNE_TREE_SORT] == 0) {
+            GH_TRY(run_sort(c, tgt, nt, nullptr, 0, 0.0, tb->box.as<double>(), 24, tb->tkeys,
+                            tb->tidx, nullptr, nullptr, nullptr, s));
+            order = tb->tidx[1].as<u32>();
+        } else {
+            hipLaunchKernelGGL(k_keys, dim3(blocks_for(nt, kRsChunk)), dim3(kKeysBlock), 0, s, tgt,
+                               nt, tb->box.as<double>(), 1, tb->tkeys[0].as<u64>(),
+                               tb->tidx[0].as<u32>(), (int*)nullptr, (const double*)nullptr,
+                               (double4*)nullptr, (u32*)nullptr, 0, 0);
+            GH_TRY(check_launch(c, "k_keys"));
+            int sel = 0;
+            GH_TRY(radix_sort(c, tb->tkeys, tb->tidx, tb->hist, nt, 1, 24, s, &sel));
+            order = tb->tidx[sel].as<u32>();
+        }
     }
     if (precision == GH_FP64) {
         // Targets per walk.  More of them share a walk's nodes, but its list also holds what

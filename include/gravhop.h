@@ -242,11 +242,12 @@ int gh_timing_read(gh_ctx *ctx, int kernel_class, double *total_ms, int64_t *lau
  *   GH_TUNE_SORT_DIRECT  spatial order of the FP32 direct sum: 0 automatic (two launches
  *                        while points times points of the largest simulation stay within
  *                        2^33, else radix passes), -1 always radix passes
- *   GH_TUNE_TREE_SORT    octree key sort: 0 automatic (radix passes over the digits of
- *                        levels 0-12, then each run of keys equal there sorted on its
- *                        own; a run of more than 64 keys makes the build sort over all
- *                        digits, and so do the context's next 64 builds), 1 the same
- *                        without the 64 builds, -1 always over all digits
+ *   GH_TUNE_TREE_SORT    octree key sort: 0 automatic (two launches up to 100000 keys;
+ *                        beyond, radix passes over the digits of levels 0-12, then each
+ *                        run of keys equal there sorted on its own; a run of more than 64
+ *                        keys makes the build sort over all digits, and so do the
+ *                        context's next 64 builds), 1 the radix passes at every size,
+ *                        without the 64 builds, -1 those, always over all digits
  *   GH_TUNE_WALK_PREFIX  FP32 tree walk: 0 each block of 64 groups first decides once the
  *                        nodes decided alike for all of its groups (k_walk_prefix), and
  *                        the groups start from there; -1 every group from the root

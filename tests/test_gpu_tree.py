@@ -95,6 +95,30 @@ def tree_cases():
     return cases
 
 
+# edges of a wavefront's list, of the runs and of the range of the two-launch sort
+@pytest.mark.parametrize("n", [2, 64, 65, 1023, 1024, 1025, 17000, 100000, 100001])
+def test_key_sort_forms_agree(ctx, n):
+    # clusters of equal high digits, and (not for the smallest) two particles that only a
+    # second key word separates
+    sizes = [66, 2] if n > 100 else []
+    pos, mass = clustered(n - sum(sizes), sizes, seed=n)
+    if n > 64:
+        pos[5] = pos[4] * (1.0 + 1e-14)
+    fpos = np.random.default_rng(n).normal(size=(max(n, 4096), 3)) * 2.0
+    fpos[7:90] = fpos[7]  # equal keys
+    out = {}
+    for mode in (0, 1, 0, -1):
+        ctx.set_tuning(_native.TUNE_TREE_SORT, mode)
+        try:
+            out[mode] = (ctx.tree(pos, mass, 1e-3, 0.7, FP64),
+                         ctx.tree(pos, mass, 1e-3, 0.7, FP32, force_pos=fpos))
+        finally:
+            ctx.set_tuning(_native.TUNE_TREE_SORT, 0)
+    for mode in (1, -1):
+        for g, w in zip(out[0], out[mode]):
+            assert_bitwise(g, w, "mode %d" % mode)
+
+
 @pytest.mark.parametrize("case", tree_cases(), ids=lambda c: c[0])
 def test_topology_bitwise(ctx, oracle, case):
     name, pos, mass, eps = case
