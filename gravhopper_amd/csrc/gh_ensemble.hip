@@ -18,6 +18,8 @@
 // and replayed.
 #include <algorithm>
 #include <cstring>
+#include <system_error>
+#include <thread>
 
 #include "gh_internal.h"
 
@@ -32,6 +34,7 @@ struct gh_ensemble {
     std::vector<int64_t> start, count;
     gh::DevBuf x, v, xh, m, acc, part, work, eps_blk, nb_blk, valid_blk, dt_blk, queue;
     gh::DevBuf seg_blk, seg_start, seg_count;  // simulation of each block, ranges
+    gh::DevBuf seg_first;  // each simulation's first particle without the padding
     gh::OrderBufs ord;                           // per-step order and frames
     bool guard = false;
     hipGraph_t graph = nullptr;
@@ -50,6 +53,23 @@ __global__ __launch_bounds__(kBlock) void k_ens_half_drift(
     if ((int)(p - b * blk) >= valid_blk[b]) return;  // padding: never updated
     const double dt = dt_blk[b];
     for (int k = 0; k < 3; k++) xh[3 * p + k] = x[3 * p + k] + 0.5 * v[3 * p + k] * dt * kDriftScale;
+}
+
+// Positions and velocities (to_x / to_v, nullable) without the padding.
+__global__ __launch_bounds__(kBlock) void k_ens_pack(
+    const double* __restrict__ x, const double* __restrict__ v, int64_t n_pad, int blk,
+    const int* __restrict__ seg, const int64_t* __restrict__ seg_start,
+    const int64_t* __restrict__ seg_count, const int64_t* __restrict__ seg_first,
+    double* __restrict__ to_x, double* __restrict__ to_v)
+{
+    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t p = k / 3;
+    if (p >= n_pad) return;
+    const int g = seg[p / blk];
+    if (p - seg_start[g] >= seg_count[g]) return;
+    const int64_t to = k + 3 * (seg_first[g] - seg_start[g]);
+    if (to_x) to_x[to] = x[k];
+    if (to_v) to_v[to] = v[k];
 }
 
 // v' = v + (a A + 0) dt; x' = xh + ((0.5 v') dt) D; xh' = x' + ((0.5 v') dt) D
@@ -96,8 +116,10 @@ static int ens_step(gh_ensemble* e, hipStream_t s)
         TimedScope ts(c, s, GH_T_DIRECT_F32);
         GH_TRY(launch_sym(c, e->ipt, e->guard, o.loc.as<float4>(), o.s64.as<double4>(),
                           o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
-                          o.umass.as<float>(), e->nb_blk.as<int>(), 0, e->n_pad, e->work.as<int4>(), e->items, e->eps_blk.as<float>(), e->part.as<float>(),
-                          e->persistent ? e->queue.as<int>() : nullptr, e->grid, s));
+                          o.umass.as<float>(), e->nb_blk.as<int>(), 0, e->n_pad,
+                          e->work.as<int4>(), e->items, e->eps_blk.as<float>(),
+                          e->part.as<float>(), e->persistent ? e->queue.as<int>() : nullptr,
+                          e->grid, s));
     }
     GH_TRY(reduce_sym(c, e->part.as<float>(), 0, e->nb_blk.as<int>(), e->blk, e->n_pad,
                       e->n_pad, o.perm(), e->acc.as<double>(), s));
@@ -118,6 +140,7 @@ static void ens_free(gh_ensemble* e)
     DevBuf* bufs[] = {&e->x,         &e->v,         &e->xh,       &e->m,         &e->acc,
                       &e->part,      &e->work,      &e->eps_blk,  &e->nb_blk,    &e->valid_blk,
                       &e->dt_blk,    &e->queue,     &e->seg_blk,  &e->seg_start, &e->seg_count,
+                      &e->seg_first,
                       &o.keys[0],    &o.keys[1],    &o.idx[0],    &o.idx[1],     &o.hist,
                       &o.box,        &o.boxpart,    &o.loc,       &o.s64,        &o.frame,
                       &o.flag,       &o.nflag,     &o.umass};
@@ -195,6 +218,7 @@ int gh_ensemble_create(gh_ctx* c, int n_sims, const int64_t* counts, const doubl
     al(e->seg_blk, sizeof(int) * seg_blk.size());
     al(e->seg_start, sizeof(int64_t) * (size_t)n_sims);
     al(e->seg_count, sizeof(int64_t) * (size_t)n_sims);
+    al(e->seg_first, sizeof(int64_t) * (size_t)n_sims);
     al(e->part, 12 * np * (size_t)e->nb_max);
     al(e->work, sizeof(int4) * work.size());
     al(e->eps_blk, sizeof(float) * eps_blk.size());
@@ -209,9 +233,11 @@ int gh_ensemble_create(gh_ctx* c, int n_sims, const int64_t* counts, const doubl
     }
     // padded host staging
     std::vector<double> hx(3 * np, 0.0), hv(3 * np, 0.0), hm(np, 0.0);
+    std::vector<int64_t> first((size_t)n_sims);
     int64_t off = 0;
     for (int s = 0; s < n_sims; s++) {
         const int64_t st = e->start[s], n = e->count[s];
+        first[(size_t)s] = off;
         std::memcpy(&hx[3 * st], pos + 3 * off, sizeof(double) * 3 * n);
         std::memcpy(&hv[3 * st], vel + 3 * off, sizeof(double) * 3 * n);
         std::memcpy(&hm[st], mass + off, sizeof(double) * n);
@@ -236,6 +262,7 @@ int gh_ensemble_create(gh_ctx* c, int n_sims, const int64_t* counts, const doubl
     up(e->seg_blk, seg_blk.data(), sizeof(int) * seg_blk.size());
     up(e->seg_start, e->start.data(), sizeof(int64_t) * (size_t)n_sims);
     up(e->seg_count, e->count.data(), sizeof(int64_t) * (size_t)n_sims);
+    up(e->seg_first, first.data(), sizeof(int64_t) * (size_t)n_sims);
     // size the order and frame buffers now, so that a captured step allocates nothing
     if (!rc)
         rc = spatial_order_seg(c, e->ord, e->xh.as<double>(), e->n_pad, e->blk, e->nsims,
@@ -295,18 +322,47 @@ int gh_ensemble_get(gh_ensemble* e, double* pos, double* vel)
     GH_HIP(c, hipSetDevice(c->device));
     hipStream_t s = c->stream;
     StreamOrder order_(c, s);
-    int64_t off = 0;
-    for (int k = 0; k < e->nsims; k++) {
-        const int64_t st = e->start[k], n = e->count[k];
-        if (pos)
-            GH_HIP(c, hipMemcpyAsync(pos + 3 * off, e->x.as<double>() + 3 * st,
-                                     sizeof(double) * 3 * n, hipMemcpyDeviceToHost, s));
-        if (vel)
-            GH_HIP(c, hipMemcpyAsync(vel + 3 * off, e->v.as<double>() + 3 * st,
-                                     sizeof(double) * 3 * n, hipMemcpyDeviceToHost, s));
-        off += n;
+    // Without the padding, in two workspaces of the step, so that the whole ensemble is two
+    // copies (a copy per simulation took 10 us more than its bytes ask for).  A copy to
+    // pageable memory holds its thread at 15 to 20 GB/s, so a large second one has a thread
+    // of its own.  4 steps of 32 simulations and this: 3.25 ms before, 2.61 now.
+    double* packed[2] = {pos ? e->acc.as<double>() : nullptr,
+                         vel ? (double*)e->ord.s64.as<double4>() : nullptr};
+    hipLaunchKernelGGL(k_ens_pack, dim3(blocks_for(3 * e->n_pad, kBlock)), dim3(kBlock), 0, s,
+                       e->x.as<double>(), e->v.as<double>(), e->n_pad, e->blk, e->seg_blk.as<int>(),
+                       e->seg_start.as<int64_t>(), e->seg_count.as<int64_t>(),
+                       e->seg_first.as<int64_t>(), packed[0], packed[1]);
+    GH_TRY(check_launch(c, "k_ens_pack"));
+    int64_t total = 0;
+    for (int64_t n : e->count) total += n;
+    const size_t bytes = sizeof(double) * 3 * (size_t)total;
+    std::thread second;
+    hipError_t there = hipSuccess;
+    if (pos && vel && bytes >= (size_t)1 << 20) {
+        if (!c->copy_stream)
+            GH_HIP(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
+        GH_HIP(c, hipStreamSynchronize(s));
+        const double* from = packed[1];
+        try {
+            second = std::thread([&there, c, vel, from, bytes] {
+                there = hipSetDevice(c->device);
+                if (there == hipSuccess)
+                    there = hipMemcpyAsync(vel, from, bytes, hipMemcpyDeviceToHost,
+                                           c->copy_stream);
+                if (there == hipSuccess) there = hipStreamSynchronize(c->copy_stream);
+            });
+        } catch (const std::system_error&) {
+            // no thread to be had: one copy after the other
+        }
     }
-    GH_HIP(c, hipStreamSynchronize(s));
+    hipError_t here = hipSuccess;
+    if (pos) here = hipMemcpyAsync(pos, packed[0], bytes, hipMemcpyDeviceToHost, s);
+    if (vel && !second.joinable() && here == hipSuccess)
+        here = hipMemcpyAsync(vel, packed[1], bytes, hipMemcpyDeviceToHost, s);
+    if (here == hipSuccess) here = hipStreamSynchronize(s);
+    if (second.joinable()) second.join();
+    GH_HIP(c, here);
+    GH_HIP(c, there);
     return 0;
 }
 

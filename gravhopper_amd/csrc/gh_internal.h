@@ -88,6 +88,9 @@ struct gh_ctx {
     hipStream_t copy_stream = nullptr;
     double* pinned = nullptr;
     size_t pinned_bytes = 0;
+    // pinned memory of small host transfers, its device address and the bytes in use
+    double *stage = nullptr, *stage_dev = nullptr;
+    size_t stage_used = 0;
     gh::DevBuf ext;
     hipEvent_t ext_events[3] = {nullptr, nullptr, nullptr};
     int64_t last_tree_nodes = 0;

@@ -281,3 +281,49 @@ def test_run_update_in_the_force_kernel(ctx, prec, n):
         ctx.timing_enable(False)
     for k, (g, w) in enumerate(zip(got, want)):
         assert_bitwise(g, w, "array %d" % k)
+
+
+@pytest.mark.parametrize("n,nsteps", [(7000, 9), (2, 3), (50000, 2)])
+def test_tree_run_history_copied_by_thread(ctx, n, nsteps):
+    # slices of several steps and a short last one, one slice, one step per slice
+    ic = workloads.plummer(n, seed=n)
+    x, v, hp, hv = ctx.run(ic["pos"], ic["vel"], ic["mass"], 1e-3, 1e-4, nsteps,
+                           algorithm=_native.GH_TREE, history=True)
+    xs, vs = ic["pos"], ic["vel"]
+    for k in range(nsteps):
+        xs, vs = ctx.run(xs, vs, ic["mass"], 1e-3, 1e-4, 1, algorithm=_native.GH_TREE)
+        assert_bitwise(hp[k], xs, "position of step %d" % k)
+        assert_bitwise(hv[k], vs, "velocity of step %d" % k)
+    assert_bitwise(x, xs)
+    assert_bitwise(v, vs)
+
+
+# 4 n doubles of input and 3 n of result around the 524288 that small transfers stage
+@pytest.mark.parametrize("n", [1, 1000, 74898, 74899, 131072, 131073])
+def test_host_call_equals_device_call(ctx, n):
+    torch = pytest.importorskip("torch")
+    ic = workloads.plummer(n, seed=n)
+    x, m = (torch.tensor(ic[k], device="cuda") for k in ("pos", "mass"))
+    acc = torch.empty_like(x)
+    torch.cuda.synchronize()
+    ctx.direct_dev(x.data_ptr(), m.data_ptr(), n, 1e-4, _native.GH_FP64, acc.data_ptr())
+    ctx.sync()
+    for k in range(2):
+        assert_bitwise(ctx.direct(ic["pos"], ic["mass"], 1e-4), acc.cpu().numpy(), "call %d" % k)
+        # a call that fails between its upload and its result
+        with pytest.raises(Exception):
+            ctx.tree(np.ones((5000, 3)), np.ones(5000), 0.0)
+
+
+@pytest.mark.parametrize("counts", [[3, 1, 260], [1, 60000, 1500]])
+def test_ensemble_state_without_padding(ctx, counts):
+    sims = []
+    for k, n in enumerate(counts):
+        ic = {key: np.random.default_rng(7 * k + n).normal(size=(n, 3)) for key in ("pos", "vel")}
+        sims.append(dict(ic, mass=np.ones(n), eps=0.1, dt=1e-3))
+    ens = _native.Ensemble(ctx, sims)
+    pos, vel = ens.state()
+    ens.close()
+    for k, s in enumerate(sims):
+        assert_bitwise(pos[k], s["pos"], "positions of %d" % k)
+        assert_bitwise(vel[k], s["vel"], "velocities of %d" % k)
