@@ -39,10 +39,16 @@ __device__ __forceinline__ float rotn(float v)
 
 // The particles are in the sorted order of gh_frames.hip and the workgroup works in
 // block I's frame, as the force kernel does: src holds local FP32 coordinates and
-// masses, block J's coordinates are shifted by fl(o_J - o_I).  The DS instance takes the
-// items with a flagged block, with both sides as hi + lo words of FP64 differences
-// from o_I (src64), and separations (hi_j - hi_k) + (lo_j - lo_k).
-// j-side records in LDS: (x, y, z, m), (mu_x, mu_y, mu_z, 0) and, DS, (lo x, y, z, 0).
+// masses, block J's coordinates are shifted by fl(o_J - o_I).  DS, the items with a flagged
+// block: both sides as hi + lo words of FP64 differences from o_I (src64), and separations
+// (hi_j - hi_k) + (lo_j - lo_k).  Padding is left out as in the force kernel.
+// j-side records in LDS: (x, y, z, m) and (mu_x, mu_y, mu_z), each chunk of 64 twice in a row
+// so that lane l's rotating index l + s needs no wrap-around; DS has each once and, in the
+// place of the other, (lo x, y, z).
+struct Vec3 {
+    float x, y, z;
+};
+
 __device__ __forceinline__ void split_pair(double d, float& hi, float& lo)
 {
     hi = (float)d;
@@ -50,24 +56,17 @@ __device__ __forceinline__ void split_pair(double d, float& hi, float& lo)
 }
 
 template <int IPT, bool GUARD, bool DS>
-__global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict__ src,
-                                                        const double4* __restrict__ src64,
-                                                        const double4* __restrict__ frame,
-                                                        const int* __restrict__ flag,
-                                                        const float4* __restrict__ mu,
-                                                        int64_t np_pad,
-                                                        const int4* __restrict__ work,
-                                                        float eps2, float4* __restrict__ part)
+__device__ __forceinline__ void vjp_item(const float4* __restrict__ src,
+                                         const double4* __restrict__ src64,
+                                         const double4* __restrict__ frame,
+                                         const float4* __restrict__ mu, int64_t np_pad, int4 it,
+                                         float eps2, int nI, int nJ, float4* __restrict__ part,
+                                         float4* tp, Vec3* tm, float (*jp)[8][64])
 {
     constexpr int BLK = kBlock * IPT;
-    constexpr int NCH = BLK / 64;
-    __shared__ float4 tp[NCH * 128];
-    __shared__ float4 tm[NCH * 128];
-    __shared__ float4 tl[DS ? NCH * 128 : 1];
-    __shared__ float jp[kBlock / 64][8][64];
-    const int4 it = work[blockIdx.x];
+    constexpr int ROW = DS ? 64 : 128;
+    Vec3* const tl = tm + (DS ? BLK : 0);
     const int I = it.x, J = it.y;
-    if ((flag[I] | flag[J]) != (DS ? 1 : 0)) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t ibase = (int64_t)I * BLK + wave * 64 * IPT + lane;
     const int64_t jbase = (int64_t)J * BLK;
@@ -103,16 +102,16 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
         const double4 oJ = frame[J];
         const float offx = (float)(oJ.x - oI.x), offy = (float)(oJ.y - oI.y),
                     offz = (float)(oJ.z - oI.z);
-        for (int q = threadIdx.x; q < NCH * 128; q += kBlock) {
-            const int64_t g = jbase + (q >> 7) * 64 + (q & 63);
+        for (int q = threadIdx.x; q < BLK / 64 * ROW; q += kBlock) {
+            const int64_t g = jbase + q / ROW * 64 + (q & 63);
             if (DS) {
                 const double4 v = src64[g];
-                float4 h, l;
+                float4 h;
+                Vec3 l;
                 split_pair(v.x - oI.x, h.x, l.x);
                 split_pair(v.y - oI.y, h.y, l.y);
                 split_pair(v.z - oI.z, h.z, l.z);
                 h.w = (float)v.w;
-                l.w = 0.f;
                 tp[q] = h;
                 tl[q] = l;
             } else {
@@ -122,20 +121,23 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
                 v.z += offz;
                 tp[q] = v;
             }
-            tm[q] = mu[g];
+            const float4 u = mu[g];
+            tm[q] = Vec3{u.x, u.y, u.z};
         }
     }
     __syncthreads();
 
+    const bool live = wave * 64 * IPT < nI;
+    const int chunks = (nJ + 63) / 64;
     if (I == J) {
         // one-sided over the block, self pair excluded
-        for (int c = 0; c < NCH; c++) {
-#pragma unroll 4
+        for (int c = 0; c < (live ? chunks : 0); c++) {
+#pragma unroll(DS ? 1 : 4)
             for (int q = 0; q < 64; q++) {
-                const float4 s = tp[c * 128 + q];
-                const float4 m4 = tm[c * 128 + q];
-                float4 sl = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (DS) sl = tl[c * 128 + q];
+                const float4 s = tp[c * ROW + q];
+                const Vec3 m4 = tm[c * ROW + q];
+                Vec3 sl = {0.f, 0.f, 0.f};
+                if (DS) sl = tl[c * ROW + q];
                 const int jl = c * 64 + q;
 #pragma unroll
                 for (int k = 0; k < IPT; k++) {
@@ -170,18 +172,16 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
             }
         }
     } else {
-        for (int c = 0; c < NCH; c++) {
-            const float4* rp = &tp[c * 128 + lane];
-            const float4* rm = &tm[c * 128 + lane];
-            const float4* rl = &tl[DS ? c * 128 + lane : 0];
+        for (int c = 0; c < chunks; c++) {
             float a = 0.f, bx = 0.f, by = 0.f, bz = 0.f, cx = 0.f, cy = 0.f, cz = 0.f, l = 0.f;
-            for (int s0 = 0; s0 < 64; s0 += 4) {
-#pragma unroll
+            for (int s0 = 0; s0 < (live ? 64 : 0); s0 += 4) {
+#pragma unroll(DS ? 1 : 4)
                 for (int st = 0; st < 4; st++) {
-                    const float4 s = rp[s0 + st];
-                    const float4 m4 = rm[s0 + st];
-                    float4 sl = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (DS) sl = rl[s0 + st];
+                    const int q = c * ROW + (DS ? (lane + s0 + st) & 63 : lane + s0 + st);
+                    const float4 s = tp[q];
+                    const Vec3 m4 = tm[q];
+                    Vec3 sl = {0.f, 0.f, 0.f};
+                    if (DS) sl = tl[q];
 #pragma unroll
                     for (int k = 0; k < IPT; k++) {
                         float dx = s.x - xk[k], dy = s.y - yk[k], dz = s.z - zk[k];
@@ -230,28 +230,23 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
                     l = rotn(l);
                 }
             }
-            // lane l holds this wavefront's sums for j = chunk particle l
-            jp[wave][0][lane] = a;
-            jp[wave][1][lane] = bx;
-            jp[wave][2][lane] = by;
-            jp[wave][3][lane] = bz;
-            jp[wave][4][lane] = cx;
-            jp[wave][5][lane] = cy;
-            jp[wave][6][lane] = cz;
-            jp[wave][7][lane] = l;
+            // lane l holds this wavefront's sums for j = chunk particle l; wavefront 0 adds the
+            // others' to its own
+            float r[8] = {a, bx, by, bz, cx, cy, cz, l};
+            if (wave > 0) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) jp[wave - 1][q][lane] = r[q];
+            }
             __syncthreads();
-            if (threadIdx.x < 64) {
-                const int t = threadIdx.x;
-                float r[8];
+            if (wave == 0) {
+                const int t = lane;
 #pragma unroll
                 for (int q = 0; q < 8; q++) {
-                    float acc = jp[0][q][t];
 #pragma unroll
-                    for (int w = 1; w < kBlock / 64; w++) acc += jp[w][q][t];
-                    r[q] = acc;
+                    for (int w = 1; w < kBlock / 64; w++) r[q] += jp[w - 1][q][t];
                 }
-                const float4 sj = tp[c * 128 + t];
-                const float4 mj = tm[c * 128 + t];
+                const float4 sj = tp[c * ROW + t];
+                const Vec3 mj = tm[c * ROW + t];
                 // g_j = -mu_j A' + m_j B' - C',  lm_j = L'
                 const float4 o = make_float4(
                     __builtin_fmaf(sj.w, r[1], -mj.x * r[0]) - r[4],
@@ -262,6 +257,7 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
             __syncthreads();
         }
     }
+    if (!live) return;
 #pragma unroll
     for (int k = 0; k < IPT; k++) {
         // g_k = m_k A - B mu_k + C,  lm_k = -L
@@ -270,6 +266,31 @@ __global__ __launch_bounds__(kBlock) void k_vjp_sym_f32(const float4* __restrict
                                      __builtin_fmaf(mk[k], Az[k], -B[k] * uz[k]) + Cz[k], -L[k]);
         part[(int64_t)it.z * np_pad + ibase + k * 64] = o;
     }
+}
+
+// Bound by the issue of VALU instructions: 44 per pair and lane, of which 8 are DPP moves (4.4
+// cycles each, 2.4 the others, 8.3 the square root).  Padding left out, 28 instead of 32 bytes
+// a particle in LDS and one launch for both forms (the flagged items' own took 4.6 us):
+// N = 16384 195 -> 177 us, 20000 264 -> 229, 40000 889 -> 843, 100000 4747 -> 4530.
+template <int IPT, bool GUARD>
+__global__ __launch_bounds__(kBlock, IPT == 1 ? 6 : IPT == 2 ? 4 : 2) void k_vjp_sym_f32(
+    const float4* __restrict__ src, const double4* __restrict__ src64,
+    const double4* __restrict__ frame, const int* __restrict__ flag,
+    const int* __restrict__ used, const float4* __restrict__ mu, int64_t np_pad,
+    const int4* __restrict__ work, float eps2, float4* __restrict__ part)
+{
+    constexpr int NCH = kBlock * IPT / 64;
+    __shared__ float4 tp[NCH * 128];
+    __shared__ Vec3 tm[NCH * 128];
+    __shared__ float jp[kBlock / 64 - 1][8][64];
+    const int4 it = work[blockIdx.x];
+    const int nI = used[it.x], nJ = used[it.y];
+    if ((flag[it.x] | flag[it.y]) == 0)
+        vjp_item<IPT, GUARD, false>(src, nullptr, frame, mu, np_pad, it, eps2, nI, nJ, part, tp,
+                                    tm, jp);
+    else
+        vjp_item<IPT, GUARD, true>(nullptr, src64, frame, mu, np_pad, it, eps2, nI, nJ, part, tp,
+                                   tm, jp);
 }
 
 // mv = lv + c lx; mu = dt A mv (FP32 copy for the pair kernel, in sorted order: mu[p]
@@ -353,25 +374,6 @@ static int copy_d(gh_ctx* c, const double* a, double* b, int64_t n, hipStream_t 
     return check_launch(c, "k_copy_d");
 }
 
-__global__ __launch_bounds__(kBlock) void k_copy_u32(const u32* __restrict__ a,
-                                                     u32* __restrict__ b, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) b[i] = a[i];
-}
-
-// Puts back a spatial order that the forward replay saved for the same positions and
-// clears the count of flagged groups as k_morton does: the order buffers are then as
-// spatial_order leaves them, without sorting again.
-__global__ __launch_bounds__(kBlock) void k_restore_order(const u32* __restrict__ saved,
-                                                          u32* __restrict__ perm, int64_t n,
-                                                          int* __restrict__ nflag)
-{
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i == 0) *nflag = 0;
-    if (i < n) perm[i] = saved[i];
-}
-
 static int vjp_ipt(int64_t n)
 {
     if (n >= 65536) return 4;
@@ -387,10 +389,8 @@ static void launch_vjp_g(unsigned items, hipStream_t s, const OrderBufs& o, cons
     const double4* s64 = o.s64.as<double4>();
     const double4* fr = o.frame.as<double4>();
     const int* fl = o.flag.as<int>();
-    hipLaunchKernelGGL((k_vjp_sym_f32<IPT, GUARD, false>), dim3(items), dim3(kBlock), 0, s, src,
-                       s64, fr, fl, mu, np_pad, work, eps2, part);
-    hipLaunchKernelGGL((k_vjp_sym_f32<IPT, GUARD, true>), dim3(items), dim3(kBlock), 0, s, src,
-                       s64, fr, fl, mu, np_pad, work, eps2, part);
+    hipLaunchKernelGGL((k_vjp_sym_f32<IPT, GUARD>), dim3(items), dim3(kBlock), 0, s, src, s64, fr,
+                       fl, o.used.as<int>(), mu, np_pad, work, eps2, part);
 }
 
 template <int IPT>
@@ -445,17 +445,16 @@ static int reverse_step(gh_ctx* c, const AdjWork& w, const double* xh, const dou
     double* mv = c->adj_mv.as<double>();
     float4* part = c->adj_part.as<float4>();
     OrderBufs& o = c->ord_p;
-    if (saved && o.sorted_n == n) {
-        hipLaunchKernelGGL(k_restore_order, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
-                           saved, o.idx[o.sel].as<u32>(), n, o.nflag.as<int>());
-        GH_TRY(check_launch(c, "k_restore_order"));
-        o.sorted = xh;
-    } else {
+    const u32* perm = saved;
+    if (!saved) {
         GH_TRY(spatial_order(c, o, xh, n, s));
+        perm = o.perm();
     }
-    GH_TRY(gather_frames(c, o, xh, m, o.perm(), n, w.n_pad, kBlock * w.ipt, nullptr, true, s));
+    // (the count of flagged blocks that this adds to is read by forces only, after an order of
+    // their own has cleared it)
+    GH_TRY(gather_frames(c, o, xh, m, perm, n, w.n_pad, kBlock * w.ipt, nullptr, true, s));
     hipLaunchKernelGGL(k_adj_pre, dim3(blocks_for(w.n_pad, kBlock)), dim3(kBlock), 0, s, lx, lv,
-                       n, w.n_pad, o.perm(), cdrift, dtA, mv, mu);
+                       n, w.n_pad, perm, cdrift, dtA, mv, mu);
     GH_TRY(check_launch(c, "k_adj_pre"));
     const float eps2 = (float)(eps * eps);
     const bool guard = fp32_guard(eps);
@@ -470,7 +469,7 @@ static int reverse_step(gh_ctx* c, const AdjWork& w, const double* xh, const dou
         GH_TRY(check_launch(c, "k_vjp_sym_f32"));
     }
     hipLaunchKernelGGL(k_adj_post, dim3(blocks_for(n, 64)), dim3(kBlock), 0, s, part, w.nb,
-                       w.n_pad, n, o.perm(), mv, cdrift, lx, lv, lm);
+                       w.n_pad, n, perm, mv, cdrift, lx, lv, lm);
     return check_launch(c, "k_adj_post");
 }
 
@@ -504,13 +503,9 @@ static int forward_segment(gh_ctx* c, double* x, double* v, const double* m, int
         if (n > 1) {
             OrderBufs& o = c->ord_p;
             o.sorted = nullptr;
+            OrderTo to(o, hperm ? hperm + st * n : nullptr);
             GH_TRY(direct_dev(c, xh, m, n, nullptr, n, eps, precision, acc, s, &up, &updated));
-            if (hperm && have && o.sorted == xh && o.sorted_n == n) {
-                hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
-                                   o.perm(), hperm + st * n, n);
-                GH_TRY(check_launch(c, "k_copy_u32"));
-                (*have)[(size_t)st] = 1;
-            }
+            if (hperm && have && o.sorted == xh && o.sorted_n == n) (*have)[(size_t)st] = 1;
         } else {
             GH_TRY(zero_dev(c, acc, n3, s));
         }

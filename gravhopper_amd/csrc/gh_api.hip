@@ -598,7 +598,7 @@ void gh_ctx_destroy(gh_ctx* c)
     for (OrderBufs* o : {&c->ord_p, &c->ord_t}) {
         DevBuf* ob[] = {&o->keys[0], &o->keys[1], &o->idx[0], &o->idx[1], &o->hist, &o->box,
                         &o->boxpart, &o->loc,     &o->s64,    &o->frame,  &o->flag,
-                        &o->nflag,   &o->umass};
+                        &o->nflag,   &o->umass,   &o->used};
         for (DevBuf* b : ob) release(c, *b);
     }
     release_spans(c);

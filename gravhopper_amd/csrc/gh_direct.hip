@@ -579,13 +579,14 @@ struct SymOut {
 // simulation) and the slot of the j-side field (I's index within its simulation).
 // UNI: the particles of block I all have mass mI and those of block J mass mJ, so the masses
 // multiply the sums instead of every pair's factor: 15 instead of 17 VALU operations per
-// pair.
+// pair.  nI, nJ: the particles of either block.  Wavefronts that hold only padding, and
+// chunks of it, are left out: padding is massless, its terms are zeros.
 template <int IPT, bool GUARD, bool DS, bool UNI>
 __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
                                          const double4* __restrict__ s64,
                                          const double4* __restrict__ frame, int64_t np_pad,
-                                         int4 it, float eps2, float mI, float mJ,
-                                         const SymOut out, float4* tile, float (*jp)[3][64])
+                                         int4 it, float eps2, float mI, float mJ, int nI,
+                                         int nJ, const SymOut out, float4* tile, float (*jp)[3][64])
 {
     constexpr int BLK = kBlock * IPT;
     constexpr int NCH = BLK / 64;
@@ -646,8 +647,10 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
     }
     __syncthreads();
 
+    const bool live = wave * 64 * IPT < nI;
+    const int chunks = (nJ + 63) / 64;
     if (I == J) {
-        for (int c = 0; c < NCH; c++) {
+        for (int c = 0; c < (live ? chunks : 0); c++) {
 #pragma unroll(DS ? 1 : 8)
             for (int q = 0; q < 64; q++) {
                 const float4 s = tile[c * ROW + q];
@@ -674,9 +677,9 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
             }
         }
     } else {
-        for (int c = 0; c < NCH; c++) {
+        for (int c = 0; c < chunks; c++) {
             float fx = 0.f, fy = 0.f, fz = 0.f;
-            for (int s0 = 0; s0 < 64; s0 += 8) {
+            for (int s0 = 0; s0 < (live ? 64 : 0); s0 += 8) {
 #pragma unroll(DS ? 1 : 8)
                 for (int s = 0; s < 8; s++) {
                     const int q = c * ROW + (DS ? (lane + s0 + s) & 63 : lane + s0 + s);
@@ -729,6 +732,7 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
             __syncthreads();
         }
     }
+    if (!live) return;
 #pragma unroll
     for (int k = 0; k < IPT; k++) {
         float* o = out.part + ((int64_t)it.z * np_pad + ibase + k * 64) * 3;
@@ -752,14 +756,17 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
 //    equal masses, per launch): 13.33 -> 11.98 ms.  Below kUniMin the sort, the reduction
 //    and the launches are a growing share of a step (N = 16384: 2 % of a gradient gained),
 //    and results keep the bits of the general form.
+//  - Registers for six wavefronts per SIMD where a lane has one particle and five otherwise,
+//    as LDS allows: N = 16384 118 -> 113 us a call, 32768 334 -> 319 (four lose 3 % at 65536
+//    and beyond).  Padding left out: 128 spheres of 1024 to 65536 15.0 -> 14.6 ms a step.
 constexpr int kUniMin = 131072;
 
 template <int IPT, bool GUARD>
-__global__ __launch_bounds__(kBlock) void k_direct_sym_f32(
+__global__ __launch_bounds__(kBlock, IPT == 1 ? 6 : 5) void k_direct_sym_f32(
     const float4* __restrict__ src, const double4* __restrict__ s64,
     const double4* __restrict__ frame, const int* __restrict__ flag,
     const int* __restrict__ nflag, const float* __restrict__ umass,
-    const int* __restrict__ nb_blk, int nb, int64_t np_pad, const int4* __restrict__ work,
+    const int* __restrict__ used, const int* __restrict__ nb_blk, int nb, int64_t np_pad, const int4* __restrict__ work,
     int64_t items, const float* __restrict__ eps2_blk, const SymOut out, int* __restrict__ queue)
 {
     constexpr int NCH = kBlock * IPT / 64;
@@ -785,16 +792,17 @@ __global__ __launch_bounds__(kBlock) void k_direct_sym_f32(
         const bool ds = (flag[it.x] | flag[it.y]) != 0;
         const float mI = umass[it.x], mJ = umass[it.y], eps2 = eps2_blk[it.x];
         const int blocks = nb_blk ? nb_blk[it.x] : nb;
+        const int nI = used[it.x], nJ = used[it.y];
         if (ds && flagged == first)
             sym_item<IPT, GUARD, true, false>(nullptr, s64, frame, np_pad, it, eps2, 0.f, 0.f,
-                                              out, tile, jp);
+                                              nI, nJ, out, tile, jp);
         else if (!ds && !flagged && !GUARD && blocks >= kUniMin / (kBlock * IPT) && mI == mI &&
                  mJ == mJ)
             sym_item<IPT, GUARD, false, !GUARD>(src, nullptr, frame, np_pad, it, eps2, mI, mJ,
-                                                out, tile, jp);
+                                                nI, nJ, out, tile, jp);
         else if (!ds && !flagged)
             sym_item<IPT, GUARD, false, false>(src, nullptr, frame, np_pad, it, eps2, 0.f, 0.f,
-                                               out, tile, jp);
+                                               nI, nJ, out, tile, jp);
         if (!queue) break;
         __syncthreads();
         if (flagged) k += gridDim.x;
@@ -1032,7 +1040,7 @@ int sym_ipt(gh_ctx* c, int64_t np)
 
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,
                const double4* frame, const int* flag, const int* nflag, const float* umass,
-               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
+               const int* used, const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
                const float* eps2_blk, float* part,
                int* queue, unsigned persistent_grid, hipStream_t s, float* jpart, int64_t jstride,
                int64_t joff)
@@ -1049,12 +1057,12 @@ int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4*
     case IPT:                                                                                  \
         if (guard)                                                                             \
             hipLaunchKernelGGL((k_direct_sym_f32<IPT, true>), dim3(grid), dim3(kBlock), 0, s,  \
-                               src, s64, frame, flag, nflag, umass, nb_blk, nb, np_pad, work,  \
-                               items, eps2_blk, out, queue);                                   \
+                               src, s64, frame, flag, nflag, umass, used, nb_blk, nb, np_pad,  \
+                               work, items, eps2_blk, out, queue);                             \
         else                                                                                   \
             hipLaunchKernelGGL((k_direct_sym_f32<IPT, false>), dim3(grid), dim3(kBlock), 0, s, \
-                               src, s64, frame, flag, nflag, umass, nb_blk, nb, np_pad, work,  \
-                               items, eps2_blk, out, queue);                                   \
+                               src, s64, frame, flag, nflag, umass, used, nb_blk, nb, np_pad,  \
+                               work, items, eps2_blk, out, queue);                             \
         break
     switch (ipt) {
         GH_SYM(1);
@@ -1142,8 +1150,8 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
             TimedScope ts(c, s, GH_T_DIRECT_F32);
             GH_TRY(launch_sym(c, ipt, guard, o.loc.as<float4>(), o.s64.as<double4>(),
                               o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
-                              o.umass.as<float>(), nullptr, nb, np_pad, c->work.as<int4>(), items,
-                              c->eps_blk.as<float>(), part, nullptr, 0, s));
+                              o.umass.as<float>(), o.used.as<int>(), nullptr, nb, np_pad,
+                              c->work.as<int4>(), items, c->eps_blk.as<float>(), part, nullptr, 0, s));
         }
         if (up) *updated = true;
         return reduce_sym(c, part, nb, nullptr, (int)blk, np_pad, np, o.perm(), d_acc, s, up);
@@ -1156,8 +1164,8 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
             TimedScope ts(c, s, GH_T_DIRECT_F32);
             GH_TRY(launch_sym(c, ipt, guard, o.loc.as<float4>(), o.s64.as<double4>(),
                               o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
-                              o.umass.as<float>(), nullptr, nb, np_pad, c->work.as<int4>() + i0, ni,
-                              c->eps_blk.as<float>(), part, nullptr, 0, s, partj,
+                              o.umass.as<float>(), o.used.as<int>(), nullptr, nb, np_pad,
+                              c->work.as<int4>() + i0, ni, c->eps_blk.as<float>(), part, nullptr, 0, s, partj,
                               (int64_t)w * blk, (int64_t)c0 * blk));
         }
         hipLaunchKernelGGL(k_reduce_band, dim3(blocks_for(3 * np, kBlock)), dim3(kBlock), 0, s,

@@ -116,7 +116,7 @@ static int ens_step(gh_ensemble* e, hipStream_t s)
         TimedScope ts(c, s, GH_T_DIRECT_F32);
         GH_TRY(launch_sym(c, e->ipt, e->guard, o.loc.as<float4>(), o.s64.as<double4>(),
                           o.frame.as<double4>(), o.flag.as<int>(), o.nflag.as<int>(),
-                          o.umass.as<float>(), e->nb_blk.as<int>(), 0, e->n_pad,
+                          o.umass.as<float>(), o.used.as<int>(), e->nb_blk.as<int>(), 0, e->n_pad,
                           e->work.as<int4>(), e->items, e->eps_blk.as<float>(),
                           e->part.as<float>(), e->persistent ? e->queue.as<int>() : nullptr,
                           e->grid, s));
@@ -143,7 +143,7 @@ static void ens_free(gh_ensemble* e)
                       &e->seg_first,
                       &o.keys[0],    &o.keys[1],    &o.idx[0],    &o.idx[1],     &o.hist,
                       &o.box,        &o.boxpart,    &o.loc,       &o.s64,        &o.frame,
-                      &o.flag,       &o.nflag,     &o.umass};
+                      &o.flag,       &o.nflag,     &o.umass,     &o.used};
     for (DevBuf* b : bufs) release(c, *b);
 }
 

@@ -153,7 +153,7 @@ static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, i
                       hipStream_t s)
 {
     const dim3 runs((unsigned)(n_pad / run)), blocks((unsigned)(n_pad / 64)), threads(kRunThreads);
-    u32 *keys = o.keys[0].as<u32>(), *from = o.keys[1].as<u32>(), *perm = o.idx[0].as<u32>();
+    u32 *keys = o.keys[0].as<u32>(), *from = o.keys[1].as<u32>(), *perm = o.kept ? o.kept : o.idx[0].as<u32>();
 #define GH_RANK(RUN)                                                                          \
     case RUN:                                                                                 \
         hipLaunchKernelGGL(k_rank_runs<RUN>, runs, threads, 0, s, d_pos, n, seg, start, count, \
@@ -171,6 +171,13 @@ static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, i
 #undef GH_RANK
     o.sel = 0;
     return check_launch(c, "k_run_merge");
+}
+
+__global__ __launch_bounds__(kBlock) void k_copy_order(const u32* __restrict__ a,
+                                                       u32* __restrict__ b, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) b[i] = a[i];
 }
 
 // Every run forms the box of all its segment's points, and every 64 points search all its runs,
@@ -211,6 +218,11 @@ int spatial_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, hipSt
     // 65536 particles, 1024-particle blocks: median relative error 3.0e-8 with 10 levels,
     // 3.4e-8 with 16) and cost two more passes.
     GH_TRY(radix_sort(c, o.keys, o.idx, o.hist, n, 1, kKeyShift, s, &o.sel, 63));
+    if (o.kept) {
+        hipLaunchKernelGGL(k_copy_order, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s,
+                           o.idx[o.sel].as<u32>(), o.kept, n);
+        GH_TRY(check_launch(c, "k_copy_order"));
+    }
     o.sorted = d_pos;
     o.sorted_n = n;
     return 0;
@@ -349,7 +361,8 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
                                                    double4* __restrict__ frame,
                                                    int* __restrict__ flag,
                                                    int* __restrict__ nflag,
-                                                   float* __restrict__ umass)
+                                                   float* __restrict__ umass,
+                                                   int* __restrict__ used)
 {
     __shared__ float sLo[kBlock / 64], sHi[kBlock / 64];
     __shared__ double sR[kBlock / 64];
@@ -419,6 +432,7 @@ __global__ __launch_bounds__(kBlock) void k_frames(const double* __restrict__ po
             mlo = fminf(mlo, sLo[w]);
             mhi = fmaxf(mhi, sHi[w]);
         }
+        used[blockIdx.x] = cnt;
         umass[blockIdx.x] = mlo == mhi ? mlo : __builtin_nanf("");
         // log2 R - mean log2 gap > kFrameLog2, in integer exponents
         const long long eR = exponent_of(R);
@@ -442,11 +456,13 @@ int gather_frames(gh_ctx* c, OrderBufs& o, const double* d_pos, const double* d_
     GH_TRY(ensure(c, o.flag, sizeof(int) * (size_t)ng));
     GH_TRY(ensure(c, o.nflag, 256));
     GH_TRY(ensure(c, o.umass, sizeof(float) * (size_t)ng));
+    GH_TRY(ensure(c, o.used, sizeof(int) * (size_t)ng));
     double4* s64 = want_s64 ? o.s64.as<double4>() : nullptr;
 #define GH_FRAMES(GG)                                                                       \
     hipLaunchKernelGGL(k_frames<GG>, dim3((unsigned)ng), dim3(kBlock), 0, s, d_pos, d_mass,  \
                        perm, n, valid, o.loc.as<float4>(), s64, o.frame.as<double4>(),       \
-                       o.flag.as<int>(), o.nflag.as<int>(), o.umass.as<float>())
+                       o.flag.as<int>(), o.nflag.as<int>(), o.umass.as<float>(),              \
+                       o.used.as<int>())
     switch (group) {
         case 256: GH_FRAMES(256); break;
         case 512: GH_FRAMES(512); break;

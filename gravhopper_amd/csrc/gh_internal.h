@@ -50,10 +50,25 @@ struct OrderBufs {
     DevBuf flag;   // int per group: 1 if the group is not compact (see k_frames)
     DevBuf nflag;  // int: number of flagged groups (cleared by the key kernels)
     DevBuf umass;  // float per group: the mass all its points share, else NaN
+    DevBuf used;   // int per group: its points, padding behind them
     int sel = 0;   // which of idx[0] / idx[1] holds the order
     const double* sorted = nullptr;  // positions spatial_order last ordered (n of them)
     int64_t sorted_n = 0;
-    const u32* perm() const { return idx[sel].as<u32>(); }
+    u32* kept = nullptr;  // where spatial_order leaves its order instead (OrderTo)
+    const u32* perm() const { return kept ? kept : idx[sel].as<u32>(); }
+};
+
+// While it lives, spatial_order leaves its orders in `to` (nullable: in o's own buffers), which
+// does not outlive the call.
+struct OrderTo {
+    OrderBufs& o;
+    OrderTo(OrderBufs& o_, u32* to) : o(o_) { o.kept = to; }
+    ~OrderTo()
+    {
+        if (o.kept) o.sorted = nullptr;
+        o.kept = nullptr;
+    }
+    OrderTo(const OrderTo&) = delete;
 };
 
 }  // namespace gh
@@ -219,13 +234,13 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
                double eps, double* d_acc, hipStream_t s, const StepUpdate* up = nullptr,
                bool* updated = nullptr);
 // The pair-once kernel over a block-pair list (src: local FP32 coordinates per sorted
-// particle, s64: the same particles in FP64, frame/flag/umass: per block), followed by its
+// particle, s64: the same particles in FP64, frame/flag/umass/used: per block), followed by its
 // double-single instance for the items with a flagged block.
 // jpart (nullable): the j-side partials go to jpart[slot_j][p - joff] with a stride of
 // jstride particles instead of part.
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,
                const double4* frame, const int* flag, const int* nflag, const float* umass,
-               const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
+               const int* used, const int* nb_blk, int nb, int64_t np_pad, const int4* work, int64_t items,
                const float* eps2_blk, float* part, int* queue, unsigned persistent_grid,
                hipStream_t s, float* jpart = nullptr, int64_t jstride = 0, int64_t joff = 0);
 // acc[perm[p]] (perm nullable) = the FP64 sum of particle p's partial slots

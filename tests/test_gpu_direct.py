@@ -318,3 +318,21 @@ def test_fp32_direct_block_masses(ctx, n):
     want = ctx.direct(ic["pos"], mass, 2e-5, FP64)[some]
     e = rel_err(got[some], want)
     assert np.median(e) <= 1e-6 and np.percentile(e, 99) <= 1e-4, (np.median(e), e.max())
+
+
+# a last block with a few particles, a quarter, and all but one; banded too
+@pytest.mark.parametrize("ipt,n", [(1, 257), (1, 321), (2, 1025), (2, 1535), (4, 1025), (4, 1281),
+                                   (4, 4095)])
+def test_fp32_pair_once_leaves_padding_out(ctx, ipt, n):
+    ic = workloads.plummer(n, b=1e-3, mass=1e6, seed=n)
+    ref = ctx.direct(ic["pos"], ic["mass"], 1e-4, FP64)
+    ctx.set_tuning(_native.TUNE_DIRECT_SELF, ipt)
+    try:
+        got = ctx.direct(ic["pos"], ic["mass"], 1e-4, FP32)
+        ctx.set_tuning(_native.TUNE_SYM_BAND, 1)
+        band = ctx.direct(ic["pos"], ic["mass"], 1e-4, FP32)
+    finally:
+        ctx.set_tuning(_native.TUNE_SYM_BAND, 0)
+        ctx.set_tuning(_native.TUNE_DIRECT_SELF, 0)
+    for e in (rel_err(got, ref), rel_err(band, ref)):
+        assert np.median(e) <= FP32_MEDIAN and np.percentile(e, 99) <= FP32_P99
