@@ -1058,6 +1058,14 @@ __device__ __forceinline__ int64_t xcd_block(int64_t per_xcd)
 // receives each target's list length.
 constexpr int kStackCap = 768;
 constexpr int kListCap = 128;
+// Entries a lane evaluates at once.  One at a time every entry waits for its LDS read and its
+// square root; eight take registers that cost a wavefront per SIMD.  With four, the counters of
+// the walk in scalar registers and pushes without branches, a walk of 2^20 particles (16 per
+// group) went from 735 to 660 us, of 10^5 (one per group) from 190 to 166; at theta = 0.4 of
+// 2^20 from 3.95 to 3.6 ms.  Five of seven wavefronts per SIMD are there on average, as both of
+// a workgroup have to end; a grid of resident wavefronts that take groups from counters (80 us
+// of atomics) or in turn (longest wavefront) was slower.
+constexpr int kEvalUnroll = 4;
 // Walk prefixes (k_walk_prefix): groups per block, accepted nodes and steps at most, the
 // stack ids a group's walk may start with, and the ints of one block's state (stack
 // height, list length, stack, list).
@@ -1183,19 +1191,39 @@ __device__ __forceinline__ void walk_lists(
             ax += fx; ay += fy; az += fz;
         } else {
             float fx = 0.f, fy = 0.f, fz = 0.f;
-            for (int j = slice; j < take; j += nslices) {
-                const Entry e = list[j];
-                const float ex = (float)e.x - tx, ey = (float)e.y - ty, ez = (float)e.z - tz;
-                float r2 = __builtin_fmaf(ex, ex, eps2f);
-                r2 = __builtin_fmaf(ey, ey, r2);
-                r2 = __builtin_fmaf(ez, ez, r2);
-                const float ri = __builtin_amdgcn_rsqf(r2);
-                float sc = ((float)e.w * ri) * (ri * ri);
-                if (GUARD) sc = clamp_finite(sc);
-                fx = __builtin_fmaf(ex, sc, fx);
-                fy = __builtin_fmaf(ey, sc, fy);
-                fz = __builtin_fmaf(ez, sc, fz);
-            }
+            // U entries at a time: their loads and factors in flight together, their terms
+            // added in order
+            auto terms = [&](auto u_const, const Entry* at) {
+                constexpr int U = decltype(u_const)::value;
+                Entry e[U];
+                float ex[U], ey[U], ez[U], sc[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) e[u] = at[u * nslices];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    ex[u] = (float)e[u].x - tx;
+                    ey[u] = (float)e[u].y - ty;
+                    ez[u] = (float)e[u].z - tz;
+                    float r2 = __builtin_fmaf(ex[u], ex[u], eps2f);
+                    r2 = __builtin_fmaf(ey[u], ey[u], r2);
+                    r2 = __builtin_fmaf(ez[u], ez[u], r2);
+                    const float ri = __builtin_amdgcn_rsqf(r2);
+                    sc[u] = ((float)e[u].w * ri) * (ri * ri);
+                    if (GUARD) sc[u] = clamp_finite(sc[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    fx = __builtin_fmaf(ex[u], sc[u], fx);
+                    fy = __builtin_fmaf(ey[u], sc[u], fy);
+                    fz = __builtin_fmaf(ez[u], sc[u], fz);
+                }
+            };
+            if (take == 64 && nslices <= 64 / kEvalUnroll)
+                for (int j = 0; j < 64; j += kEvalUnroll * nslices)
+                    terms(std::integral_constant<int, kEvalUnroll>(), list + slice + j);
+            else
+                for (int j = slice; j < take; j += nslices)
+                    terms(std::integral_constant<int, 1>(), list + j);
             ax += (double)fx; ay += (double)fy; az += (double)fz;
         }
         // the entries after the evaluated ones move to the front (fewer than 64, so the
@@ -1368,11 +1396,16 @@ __device__ __forceinline__ void walk_lists(
         wave_sync();  // every lane has read its popped id
         if (acc_n) list[held + before] = entry_of(rec);
         if (nk > 0) {
-            const int w = top - k + pre;
+            // All eight slots, the last first: what a lane writes past its children lies in
+            // the next lanes' places, which they write in a later instruction (or past the
+            // top, up to 7 ids).  The empty asm keeps the order.
+            int* const w = stack + (top - k + pre);
             const int kk[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                if (q < nk) stack[w + q] = kk[q];
+            for (int q = 7; q >= 0; q--) {
+                w[q] = kk[q];
+                asm volatile("" ::: "memory");
+            }
         }
         held += added;
         listed += added;
@@ -1559,10 +1592,12 @@ __global__ __launch_bounds__(kGroupBlock) void k_walk_group(
     const int* __restrict__ prefixes)
 {
     typedef typename GroupEntry<F64>::T Entry;
-    __shared__ int stacks[kGroupWaves][kStackCap];
+    __shared__ int stacks[kGroupWaves][kStackCap + 8];
     __shared__ Entry lists[kGroupWaves][kListCap];
     __shared__ u64 failss[kGroupWaves][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    // known to be one value per wavefront, so that the walk's counters stay scalar
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int* const stack = stacks[wave];
     Entry* const list = lists[wave];
     u64* const fails = failss[wave];
@@ -1611,7 +1646,8 @@ __global__ __launch_bounds__(kGroupBlock) void k_walk_group(
                  : 0;
     for (int s = 32; s > 0; s >>= 1) eg += __shfl_xor(eg, s);
     const int ext = exponent_f(fmaxf(hix - lox, fmaxf(hiy - loy, hiz - loz)));
-    const bool loose = G >= 16 && cnt > 1 && ext * (cnt - 1) - eg > kLooseLog2 * (cnt - 1);
+    const bool loose = __builtin_amdgcn_readfirstlane(
+        G >= 16 && cnt > 1 && ext * (cnt - 1) - eg > kLooseLog2 * (cnt - 1));
 
     if (!loose) {
         // box centre and half-sizes, the half-sizes widened by a few ulp so that rounding
