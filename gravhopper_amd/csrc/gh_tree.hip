@@ -86,6 +86,7 @@ struct TreeBufs {
     DevBuf hist, bbox_part, box, flags, delta, off, prefix, block_sums, block_counts, packed;
     DevBuf spos;  // (x, y, z, m) of the particles in sorted order
     DevBuf nodes64, nodesw, kids, skip, level, branch, leaf;
+    DevBuf go;  // int: the nodes of the tree built last, 0 where it is not to be walked
     DevBuf wprefix;  // FP32 walk prefixes per block of groups (k_walk_prefix)
     DevBuf tkeys[2], tidx[2];  // Morton order of position targets (tree_force_position)
     long long* readback = nullptr;  // pinned host words: flags[0..1], node count, flags[2]
@@ -95,6 +96,7 @@ struct TreeBufs {
     int words = 0;
     int key_sel = 0;  // which of keys[0]/keys[1] holds the sorted keys
     int full_sorts = 0;  // builds left that sort one-word keys over all bits
+    int no_ahead = 0;    // builds left that wait for their node count
 };
 
 // ------------------------------------------------------------------------------
@@ -792,12 +794,13 @@ __global__ __launch_bounds__(kBlock) void k_scan_local_fill(
 // chunk totals (total to pref[n]); workgroup 0 scans the node counts' (total to off[n]),
 // forms the end-search levels 3 and up, and writes the words the host reads back to its
 // pinned memory: the two flag counts of k_delta, the node count and the long-run count
-// of k_sort_runs.
+// of k_sort_runs.  go: the node count for the kernels behind, or 0 if the tree is not to be
+// walked or has more nodes than cap.
 __global__ __launch_bounds__(kBlock) void k_scan_sums_fill(
     long long* __restrict__ off_sums, DD4* __restrict__ pref_sums, int64_t nb,
     long long* __restrict__ off_total, DD4* __restrict__ pref_total,
     unsigned char* __restrict__ dp, int64_t n, int levels, const int* __restrict__ flags,
-    long long* __restrict__ host)
+    long long cap, int* __restrict__ go, long long* __restrict__ host)
 {
     __shared__ long long shi[kBlock];
     __shared__ DD4 shd[kBlock];
@@ -812,7 +815,11 @@ __global__ __launch_bounds__(kBlock) void k_scan_sums_fill(
         hf[0] = flags[0];
         hf[1] = flags[1];
         host[2] = flags[2];
-        host[1] = nodes;
+        const bool good = (flags[0] | flags[1] | flags[2]) == 0 && nodes > 0 && nodes <= cap;
+        *go = good ? (int)nodes : 0;
+        // the host may be waiting for the count: the flags are there before it
+        __threadfence_system();
+        __hip_atomic_store(&host[1], nodes, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -854,6 +861,7 @@ struct FillArgs {
     signed char* branch;
     int* leaf;  // original particle index, -1 for internal nodes
     int what;   // kFill* bits: which records this build needs
+    const int* go;
 };
 
 constexpr int kFillF64 = 1;   // NodeD + leaf flags (FP64 walk, dump)
@@ -943,6 +951,7 @@ constexpr int kFillBlock = 64;
 __global__ __launch_bounds__(kFillBlock) void k_fill_nodes(FillArgs a, int64_t n)
 {
     __shared__ FillEntry queue[kFillQueue];
+    if (*a.go == 0) return;
     const int lane = threadIdx.x;
     const int64_t i = (int64_t)blockIdx.x * kFillBlock + lane;
     const bool live = i < n;  // every lane takes part in the wave-wide steps
@@ -1444,11 +1453,12 @@ __device__ __forceinline__ int exponent_f(float x)
 // walk starting with them still pops 64 per step); what is left on its stack is deferred
 // too.  A block with a target that is not finite starts its walks at the root.
 __global__ __launch_bounds__(64) void k_walk_prefix(
-    const NodeW* __restrict__ nodes, const int* __restrict__ kids, int n_nodes,
+    const NodeW* __restrict__ nodes, const int* __restrict__ kids, const int* __restrict__ go,
     const double* __restrict__ tgt, const double4* __restrict__ stgt,
     const u32* __restrict__ order, int64_t nt, int G, double inv_theta,
     int* __restrict__ prefixes)
 {
+    const int n_nodes = *go;
     __shared__ int stack[kStackCap];
     __shared__ int list[kPrefixCap];
     __shared__ int defer[kStackCap];
@@ -1586,11 +1596,13 @@ __global__ __launch_bounds__(64) void k_walk_prefix(
 template <bool F64, bool GUARD>
 __global__ __launch_bounds__(kGroupBlock) void k_walk_group(
     const NodeW* __restrict__ nodes, const int* __restrict__ kids, const int* __restrict__ skip,
-    int n_nodes, const double* __restrict__ tgt, const double4* __restrict__ stgt,
-    const u32* __restrict__ order, int64_t nt, int G, float inv_theta, double eps2,
+    const int* __restrict__ go, const double* __restrict__ tgt,
+    const double4* __restrict__ stgt, const u32* __restrict__ order, int64_t nt, int G,
+    float inv_theta, double eps2,
     double* __restrict__ acc, int* __restrict__ counts, int64_t per_xcd,
     const int* __restrict__ prefixes)
 {
+    const int n_nodes = *go;
     typedef typename GroupEntry<F64>::T Entry;
     __shared__ int stacks[kGroupWaves][kStackCap + 8];
     __shared__ Entry lists[kGroupWaves][kListCap];
@@ -1649,6 +1661,7 @@ __global__ __launch_bounds__(kGroupBlock) void k_walk_group(
     const bool loose = __builtin_amdgcn_readfirstlane(
         G >= 16 && cnt > 1 && ext * (cnt - 1) - eg > kLooseLog2 * (cnt - 1));
 
+    if (n_nodes == 0) return;  // nothing is written
     if (!loose) {
         // box centre and half-sizes, the half-sizes widened by a few ulp so that rounding
         // never shrinks the box
@@ -1694,11 +1707,12 @@ __global__ __launch_bounds__(kGroupBlock) void k_walk_group(
 // leaf (skip[n] = n + 1) has none.  The walk reads only the lists of nodes it opens, but
 // leaves' lists are written too: they share cache lines with internal nodes' lists, and
 // a line left partly unwritten costs the walk a fetch of the rest from memory.
-__global__ __launch_bounds__(kBlock) void k_kids(const int* __restrict__ skip, int n_nodes,
+__global__ __launch_bounds__(kBlock) void k_kids(const int* __restrict__ skip,
+                                                 const int* __restrict__ go,
                                                  int* __restrict__ kids)
 {
     const int n = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (n >= n_nodes) return;
+    if (n >= *go) return;
     const int end = skip[n];
     int k[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
     int c = n + 1, q = 0;
@@ -1780,7 +1794,8 @@ struct WalkMask<64> {
 template <int T, bool COUNT, int CAP>
 __global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __restrict__ nodes,
                                                  const int* __restrict__ kids,
-                                                 const int* __restrict__ skip, int n_nodes,
+                                                 const int* __restrict__ skip,
+                                                 const int* __restrict__ go,
                                                  const double* __restrict__ tgt,
                                                  const double4* __restrict__ stgt,
                                                  const u32* __restrict__ order, int64_t nt,
@@ -1788,6 +1803,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __res
                                                  double c_hi, double* __restrict__ acc,
                                                  int* __restrict__ counts, int64_t per_xcd)
 {
+    const int n_nodes = *go;
     typedef typename WalkMask<T>::M Mask;
     constexpr int S = 64 / T;                  // lanes per target
     constexpr int U = T < 4 ? T : 4;           // terms per lane and round (T < 64)
@@ -1960,7 +1976,8 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __res
         ids[0] = 0;
         masks[0] = all;
     }
-    int top = n_nodes > 0 ? 1 : 0;
+    if (n_nodes == 0) return;  // nothing is written
+    int top = 1;
     int sub = 0, sub_end = 0, my_skip = 0;  // the subtree walked one node at a time
     wave_sync();
     for (;;) {
@@ -2208,10 +2225,29 @@ static int run_sort(gh_ctx* c, const double* d_pos, int64_t n, const double* par
     return check_launch(c, "k_run_merge");
 }
 
-// Builds the tree of (d_pos, d_mass) into c->tree.  One host synchronisation reads the
-// node count and the key checks.
+// How many nodes the buffers of earlier builds hold of the records `what`.  kids: which buffer
+// has the children's lists then.
+static int64_t spare_nodes(const TreeBufs* tb, int what, const DevBuf** kids)
+{
+    size_t cap = std::min<size_t>(tb->skip.cap / sizeof(int), 0x7fffffff);
+    if (what & kFillF64)
+        cap = std::min({cap, tb->nodes64.cap / sizeof(NodeD), tb->leaf.cap / sizeof(int)});
+    if (what & kFillW) cap = std::min(cap, tb->nodesw.cap / sizeof(NodeW));
+    *kids = (what & kFillF64) && tb->prefix.cap >= tb->kids.cap ? &tb->prefix : &tb->kids;
+    if (what & kFillKids) cap = std::min(cap, (*kids)->cap / (8 * sizeof(int)));
+    return (int64_t)cap;
+}
+
+// Builds the tree of (d_pos, d_mass) into c->tree.  One wait of the host reads the node count
+// and the key checks: a synchronisation, or, with `pending`, a look that built_ahead takes
+// later.  Then the records are filled into what earlier builds have left, if that holds 2 n + 64
+// nodes or as many as it does hold, and the walk can be queued behind; if it turns out that the
+// tree has more or is not one to be walked, the kernels behind the count do nothing.  (The
+// device stood still meanwhile.  FP64 force, us with the synchronisation and ahead: 66 and 48
+// for 2 particles, 102 and 90 for 2000, 141 and 130 for 10000, 223 and 225 for 40001, 327 and
+// 321 for 70000; FP32 230 and 225 for 40001.)
 static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t n,
-                      double eps, double theta, int what, hipStream_t s)
+                      double eps, double theta, int what, hipStream_t s, bool* pending = nullptr)
 {
     if (!c->tree) c->tree = new TreeBufs();
     TreeBufs* tb = c->tree;
@@ -2232,6 +2268,7 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     unsigned char* const dp = tb->delta.as<unsigned char>();
     const int search_lv = search_levels(n);
     GH_TRY(ensure(c, tb->flags, sizeof(int) * 4));
+    GH_TRY(ensure(c, tb->go, sizeof(int)));
     if (!tb->readback) {
         // coherent, so that the kernel's stores reach the host without any cache flush
         GH_HIP(c, hipHostMalloc((void**)&tb->readback, 4 * sizeof(long long),
@@ -2256,6 +2293,10 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     // next kFullSortBuilds builds of the context sort over all bits.
     constexpr int kFullSortBuilds = 64;
     const int sort_mode = c->tune[GH_TUNE_TREE_SORT];
+    const DevBuf* spare_kids = nullptr;
+    const int64_t spare =
+        pending && tb->no_ahead == 0 ? std::min(spare_nodes(tb, what, &spare_kids), 2 * n + 64) : 0;
+    if (pending && tb->no_ahead > 0) tb->no_ahead--;
     bool all_bits = sort_mode < 0 || (sort_mode == 0 && tb->full_sorts > 0);
     if (sort_mode == 0 && tb->full_sorts > 0) tb->full_sorts--;
     // Keys with `words` words, sort, shared levels, numbering and moments, then one
@@ -2321,6 +2362,7 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
         hipLaunchKernelGGL(k_scan_sums_fill, dim3(2), dim3(kBlock), 0, s,
                            tb->block_counts.as<long long>(), tb->block_sums.as<DD4>(), nb,
                            off + n, pref + n, dp, n, search_lv, tb->flags.as<int>(),
+                           spare > 0 ? (long long)spare : 0x7fffffffll, tb->go.as<int>(),
                            tb->readback_dev);
         GH_TRY(check_launch(c, "k_scan_sums_fill"));
         off_view.local = off;
@@ -2329,6 +2371,12 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
         pref_view.local = pref;
         pref_view.blocks = tb->block_sums.as<DD4>();
         pref_view.n = n;
+        if (spare > 0) {
+            *pending = true;
+            tb->words = words;
+            total = spare;
+            break;
+        }
         GH_HIP(c, hipStreamSynchronize(s));
         if (tb->readback[1] < 0)
             return fail(c, GH_EHIP, "internal: the tree build's readback was not written");
@@ -2354,7 +2402,7 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     const u32* perm = tb->idx[tb->key_sel].as<u32>();
     if (total <= 0 || total >= ((long long)1 << 31))
         return fail(c, GH_EDEPTH, "octree of %lld nodes is out of range", total);
-    tb->n_nodes = total;
+    tb->n_nodes = total;  // or, ahead of the count, the nodes there is room for
     const size_t T = (size_t)total;
     GH_TRY(ensure(c, tb->skip, sizeof(int) * T));
     if (what & (kFillF64 | kFillDump)) {
@@ -2364,7 +2412,8 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     // the FP64 walk's children lists take the place of the moment prefix sums once the fill
     // has read them (they fit unless the tree has more than two nodes per particle)
     const size_t kids_bytes = 8 * sizeof(int) * T;
-    const bool kids_in_prefix = (what & kFillF64) && kids_bytes <= tb->prefix.cap;
+    const bool kids_in_prefix = spare > 0 ? spare_kids == &tb->prefix
+                                          : (what & kFillF64) && kids_bytes <= tb->prefix.cap;
     if ((what & kFillKids) && !kids_in_prefix) GH_TRY(ensure(c, tb->kids, kids_bytes));
     if (what & kFillW) GH_TRY(ensure(c, tb->nodesw, sizeof(NodeW) * T));
     if (what & kFillDump) {
@@ -2387,17 +2436,53 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     fa.branch = tb->branch.as<signed char>();
     fa.leaf = tb->leaf.as<int>();
     fa.what = what;
+    fa.go = tb->go.as<int>();
     hipLaunchKernelGGL(k_fill_nodes, dim3(blocks_for(n, kFillBlock)), dim3(kFillBlock), 0, s, fa,
                        n);
     GH_TRY(check_launch(c, "k_fill_nodes"));
     if (what & kFillKids) {
         int* const kids = kids_in_prefix ? tb->prefix.as<int>() : tb->kids.as<int>();
         hipLaunchKernelGGL(k_kids, dim3(blocks_for(total, kBlock)), dim3(kBlock), 0, s,
-                           tb->skip.as<int>(), (int)total, kids);
+                           tb->skip.as<int>(), tb->go.as<int>(), kids);
         if (what & kFillF64) tb->kids_f64 = kids;
         GH_TRY(check_launch(c, "k_kids"));
     }
     c->last_tree_nodes = total;
+    return 0;
+}
+
+// After a build with a look pending, and the walk behind it: waits for the count.  good: the
+// walk has run; otherwise the build is to be repeated without going ahead.
+static int built_ahead(gh_ctx* c, int64_t n, hipStream_t s, bool* good)
+{
+    TreeBufs* tb = c->tree;
+    *good = false;
+    const long long* count = tb->readback + 1;
+    for (int64_t k = 1; __atomic_load_n(count, __ATOMIC_ACQUIRE) < 0; k++) {
+        __builtin_ia32_pause();
+        if (k % 4096 != 0) continue;
+        // a stream that has come to its end, or to an error, writes no more
+        const hipError_t q = hipStreamQuery(s);
+        if (q == hipErrorNotReady) {
+            (void)hipGetLastError();
+            continue;
+        }
+        GH_HIP(c, q);
+        if (__atomic_load_n(count, __ATOMIC_ACQUIRE) < 0)
+            return fail(c, GH_EHIP, "internal: the tree build's readback was not written");
+    }
+    const int* got = (const int*)tb->readback;
+    *good = got[0] == 0 && got[1] == 0 && tb->readback[2] == 0 && tb->readback[1] > 0 &&
+            tb->readback[1] <= tb->n_nodes;
+    if (*good) {
+        tb->n_nodes = tb->readback[1];
+        c->last_tree_nodes = tb->n_nodes;
+        return 0;
+    }
+    // a tree that grew finds room from the next build on; one of another kind does not
+    constexpr int kNoAheadBuilds = 64;
+    if (got[0] != 0 || got[1] != 0 || tb->readback[2] != 0 || tb->readback[1] > 2 * n + 64)
+        tb->no_ahead = kNoAheadBuilds;
     return 0;
 }
 
@@ -2412,7 +2497,7 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
 #define GH_WALK64(COUNT, CAP)                                                                 \
     hipLaunchKernelGGL((k_walk_f64<T, COUNT, CAP>), grid, dim3(64 * kWalkWaves), 0, s,        \
                        tb->nodes64.as<NodeD>(), tb->kids_f64, tb->skip.as<int>(),             \
-                       (int)tb->n_nodes, tgt, stgt, order, nt, eps * eps, theta, c_lo, c_hi,  \
+                       tb->go.as<int>(), tgt, stgt, order, nt, eps * eps, theta, c_lo, c_hi,  \
                        acc, counts, per)
     // Stack entries: the window of 64 nodes needs more the smaller theta is (at most 484,
     // 833 and 1702 in walks of 64 targets at theta = 0.7, 0.5 and 0.3), and a full stack
@@ -2526,7 +2611,7 @@ static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps,
     const NodeW* nd = tb->nodesw.as<NodeW>();
     const int* kd = tb->kids.as<int>();
     const int* sk = tb->skip.as<int>();
-    const int T = (int)tb->n_nodes;
+    const int* const T = tb->go.as<int>();
     const double eps2 = eps * eps;
     // the walks' shared first steps, per block of kPrefixGroups groups
     int* pf = nullptr;
@@ -2561,9 +2646,17 @@ int tree_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     if (np == 0) return zero_dev(c, d_acc, 3 * nt, s);
     if (precision != GH_FP64 && precision != GH_FP32)
         return fail(c, GH_EARG, "unknown precision %d", precision);
-    GH_TRY(build_tree(c, d_pos, d_mass, np, eps, theta,
-                      kFillKids | (precision == GH_FP64 ? kFillF64 : kFillW), s));
-    return walk(c, self ? d_pos : d_fpos, self, nt, eps, theta, precision, d_acc, nullptr, s);
+    const int what = kFillKids | (precision == GH_FP64 ? kFillF64 : kFillW);
+    const double* tgt = self ? d_pos : d_fpos;
+    bool pending = false, good = false;
+    int rc = build_tree(c, d_pos, d_mass, np, eps, theta, what, s, &pending);
+    if (!rc) rc = walk(c, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
+    if (!pending) return rc;
+    const int seen = built_ahead(c, np, s, &good);  // also after an error: its words are written
+    if (rc || seen) return rc ? rc : seen;
+    if (good) return 0;
+    GH_TRY(build_tree(c, d_pos, d_mass, np, eps, theta, what, s));
+    return walk(c, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
 }
 
 void tree_free(gh_ctx* c)
@@ -2574,7 +2667,7 @@ void tree_free(gh_ctx* c)
                       &tb->bbox_part, &tb->box,   &tb->flags,     &tb->delta,   &tb->off,
                       &tb->prefix,  &tb->spos,      &tb->block_sums, &tb->block_counts,
                       &tb->packed,
-                      &tb->nodes64, &tb->nodesw, &tb->kids,  &tb->wprefix,
+                      &tb->nodes64, &tb->nodesw, &tb->kids,  &tb->go, &tb->wprefix,
                       &tb->skip,    &tb->level,   &tb->branch,    &tb->leaf,    &tb->tkeys[0],
                       &tb->tkeys[1], &tb->tidx[0], &tb->tidx[1]};
     for (DevBuf* b : bufs) release(c, *b);

@@ -470,3 +470,39 @@ def test_fp64_walk_target_not_finite(ctx, oracle):
     assert np.all(np.isnan(got[1000]))
     fine = np.delete(np.arange(5000), [1000, 2000, 3000])
     assert np.all(np.isfinite(got[fine]))
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+def test_walk_queued_before_the_node_count(ctx, prec):
+    # One context's trees of different kinds in turn: more nodes than the last one left room
+    # for, more than 2 per particle, a second key word, equal keys, and trees that are refused.
+    # Each equals what a context that has built nothing before gives.
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(5)
+
+    def close_pairs(n, apart):
+        pos = rng.normal(size=(n // 2, 3))
+        return np.concatenate([pos, pos * (1.0 + apart)])
+
+    trees = [rng.normal(size=(n, 3)) for n in (300, 50, 3000, 2, 3000, 40000)]
+    trees += [close_pairs(2000, 1e-5), close_pairs(2000, 1e-14), rng.normal(size=(2000, 3)),
+              clustered(101000, [70], seed=3)[0], rng.normal(size=(1, 3)), close_pairs(300, 1e-5)]
+    used = _native.Context(0)
+    try:
+        for k, pos in enumerate(trees):
+            mass = rng.uniform(0.5, 1.0, len(pos))
+            fresh = _native.Context(0)
+            want = fresh.tree(pos, mass, 1e-3, 0.7, prec)
+            fresh.close()
+            for again in range(2):
+                assert_bitwise(used.tree(pos, mass, 1e-3, 0.7, prec), want, "tree %d" % k)
+            x = torch.ones((9, 3), dtype=torch.float64, device="cuda")  # all at one place
+            m = torch.ones(9, dtype=torch.float64, device="cuda")
+            acc = torch.full((9, 3), 7.0, dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            with pytest.raises(_native.GravhopError) as e:
+                used.tree_dev(x.data_ptr(), m.data_ptr(), 9, 1e-3, 0.7, prec, acc.data_ptr())
+            assert e.value.code == _native.GH_ECOINCIDENT
+            assert torch.equal(acc, torch.full_like(acc, 7.0))
+    finally:
+        used.close()
