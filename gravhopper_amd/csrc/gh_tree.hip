@@ -1024,7 +1024,7 @@ __global__ __launch_bounds__(kFillBlock) void k_fill_nodes(FillArgs a, int64_t n
 // Scheduling (both walks).  Workgroups are dealt to the 8 XCDs round-robin (workgroup
 // b runs on XCD b mod 8); xcd_block() renumbers them so that XCD x takes the x-th of 8
 // contiguous, Morton-ordered ranges of walk units, and the L2 of XCD x holds the nodes
-// of one region of the tree.  Both walks run two independent wavefronts per workgroup, as
+// of one region of the tree.  The walks run one or two independent wavefronts per workgroup;
 // a CU holds at most 16 workgroups.
 constexpr int kXcds = 8;
 constexpr int64_t kWalkUnits = 4096;  // FP32 walks in flight for small target counts
@@ -1777,8 +1777,6 @@ __device__ __forceinline__ double inv_d15(double d, double c15)
     return __builtin_fma(w, e * __builtin_fma(e, 1.875, c15), w);
 }
 
-// Wavefronts per workgroup, each with a walk of its own.
-constexpr int kWalkWaves = 2;
 constexpr int kWalkDone = (int)0x80000000;  // marks an accepted entry on the stack
 
 template <int T>
@@ -1790,9 +1788,9 @@ struct WalkMask<64> {
     typedef u64 M;
 };
 
-// CAP: stack entries of a walk.
-template <int T, bool COUNT, int CAP>
-__global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __restrict__ nodes,
+// CAP: stack entries of a walk.  W: wavefronts per workgroup, each with a walk of its own.
+template <int T, bool COUNT, int CAP, int W>
+__global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ nodes,
                                                  const int* __restrict__ kids,
                                                  const int* __restrict__ skip,
                                                  const int* __restrict__ go,
@@ -1816,7 +1814,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __res
         Mask masks[CAP], lmask[128];
         int ids[CAP], lid[128];
     };
-    __shared__ Shared shared[kWalkWaves];
+    __shared__ Shared shared[W];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     auto& stage = shared[wave].stage;
@@ -1826,7 +1824,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) void k_walk_f64(const NodeD* __res
     auto& masks = shared[wave].masks;
     auto& ids = shared[wave].ids;
     const int t = lane % T, slice = lane / T;
-    const int64_t first = (xcd_block(per_xcd) * kWalkWaves + wave) * T;
+    const int64_t first = (xcd_block(per_xcd) * W + wave) * T;
     if (first >= nt) return;
     const int cnt = (int)(nt - first < T ? nt - first : T);
     const Mask all = (Mask)(cnt == 64 ? ~0ull : (1ull << cnt) - 1ull);
@@ -2491,28 +2489,37 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
                             const u32* order, int64_t nt, double eps, double theta, double c_lo,
                             double c_hi, double* acc, int* counts, hipStream_t s)
 {
-    const int64_t n_blocks = (nt + (int64_t)T * kWalkWaves - 1) / (T * kWalkWaves);
-    const int64_t per = (n_blocks + kXcds - 1) / kXcds;
-    const dim3 grid((unsigned)(per * kXcds));
-#define GH_WALK64(COUNT, CAP)                                                                 \
-    hipLaunchKernelGGL((k_walk_f64<T, COUNT, CAP>), grid, dim3(64 * kWalkWaves), 0, s,        \
-                       tb->nodes64.as<NodeD>(), tb->kids_f64, tb->skip.as<int>(),             \
-                       tb->go.as<int>(), tgt, stgt, order, nt, eps * eps, theta, c_lo, c_hi,  \
-                       acc, counts, per)
+#define GH_WALK64(COUNT, CAP, W)                                                              \
+    do {                                                                                      \
+        const int64_t per = ((nt + T * W - 1) / (T * W) + kXcds - 1) / kXcds;                 \
+        hipLaunchKernelGGL((k_walk_f64<T, COUNT, CAP, W>), dim3((unsigned)(per * kXcds)),     \
+                           dim3(64 * W), 0, s, tb->nodes64.as<NodeD>(), tb->kids_f64,         \
+                           tb->skip.as<int>(), tb->go.as<int>(), tgt, stgt, order, nt,        \
+                           eps * eps, theta, c_lo, c_hi, acc, counts, per);                   \
+    } while (0)
     // Stack entries: the window of 64 nodes needs more the smaller theta is (at most 484,
     // 833 and 1702 in walks of 64 targets at theta = 0.7, 0.5 and 0.3), and a full stack
     // makes steps small, while LDS for it takes walks off the CU.  N = 2^20, 64 targets,
     // walk ms with 448 / 768 / 1024 entries: theta 0.7 1.88 / 2.17 / -, 0.5 5.74 / 4.60 /
     // 5.05, 0.3 - / 18.1 / 15.6 (one node at a time: 2.33, 5.63, 18.7).
     const int cap = theta >= 0.6 ? 448 : theta >= 0.45 ? 768 : 1024;
+    // One wavefront per workgroup where the 16 workgroups of a CU are as many walks as its
+    // registers hold (64 targets, 448 entries), or where all walks are on the chip at once: a
+    // workgroup of two holds the place of the one that ends first.  Us with two and with one:
+    // N = 2^20 2130 and 2070, 300000 760 and 739, 40001 152 and 148; otherwise more walks wait
+    // for places and two are dealt faster (150000: 426 and 436).
+    constexpr int64_t kWalksResident = 3072;
+    const bool alone = T == 64 || nt <= T * kWalksResident;
     if (counts)
-        GH_WALK64(true, 1024);
+        GH_WALK64(true, 1024, 2);
+    else if (cap == 448 && alone)
+        GH_WALK64(false, 448, 1);
     else if (cap == 448)
-        GH_WALK64(false, 448);
+        GH_WALK64(false, 448, 2);
     else if (cap == 768)
-        GH_WALK64(false, 768);
+        GH_WALK64(false, 768, 2);
     else
-        GH_WALK64(false, 1024);
+        GH_WALK64(false, 1024, 2);
 #undef GH_WALK64
 }
 

@@ -506,3 +506,15 @@ def test_walk_queued_before_the_node_count(ctx, prec):
             assert torch.equal(acc, torch.full_like(acc, 7.0))
     finally:
         used.close()
+
+
+@pytest.mark.parametrize("n", [49152, 49153])  # the most walks of 16 that are resident, and more
+def test_fp64_walk_workgroups(ctx, n):
+    # one and two walks per workgroup: a target's bits do not depend on its neighbours
+    rng = np.random.default_rng(n)
+    pos, mass = rng.normal(size=(n, 3)), rng.uniform(0.5, 1.0, size=n)
+    whole = ctx.tree(pos, mass, 1e-3, 0.7, FP64)
+    for nf in (3072, 3073):
+        pick = rng.permutation(n)[:nf]
+        assert_bitwise(ctx.tree(pos, mass, 1e-3, 0.7, FP64, force_pos=pos[pick]), whole[pick],
+                       "%d targets" % nf)
