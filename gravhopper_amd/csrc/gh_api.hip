@@ -432,7 +432,9 @@ static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t n
     if (np == 0 || nsteps == 0) return 0;
     const int64_t n3 = 3 * np;
     const bool ahead = algorithm == GH_DIRECT;
-    if (ahead && nsteps >= 4) {
+    // the runs that replayed graphs: these end drained and are refused under capture
+    const bool drain = ahead && nsteps >= 4 && !c->timing && c->tune[GH_TUNE_RUN_GRAPH] >= 0;
+    if (drain) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         GH_HIP(c, hipStreamIsCapturing(s, &cap));
         if (cap != hipStreamCaptureStatusNone)
@@ -470,7 +472,7 @@ static int run_steps(gh_ctx* c, double* x, double* v, const double* m, int64_t n
     // would have to wait for it on the device, and there the switch takes 115 us longer (16
     // steps of 3000 particles in FP32 on three streams in turn: 672 us a run, 745 without
     // this; on one stream 672 and 632).
-    if (ahead && nsteps >= 4) GH_HIP(c, hipStreamSynchronize(s));
+    if (drain) GH_HIP(c, hipStreamSynchronize(s));
     return 0;
 }
 

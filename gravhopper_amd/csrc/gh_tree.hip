@@ -2292,8 +2292,14 @@ static int build_tree(gh_ctx* c, const double* d_pos, const double* d_mass, int6
     constexpr int kFullSortBuilds = 64;
     const int sort_mode = c->tune[GH_TUNE_TREE_SORT];
     const DevBuf* spare_kids = nullptr;
-    const int64_t spare =
+    int64_t spare =
         pending && tb->no_ahead == 0 ? std::min(spare_nodes(tb, what, &spare_kids), 2 * n + 64) : 0;
+    if (spare > 0) {
+        // a captured build never writes its count: the synchronisation refuses the capture
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        GH_HIP(c, hipStreamIsCapturing(s, &cap));
+        if (cap != hipStreamCaptureStatusNone) spare = 0;
+    }
     if (pending && tb->no_ahead > 0) tb->no_ahead--;
     bool all_bits = sort_mode < 0 || (sort_mode == 0 && tb->full_sorts > 0);
     if (sort_mode == 0 && tb->full_sorts > 0) tb->full_sorts--;

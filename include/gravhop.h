@@ -223,8 +223,9 @@ int gh_timing_read(gh_ctx *ctx, int kernel_class, double *total_ms, int64_t *lau
  *   GH_TUNE_WALK_GROUP   FP32 tree walk: 0 automatic, 1/2/4/8/16/32/64 targets per
  *                        group (the targets that share one opening test and interaction
  *                        list)
- *   GH_TUNE_RUN_GRAPH    accepted, without effect (a run's kernels are launched one by one,
- *                        which was faster than replaying graphs at every size)
+ *   GH_TUNE_RUN_GRAPH    direct-sum gh_run / gh_run_dev of 4 steps and more (their kernels
+ *                        are launched one by one): 0 the call waits for the run, -1 it
+ *                        returns once the steps are queued
  *   GH_TUNE_WALK_F64EVAL FP32 tree walk: 1 evaluates the same interaction lists in FP64
  *                        (a check of the FP32 arithmetic), 0 FP32
  *   GH_TUNE_DIRECT_F64_TPW  FP64 direct sum: 0 automatic; v > 0 the wavefronts of a
