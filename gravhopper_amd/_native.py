@@ -63,6 +63,8 @@ SIGNATURES = {
                           ctypes.POINTER(_I64)], _I),
     "gh_ensemble_destroy": ([_P], None),
     "gh_adjoint_forward": ([_P, _P, _P, _P, _I64, _D, _D, _I, _I64, _I64, _P, _P], _I),
+    "gh_adjoint_forward_kept": ([_P, _P, _P, _P, _I64, _D, _D, _I, _I64, _P, _P, _P, _P], _I),
+    "gh_adjoint_backward_kept": ([_P, _P, _P, _P, _I64, _D, _D, _I64, _P, _P, _P, _P], _I),
     "gh_adjoint_backward": ([_P, _P, _P, _I64, _D, _D, _I, _I64, _I64, _P, _P, _P, _P], _I),
     "gh_timing_read": ([_P, _I, ctypes.POINTER(_D), ctypes.POINTER(_I64)], _I),
     "gh_energy": ([_P, _P, _P, _P, _I64, _D, _P, _P, _P], _I),

@@ -6,9 +6,10 @@ initial positions, velocities and masses, through a hand-written adjoint.
 
 x0, v0: (n,3) float64 CUDA tensors (kpc, km/s); m: (n,) float64 (Msun); dt in Myr,
 eps in kpc.  The forward is the drift-kick-drift of Simulation.run (gh_adjoint_forward,
-the same kernels as gh_run) and keeps (x, v) every `checkpoint_every` steps; backward
-re-runs each segment from its checkpoint and applies the reverse step with the
-vector-Jacobian products through the softened tidal tensor (gh_adjoint_backward).
+the same kernels as gh_run).  A run whose half-step positions take at most KEEP_BYTES keeps
+them (gh_adjoint_forward_kept); a longer one keeps (x, v) every `checkpoint_every` steps and
+backward re-runs each segment from its checkpoint.  Backward applies the reverse step with
+the vector-Jacobian products through the softened tidal tensor (gh_adjoint_backward).
 Both are ordered with torch's current stream.
 """
 import ctypes
@@ -17,6 +18,9 @@ import math
 import torch
 
 from . import _native
+
+# A thousandth of the card's memory per run in the graph: 28 bytes per particle and step.
+KEEP_BYTES = 256 << 20
 
 
 def _p(t):
@@ -53,13 +57,34 @@ class DirectLeapfrog(torch.autograd.Function):
         v = v0.detach().to(torch.float64).contiguous().clone()
         mm = m.detach().to(torch.float64).contiguous()
         nseg = max(1, math.ceil(nsteps / every))
+        if n > 0 and nsteps >= 0 and every > 0 and 28 * n * nsteps <= KEEP_BYTES:
+            return DirectLeapfrog._forward_kept(ctx, lib, x, v, mm, float(dt), float(eps),
+                                                int(precision), int(nsteps))
         ckpt = torch.empty((nseg, 2, n, 3), dtype=torch.float64, device=x.device)
         with _OnTorchStream(lib, x.device) as stream:
             lib.check(lib.lib.gh_adjoint_forward(lib.handle, _p(x), _p(v), _p(mm), n, float(dt),
                                                  float(eps), int(precision), int(nsteps),
                                                  int(every), _p(ckpt), stream))
         ctx.save_for_backward(mm, ckpt)
+        ctx.kept = False
         ctx.params = (float(dt), float(eps), int(precision), int(nsteps), int(every))
+        return x, v
+
+    @staticmethod
+    def _forward_kept(ctx, lib, x, v, mm, dt, eps, precision, nsteps):
+        n = x.shape[0]
+        half = torch.empty((nsteps, n, 3), dtype=torch.float64, device=x.device)
+        order = torch.empty((nsteps, n), dtype=torch.int32, device=x.device)
+        ordered = ctypes.c_int(0)
+        with _OnTorchStream(lib, x.device) as stream:
+            lib.check(lib.lib.gh_adjoint_forward_kept(lib.handle, _p(x), _p(v), _p(mm), n, dt,
+                                                      eps, precision, nsteps, _p(half),
+                                                      _p(order), ctypes.byref(ordered), stream))
+        ctx.save_for_backward(mm, half)
+        ctx.kept = True
+        # indices, so not among the saved tensors: a hook may round what it packs
+        ctx.order = order if ordered.value else None
+        ctx.params = (dt, eps, precision, nsteps, 0)
         return x, v
 
     @staticmethod
@@ -75,9 +100,15 @@ class DirectLeapfrog(torch.autograd.Function):
         lm = torch.empty(n, dtype=torch.float64, device=dev)
         lib = _native.default_context()
         with _OnTorchStream(lib, dev) as stream:
-            lib.check(lib.lib.gh_adjoint_backward(lib.handle, _p(ckpt), _p(mm), n, dt, eps,
-                                                  precision, nsteps, every, _p(lx), _p(lv),
-                                                  _p(lm), stream))
+            if ctx.kept:
+                order = None if ctx.order is None else _p(ctx.order)
+                lib.check(lib.lib.gh_adjoint_backward_kept(lib.handle, _p(ckpt), order, _p(mm),
+                                                           n, dt, eps, nsteps, _p(lx), _p(lv),
+                                                           _p(lm), stream))
+            else:
+                lib.check(lib.lib.gh_adjoint_backward(lib.handle, _p(ckpt), _p(mm), n, dt, eps,
+                                                      precision, nsteps, every, _p(lx), _p(lv),
+                                                      _p(lm), stream))
         return lx, lv, lm, None, None, None, None, None
 
 

@@ -182,6 +182,19 @@ int gh_adjoint_backward(gh_ctx *ctx, const double *d_ckpt, const double *d_m, in
                         double dt, double eps, int precision, int64_t nsteps, int64_t every,
                         double *d_lx, double *d_lv, double *d_lm, void *stream);
 
+/* The same gradient without re-running any step, for runs whose half-step positions fit in
+ * memory.  gh_adjoint_forward_kept writes those of every step to d_half (nsteps x (n,3)
+ * doubles) and, where `ordered` and d_order are given and every force evaluation made one,
+ * the spatial orders to d_order (nsteps x n) with *ordered = 1.  gh_adjoint_backward_kept
+ * reads them; d_order is what the forward pass wrote, or NULL where *ordered was 0.  Same
+ * results as the checkpointed pair, bit for bit. */
+int gh_adjoint_forward_kept(gh_ctx *ctx, double *d_x, double *d_v, const double *d_m, int64_t n,
+                            double dt, double eps, int precision, int64_t nsteps,
+                            double *d_half, int32_t *d_order, int *ordered, void *stream);
+int gh_adjoint_backward_kept(gh_ctx *ctx, const double *d_half, const int32_t *d_order,
+                             const double *d_m, int64_t n, double dt, double eps, int64_t nsteps,
+                             double *d_lx, double *d_lv, double *d_lm, void *stream);
+
 /* Batched ensembles (no reference counterpart): n_sims independent direct-sum
  * simulations of uneven size, each advanced by the leapfrog of gh_run with its own
  * softening and time step, all with FP32 pair forces (pair-once kernel, `ipt`
