@@ -69,8 +69,8 @@ __device__ __forceinline__ void lds_barrier()
 template <bool SELF, int P, int K>
 __global__ __launch_bounds__((P + 1) * 64) void k_direct_f64_relay(
     const double* __restrict__ pos, const double* __restrict__ mass, int64_t np,
-    const double* __restrict__ tgt, int64_t nt, double eps2, double* __restrict__ acc,
-    StepUpdate up)
+    const double* __restrict__ tgt, int64_t from, int64_t nt, double eps2,
+    double* __restrict__ acc, StepUpdate up)
 {
     constexpr int T = P * K, NS = 3 * T, CH = 128;
     static_assert(NS <= 64, "one lane per sum");
@@ -80,7 +80,7 @@ __global__ __launch_bounds__((P + 1) * 64) void k_direct_f64_relay(
     __shared__ double2 terms[2][CH / 2][ROW];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t i0 = (int64_t)blockIdx.x * T;
+    const int64_t i0 = from + (int64_t)blockIdx.x * T;
     // chunks are taken in pairs; one past the last adds zeros
     const int64_t chunks = (np + 2 * CH - 1) / (2 * CH) * 2;
     if (wave == P) {
@@ -222,7 +222,8 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
                                                             const double* __restrict__ mass,
                                                             int64_t np,
                                                             const double* __restrict__ tgt,
-                                                            int64_t nt, double eps2,
+                                                            int64_t from, int64_t nt,
+                                                            double eps2,
                                                             double* __restrict__ acc)
 {
     constexpr int T = 64 / H, G = H * C, TURNS = 64 / G;
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int t = lane % T, h = lane / T;
-    const int64_t i0 = (int64_t)blockIdx.x * T;
+    const int64_t i0 = from + (int64_t)blockIdx.x * T;
     const int64_t i = i0 + t < nt ? i0 + t : nt - 1;  // past nt: computed, not stored
     const double xi = tgt[3 * i], yi = tgt[3 * i + 1], zi = tgt[3 * i + 2];
     if (threadIdx.x < T) sums[0][t] = sums[1][t] = sums[2][t] = 0.0;
@@ -339,13 +340,13 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
 // as many targets per workgroup as give each CU one workgroup.  Beyond, k_direct_f64_ring:
 // the issue rate of the terms bounds it, and the shape decides how evenly the wavefronts
 // fill the CUs: two lanes per target (32 targets per workgroup) until 64 targets per
-// workgroup give every CU one, eight wavefronts per workgroup until there are two
-// workgroups per CU.  Measured on Plummer spheres, us per evaluation (the best of the other
+// workgroup give half of the CUs one, eight wavefronts per workgroup until there are two
+// workgroups per CU (whole rounds apart, f64_whole_rounds).  Measured on Plummer spheres, us per evaluation (the best of the other
 // family beside it; "before" is one or few targets per wavefront, with the compiler's
 // division and square root):
 //   N        500  1000  2000  4000  6000 | 8000  12000  16384  20000  32768  65536  100003  262144
 //   relay    7.3  10.0  17.9  41.2  80.7 |  141    289    529    817   2063
-//   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   91367
+//   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   90900
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
 // 3001 targets of 65536 sources: 468 (before 1300); 200 of 100000: 393 (1062).
 enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
@@ -366,9 +367,28 @@ static F64Shape f64_shape(const gh_ctx* c, int64_t nt)
             if (t <= has) return {has, F64Ring::none};
         return {16, F64Ring::none};
     }
-    const bool one_lane = tune ? tune >= 64 : (nt > 8192 && nt <= 16384) || nt > 24576;
+    const bool one_lane = tune ? tune >= 64 : nt > 8192;
     if (nt <= 16384) return {0, one_lane ? F64Ring::w8_h1 : F64Ring::w8_h2};
     return {0, one_lane ? F64Ring::w4_h1 : F64Ring::w4_h2};
+}
+
+// Targets 0 .. whole - 1 that take a launch of their own, 0 for none.  A workgroup of 64 targets
+// on each of the 256 CUs is a round of 16384.  The few workgroups beyond whole rounds run last on
+// a CU each that they do not fill (N = 100003: 27 after 1536 held the launch for 1.2 rounds), so
+// they go to the shape for as many targets, which spreads them over the chip.  Up to half a round
+// that always gains; beyond, a launch of them costs more than it takes off the other.  Us with
+// one launch and with two: N = 16500 684 and 538, 24000 928 and 916, 34000 2331 and 1787, 40768
+// 2778 and 2429, 50000 4650 and 3629, 73536 8479 and 7605, 100003 16483 and 14040, 200000 57417
+// and 54251; not taken: 24884 1228 and 1263, 41768 2903 and 2897, 74536 8491 and 8663.  One round
+// is taken by eight wavefronts per workgroup, more by four (16500 538 and 602; 100003 14444 and
+// 14040).
+constexpr int64_t kF64Round = 256 * 64;
+static int64_t f64_whole_rounds(const gh_ctx* c, int64_t nt)
+{
+    const int64_t rest = nt % kF64Round;
+    return c->tune[GH_TUNE_DIRECT_F64_TPW] == 0 && nt > kF64Round && rest <= kF64Round / 2
+               ? nt - rest
+               : 0;
 }
 
 // ------------------------------------------------------------------------------
@@ -956,33 +976,66 @@ F32Shape pick_shape(gh_ctx* c, int64_t nt, int64_t np_pad)
     return sh;
 }
 
+// The FP64 sums of targets from .. nt - 1 (self: of particles, from among all np).
+struct F64Call {
+    bool self;
+    const double *pos, *mass;
+    int64_t np;
+    const double* tgt;
+    int64_t from, nt;
+    double eps2;
+    double* acc;
+    StepUpdate up;  // relay only
+    hipStream_t s;
+};
+
 template <int P, int K>
-void launch_relay(bool self, const double* pos, const double* mass, int64_t np, const double* tgt,
-                  int64_t nt, double eps2, double* acc, const StepUpdate& up, hipStream_t s)
+void launch_relay(const F64Call& q)
 {
-    const dim3 grid((unsigned)((nt + P * K - 1) / (P * K))), block((P + 1) * 64);
-    if (self)
-        hipLaunchKernelGGL((k_direct_f64_relay<true, P, K>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc, up);
+    const dim3 grid((unsigned)((q.nt - q.from + P * K - 1) / (P * K))), block((P + 1) * 64);
+    if (q.self)
+        hipLaunchKernelGGL((k_direct_f64_relay<true, P, K>), grid, block, 0, q.s, q.pos, q.mass,
+                           q.np, q.tgt, q.from, q.nt, q.eps2, q.acc, q.up);
     else
-        hipLaunchKernelGGL((k_direct_f64_relay<false, P, K>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc, up);
+        hipLaunchKernelGGL((k_direct_f64_relay<false, P, K>), grid, block, 0, q.s, q.pos, q.mass,
+                           q.np, q.tgt, q.from, q.nt, q.eps2, q.acc, q.up);
 }
 
 template <int W, int H>
-void launch_ring(bool self, const double* pos, const double* mass, int64_t np, const double* tgt,
-                 int64_t nt, double eps2, double* acc, hipStream_t s)
+void launch_ring(const F64Call& q)
 {
     // 16 sources per lane and turn: passing the turn on takes about 390 cycles, the terms
     // of 8 sources 1900 (N = 16384: 433 us with 8, 398 with 16)
     constexpr int C = 16;
-    const dim3 grid(blocks_for(nt, 64 / H)), block(64 * W);
-    if (self)
-        hipLaunchKernelGGL((k_direct_f64_ring<true, W, C, H>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc);
+    const dim3 grid(blocks_for(q.nt - q.from, 64 / H)), block(64 * W);
+    if (q.self)
+        hipLaunchKernelGGL((k_direct_f64_ring<true, W, C, H>), grid, block, 0, q.s, q.pos,
+                           q.mass, q.np, q.tgt, q.from, q.nt, q.eps2, q.acc);
     else
-        hipLaunchKernelGGL((k_direct_f64_ring<false, W, C, H>), grid, block, 0, s, pos, mass, np,
-                           tgt, nt, eps2, acc);
+        hipLaunchKernelGGL((k_direct_f64_ring<false, W, C, H>), grid, block, 0, q.s, q.pos,
+                           q.mass, q.np, q.tgt, q.from, q.nt, q.eps2, q.acc);
+}
+
+int launch_f64(gh_ctx* c, const F64Shape& sh, const F64Call& q)
+{
+    switch (sh.ring) {
+    case F64Ring::none:
+        switch (sh.targets) {
+        case 1: launch_relay<1, 1>(q); break;
+        case 3: launch_relay<3, 1>(q); break;
+        case 4: launch_relay<4, 1>(q); break;
+        case 6: launch_relay<3, 2>(q); break;
+        case 8: launch_relay<4, 2>(q); break;
+        case 12: launch_relay<6, 2>(q); break;
+        default: launch_relay<8, 2>(q); break;
+        }
+        return check_launch(c, "k_direct_f64_relay");
+    case F64Ring::w8_h2: launch_ring<8, 2>(q); break;
+    case F64Ring::w8_h1: launch_ring<8, 1>(q); break;
+    case F64Ring::w4_h2: launch_ring<4, 2>(q); break;
+    default: launch_ring<4, 1>(q); break;
+    }
+    return check_launch(c, "k_direct_f64_ring");
 }
 
 template <int IPT>
@@ -1237,37 +1290,23 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     }
     if (precision == GH_FP64) {
         const double eps2 = eps * eps;
-        const F64Shape sh = f64_shape(c, nt);
-        if (sh.ring == F64Ring::none) {
-            TimedScope ts(c, s, GH_T_DIRECT_F64);
-            const bool fuse = up && up->xh_next != up->xh;  // other workgroups read xh
-            const StepUpdate u = fuse ? *up : StepUpdate();
-            if (fuse) *updated = true;
-            switch (sh.targets) {
-            case 1: launch_relay<1, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            case 3: launch_relay<3, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            case 4: launch_relay<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            case 6: launch_relay<3, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            case 8: launch_relay<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            case 12: launch_relay<6, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            default: launch_relay<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, u, s); break;
-            }
-            return check_launch(c, "k_direct_f64_relay");
-        }
+        F64Call q = {self, d_pos, d_mass, np, tgt, 0, nt, eps2, d_acc, StepUpdate(), s};
+        F64Shape sh = f64_shape(c, nt);
         TimedScope ts(c, s, GH_T_DIRECT_F64);
-        switch (sh.ring) {
-        case F64Ring::w8_h2:
-            launch_ring<8, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
-            break;
-        case F64Ring::w8_h1:
-            launch_ring<8, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
-            break;
-        case F64Ring::w4_h2:
-            launch_ring<4, 2>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s);
-            break;
-        default: launch_ring<4, 1>(self, d_pos, d_mass, np, tgt, nt, eps2, d_acc, s); break;
+        if (sh.ring == F64Ring::none) {
+            if (up && up->xh_next != up->xh) {  // other workgroups read xh
+                q.up = *up;
+                *updated = true;
+            }
+        } else if (const int64_t whole = f64_whole_rounds(c, nt)) {
+            q.nt = whole;
+            GH_TRY(launch_f64(c, {0, whole == kF64Round ? F64Ring::w8_h1 : F64Ring::w4_h1}, q));
+            if (whole == nt) return 0;
+            q.from = whole;
+            q.nt = nt;
+            sh = f64_shape(c, nt - whole);
         }
-        return check_launch(c, "k_direct_f64_ring");
+        return launch_f64(c, sh, q);
     }
     if (precision != GH_FP32) return fail(c, GH_EARG, "unknown precision %d", precision);
     const int sym = self ? sym_ipt(c, np) : 0;

@@ -336,3 +336,21 @@ def test_fp32_pair_once_leaves_padding_out(ctx, ipt, n):
         ctx.set_tuning(_native.TUNE_DIRECT_SELF, 0)
     for e in (rel_err(got, ref), rel_err(band, ref)):
         assert np.median(e) <= FP32_MEDIAN and np.percentile(e, 99) <= FP32_P99
+
+
+# around one round of 16384 targets, half a round beyond it, two rounds, and the tails' shapes
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 16684, 23000, 24576, 24577, 32768, 32769, 34000])
+def test_fp64_whole_rounds_apart(ctx, oracle, n):
+    """FP64 sums whose last targets have a launch of their own: the bits of one launch for all
+    (64 targets per workgroup), and of the oracle at targets away from the sources."""
+    ic = workloads.plummer(n, seed=n)
+    got = ctx.direct(ic["pos"], ic["mass"], 2e-5, FP64)
+    few = workloads.plummer(300, seed=1)
+    at = ctx.direct(few["pos"], few["mass"], 2e-5, FP64, force_pos=ic["pos"])
+    ctx.set_tuning(_native.TUNE_DIRECT_F64_TPW, 64)
+    try:
+        want = ctx.direct(ic["pos"], ic["mass"], 2e-5, FP64)
+    finally:
+        ctx.set_tuning(_native.TUNE_DIRECT_F64_TPW, 0)
+    assert_bitwise(got, want, "self field")
+    assert_bitwise(at, oracle.direct_position(few["pos"], few["mass"], ic["pos"], 2e-5), "targets")
