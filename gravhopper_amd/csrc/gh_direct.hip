@@ -337,7 +337,9 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
 
 // Kernel shape for the FP64 sums.  Up to kF64RelayMax targets k_direct_f64_relay: the chain
 // of ordered additions is what bounds it, so the fewest wavefronts that keep up with it, and
-// as many targets per workgroup as give each CU one workgroup.  Beyond, k_direct_f64_ring:
+// as many targets per workgroup as give each CU one workgroup, or two of 6 or 9 where that is as
+// many as fit (us for 2100, 3001, 5000 targets of 65536 sources with 12 in six wavefronts 469, 472,
+// 767, with 9 418, 636, 968, with 6 445, 455, 767, with 20 696, 699, 704).  Beyond, k_direct_f64_ring:
 // the issue rate of the terms bounds it, and the shape decides how evenly the wavefronts
 // fill the CUs: two lanes per target (32 targets per workgroup) until 64 targets per
 // workgroup give half of the CUs one, eight wavefronts per workgroup until there are two
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
 //   relay    7.3  10.0  17.9  41.2  80.7 |  141    289    529    817   2063
 //   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   90900
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
-// 3001 targets of 65536 sources: 468 (before 1300); 200 of 100000: 393 (1062).
+// 3001 targets of 65536 sources: 455 (before 1300); 200 of 100000: 393 (1062).
 enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
 struct F64Shape {
     int targets;  // relay: per workgroup
@@ -361,11 +363,11 @@ static F64Shape f64_shape(const gh_ctx* c, int64_t nt)
     if (relay) {
         int64_t t = tune < 0 ? -(int64_t)tune : 0;
         if (tune == 0)
-            t = nt <= 256 ? 1 : nt <= 768 ? 3 : nt <= 1024 ? 4 : nt <= 2048 ? 8
-                : nt <= 3072 ? 12 : nt <= 4096 ? 16 : 6;
-        for (int has : {1, 3, 4, 6, 8, 12})
+            t = nt <= 256 ? 1 : nt <= 768 ? 3 : nt <= 1024 ? 4 : nt <= 2048 ? 8 : nt <= 2304 ? 9
+                : nt <= 3072 ? 6 : nt <= 4096 ? 16 : nt <= 4608 ? 9 : nt <= 5120 ? 20 : 6;
+        for (int has : {1, 3, 4, 6, 8, 9, 16})
             if (t <= has) return {has, F64Ring::none};
-        return {16, F64Ring::none};
+        return {20, F64Ring::none};
     }
     const bool one_lane = tune ? tune >= 64 : nt > 8192;
     if (nt <= 16384) return {0, one_lane ? F64Ring::w8_h1 : F64Ring::w8_h2};
@@ -1026,8 +1028,9 @@ int launch_f64(gh_ctx* c, const F64Shape& sh, const F64Call& q)
         case 4: launch_relay<4, 1>(q); break;
         case 6: launch_relay<3, 2>(q); break;
         case 8: launch_relay<4, 2>(q); break;
-        case 12: launch_relay<6, 2>(q); break;
-        default: launch_relay<8, 2>(q); break;
+        case 9: launch_relay<3, 3>(q); break;
+        case 16: launch_relay<8, 2>(q); break;
+        default: launch_relay<4, 5>(q); break;
         }
         return check_launch(c, "k_direct_f64_relay");
     case F64Ring::w8_h2: launch_ring<8, 2>(q); break;

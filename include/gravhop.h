@@ -245,7 +245,7 @@ int gh_timing_read(gh_ctx *ctx, int kernel_class, double *total_ms, int64_t *lau
  *                        workgroup add their terms to its targets' sums in turns, with
  *                        64 targets per workgroup for v >= 64 and 32 below; -v < 0 one
  *                        wavefront adds the others' terms, with v targets per workgroup
- *                        (rounded up to 1, 3, 4, 6, 8, 12 or 16)
+ *                        (rounded up to 1, 3, 4, 6, 8, 9, 16 or 20)
  *   GH_TUNE_ALLOC_LIMIT_MB  cap, in MiB, on the device memory the context's arenas may
  *                        hold (0: no cap); a call that would exceed it fails with
  *                        GH_ENOMEM and leaves the context usable

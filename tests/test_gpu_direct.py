@@ -354,3 +354,17 @@ def test_fp64_whole_rounds_apart(ctx, oracle, n):
         ctx.set_tuning(_native.TUNE_DIRECT_F64_TPW, 0)
     assert_bitwise(got, want, "self field")
     assert_bitwise(at, oracle.direct_position(few["pos"], few["mass"], ic["pos"], 2e-5), "targets")
+
+
+@pytest.mark.parametrize("n", [2048, 2049, 2304, 2305, 3072, 3073, 4096, 4097, 4608, 4609, 5119,
+                               5121, 6500])
+def test_fp64_relay_shapes(ctx, oracle, n):
+    """Each side of the sizes at which the targets per workgroup change; chunks of 128 sources
+    with a remainder of 1."""
+    few = workloads.plummer(513, seed=2)
+    at = workloads.plummer(n, seed=n)["pos"]
+    got = ctx.direct(few["pos"], few["mass"], 2e-5, FP64, force_pos=at)
+    assert_bitwise(got, oracle.direct_position(few["pos"], few["mass"], at, 2e-5), "targets")
+    ic = workloads.plummer(n, seed=n)
+    own = ctx.direct(ic["pos"], ic["mass"], 2e-5, FP64)[-40:]
+    assert_bitwise(own, oracle.direct(ic["pos"], ic["mass"], 2e-5)[-40:], "self field")
