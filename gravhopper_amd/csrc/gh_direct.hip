@@ -335,20 +335,20 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
     }
 }
 
-// Kernel shape for the FP64 sums.  Up to kF64RelayMax targets k_direct_f64_relay: the chain
-// of ordered additions is what bounds it, so the fewest wavefronts that keep up with it, and
-// as many targets per workgroup as give each CU one workgroup, or two of 6 or 9 where that is as
-// many as fit (us for 2100, 3001, 5000 targets of 65536 sources with 12 in six wavefronts 469, 472,
-// 767, with 9 418, 636, 968, with 6 445, 455, 767, with 20 696, 699, 704).  Beyond, k_direct_f64_ring:
-// the issue rate of the terms bounds it, and the shape decides how evenly the wavefronts
-// fill the CUs: two lanes per target (32 targets per workgroup) until 64 targets per
-// workgroup give half of the CUs one, eight wavefronts per workgroup until there are two
-// workgroups per CU (whole rounds apart, f64_whole_rounds).  Measured on Plummer spheres, us per evaluation (the best of the other
-// family beside it; "before" is one or few targets per wavefront, with the compiler's
+// Kernel shape for the FP64 sums.  Up to kF64RelayMax targets k_direct_f64_relay: the chain of
+// ordered additions is what bounds it, so the fewest wavefronts that keep up with it, and as many
+// targets per workgroup as give each CU one workgroup, or two of 6 or 9 where that is as many as
+// fit (us for 2100, 3001, 5000 targets of 65536 sources with 12 in six wavefronts 469, 472, 767,
+// with 9 418, 636, 968, with 6 445, 455, 767, with 20 696, 699, 704).  Beyond, k_direct_f64_ring:
+// the issue rate of the terms bounds it, and the shape decides how evenly the wavefronts fill the
+// CUs: two lanes per target (32 targets per workgroup) until 64 targets per workgroup give half of
+// the CUs one, eight wavefronts per workgroup until there are two workgroups per CU, and whole
+// rounds apart (f64_whole_rounds).  Measured on Plummer spheres, us per evaluation (the best of the
+// other family beside it; "before" is one or few targets per wavefront, with the compiler's
 // division and square root):
 //   N        500  1000  2000  4000  6000 | 8000  12000  16384  20000  32768  65536  100003  262144
 //   relay    7.3  10.0  17.9  41.2  80.7 |  141    289    529    817   2063
-//   ring                      60.6  86.0 |  111    293    398    731   1509   5817   16382   90900
+//   ring                      60.6  86.0 |  111    293    398    723   1509   5817   14040   90900
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
 // 3001 targets of 65536 sources: 455 (before 1300); 200 of 100000: 393 (1062).
 enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
