@@ -21,6 +21,7 @@
 
 #include "gh_internal.h"
 #include "gh_pairf64.h"
+#include "gh_turn.h"
 
 namespace gh {
 
@@ -298,8 +299,7 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
             }
             // every wavefront of the workgroup is resident and passes each of its turns on,
             // so this ends
-            while (__hip_atomic_load(&turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != g)
-                __builtin_amdgcn_s_sleep(1);
+            while (!turn_is(&turn, g)) __builtin_amdgcn_s_sleep(1);
             __builtin_amdgcn_s_setprio(3);
             double f0 = sums[0][t], f1 = sums[1][t], f2 = sums[2][t];
 #pragma unroll
@@ -321,9 +321,7 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
                 sums[1][t] = f1;
                 sums[2][t] = f2;
             }
-            asm volatile("" ::: "memory");
-            if (lane == 0)
-                __hip_atomic_store(&turn, g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            turn_pass(&turn, g + 1);
             __builtin_amdgcn_s_setprio(0);
         }
     }
