@@ -1765,6 +1765,9 @@ __global__ __launch_bounds__(kBlock) void k_kids(const int* __restrict__ skip,
 // once into LDS, and one lane per sum adds them in order (+0.0 where the target did not
 // accept the entry, which changes no sum, as none is ever -0).
 //
+// A node without mass has no centre of mass (0 / 0, as in the reference): its acceptors get NaN
+// (`hit`), and its record in the list is 0, as 0 times NaN would reach the others' sums.
+//
 // A step pops only as many entries as leave room for what goes back; where that is none,
 // the top entry's subtree is walked one node at a time with the skip pointers.
 // COUNT: counts receives the accepted-node count per target.
@@ -1889,6 +1892,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
     // their monopoles; evaluate() uses them a traversal step later, which hides the loads.
     int have = 0;
     Mask m_have = 0;
+    Mask hit = 0;  // targets that have accepted a node without a centre of mass
     double2 q0, q1;
     auto fetch = [&]() {
         have = held < 64 ? held : 64;
@@ -1908,8 +1912,6 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
     };
     auto evaluate_as = [&](auto guarded) {
         constexpr bool guard = decltype(guarded)::value;
-        stage[lane] = make_double4(q0.x, q0.y, q1.x, q1.y);
-        wave_sync();
         if constexpr (T == 64) {
             for (int e0 = 0; e0 < have; e0 += 4) {
                 double dx[4], dy[4], dz[4], mi[4];
@@ -1962,8 +1964,14 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
         have = 0;
         wave_sync();
     };
-    // a separation of 0 counts as 0; only without softening is there one
+    // (a separation of 0 counts as 0; only without softening is there one)
     auto evaluate = [&]() {
+        const bool none = !(isfinite(q0.x) && isfinite(q0.y) && isfinite(q1.x));
+        for (u64 left = __ballot(none && lane < have); left != 0; left &= left - 1)
+            hit |= lane_value(m_have, (int)__builtin_ctzll(left));
+        stage[lane] = none || lane >= have ? make_double4(0.0, 0.0, 0.0, 0.0)
+                                           : make_double4(q0.x, q0.y, q1.x, q1.y);
+        wave_sync();
         if (eps2 > 0.0)
             evaluate_as(std::false_type());
         else
@@ -1978,14 +1986,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
     int top = 1;
     int sub = 0, sub_end = 0, my_skip = 0;  // the subtree walked one node at a time
     wave_sync();
-    for (;;) {
-        const bool walked = top == 0 && sub == sub_end;
-        if (held >= 64 || (walked && held > 0)) fetch();
-        if (walked) {
-            if (have == 0) break;
-            evaluate();
-            continue;
-        }
+    auto step = [&]() {
         if (sub != sub_end) {
             const NodeD nd = nodes[sub];
             const bool active = my_skip <= sub;
@@ -2004,8 +2005,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
                 wave_sync();
             }
             sub = opens ? sub + 1 : sk;
-            if (have > 0) evaluate();
-            continue;
+            return;
         }
         int n_pop = top < 64 ? top : 64;
         bool popped = lane < n_pop;
@@ -2076,8 +2076,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
                 my_skip = (masks[top - 1] & own) != 0 ? 0 : 0x7fffffff;  // waits below it
                 top -= 1;
                 wave_sync();
-                if (have > 0) evaluate();
-                continue;
+                return;
             }
             total = __builtin_amdgcn_readlane(before, n_pop);
             popped = lane < n_pop;
@@ -2108,9 +2107,19 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
         top = new_top;
         held += n_out;
         wave_sync();
+    };
+    for (;;) {
+        const bool walked = top == 0 && sub == sub_end;
+        if (held >= 64 || (walked && held > 0)) fetch();
+        if (!walked)
+            step();
+        else if (have == 0)
+            break;
         if (have > 0) evaluate();
     }
+    const double nan = __builtin_nan("");
     if constexpr (T == 64) {
+        if ((hit & own) != 0) ax = ay = az = nan;
         if (lane < cnt) {
             acc[3 * ti] = ax;
             acc[3 * ti + 1] = ay;
@@ -2120,6 +2129,7 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
     } else {
         if (lane < 3 * cnt) {
             const int64_t kt = first + lane / 3;
+            if ((hit >> (lane / 3) & 1) != 0) f = nan;
             acc[3 * (order ? (int64_t)order[kt] : kt) + lane % 3] = f;
         }
         if (COUNT) {

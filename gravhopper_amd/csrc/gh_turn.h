@@ -1,7 +1,7 @@
 // Turns of several wavefronts at data they share: whoever holds turn g waits for it, works on
 // the data and passes g + 1 on.  The wait is an acquire and the pass a release, so each turn's
-// writes come before the next turn's reads by the memory model.  Plain C++ without hipcc: tests/host/turn_check.cpp
-// runs the same turns on threads under ThreadSanitizer.
+// writes come before the next turn's reads by the memory model.  Plain C++ without hipcc:
+// tests/host/turn_check.cpp runs the same turns on threads under ThreadSanitizer.
 #pragma once
 
 namespace gh {

@@ -518,3 +518,40 @@ def test_fp64_walk_workgroups(ctx, n):
         pick = rng.permutation(n)[:nf]
         assert_bitwise(ctx.tree(pos, mass, 1e-3, 0.7, FP64, force_pos=pos[pick]), whole[pick],
                        "%d targets" % nf)
+
+
+def massless(case):
+    rng = np.random.default_rng(11)
+    if case == "pair":
+        pos = np.array([[0.0, 0, 0], [1.0, 0.5, 0.2]])
+    elif case == "octants":
+        pos = rng.uniform(0.5, 1.0, (8, 3)) * (2 * np.indices((2, 2, 2)).reshape(3, 8).T - 1)
+    elif case == "close pair":
+        pos = np.array([[0.0, 0, 0], [1e-3, 0, 0], [1.0, 0.5, 0.2]])
+    else:  # a massless pair among others, whose node few, some or most of them accept
+        pos = rng.normal(size=(int(case), 3))
+        pos[[1, 4]] = [[4.0, 4.0, 4.0], [4.5, 4.0, 4.0]]
+        mass = rng.uniform(0.5, 2.0, len(pos))
+        mass[[1, 4]] = 0.0
+        return pos, mass
+    return pos, np.zeros(len(pos))
+
+
+# targets per walk: 1 of them up to 2560 particles, 2, 4, 16 and 64
+@pytest.mark.parametrize("eps", [0.01, 0.0])
+@pytest.mark.parametrize("case", ["pair", "octants", "close pair", "6", "2000", "3000", "6000",
+                                  "30000", "200002"])
+def test_fp64_walk_massless(ctx, oracle, case, eps):
+    """A node without mass has no centre of mass (0/0, as in the reference): who accepts it
+    gets NaN, and nobody else does."""
+    pos, mass = massless(case)
+    some = np.unique(np.concatenate([np.arange(min(len(pos), 9)),
+                                     np.random.default_rng(1).integers(0, len(pos), 300)]))
+    for theta in (0.7, 0.15, 0.05):
+        want = oracle.tree(pos, mass, eps, theta, force_pos=pos[some])
+        got = ctx.tree(pos, mass, eps, theta, FP64)[some]
+        own = ctx.tree(pos, mass, eps, theta, FP64, force_pos=pos[some])
+        assert np.array_equal(np.isnan(got), np.isnan(want)), theta
+        np.testing.assert_allclose(got, want, rtol=1e-10, err_msg="theta=%g" % theta,
+                                   atol=1e-10 * np.nanmax(np.abs(want), initial=0.0))
+        assert np.array_equal(got, own, equal_nan=True), theta
