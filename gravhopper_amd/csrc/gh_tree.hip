@@ -1850,9 +1850,15 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
         loz = fmin(loz, __shfl_xor(loz, o)), hiz = fmax(hiz, __shfl_xor(hiz, o));
     }
     double bcx = 0.5 * (lox + hix), bcy = 0.5 * (loy + hiy), bcz = 0.5 * (loz + hiz);
-    const double bhx = 0.5 * (hix - lox), bhy = 0.5 * (hiy - loy), bhz = 0.5 * (hiz - loz);
+    // Per axis, a node at distance g from the box's centre is at least kNear g - bh and at most
+    // kFar g + bh from every target: bh is how far targets are from the centre as it is rounded
+    // (far from the origin an ulp of a coordinate can be more than the box's size), and the
+    // 2^-50 cover the rounding by 2^-53 of g, of that distance and of what is formed of them.
+    constexpr double kNear = 1.0 - 0x1p-50, kFar = 1.0 + 0x1p-50;
+    const double bhx = kFar * fmax(hix - bcx, bcx - lox), bhy = kFar * fmax(hiy - bcy, bcy - loy),
+                 bhz = kFar * fmax(hiz - bcz, bcz - loz);
     if (__ballot(!(isfinite(x) && isfinite(y) && isfinite(z))) != 0) bcx = __builtin_nan("");
-    // bounds on the box's squared distances; the margin covers their rounding
+    // bounds on the squared distances; the margin covers the rounding of the squares and sums
     const double box_hi = c_hi * (1.0 + 1e-12), box_lo = c_lo * (1.0 - 1e-12);
 
     double ax = 0.0, ay = 0.0, az = 0.0;  // T = 64: the lane's target's sums
@@ -2029,8 +2035,11 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
         const bool leaf = __double_as_longlong(c2s.y) < 0;
         const double s2 = c2s.y * c2s.y;
         const double gx = fabs(c01.x - bcx), gy = fabs(c01.y - bcy), gz = fabs(c2s.x - bcz);
-        const double nx = fmax(0.0, gx - bhx), ny = fmax(0.0, gy - bhy), nz = fmax(0.0, gz - bhz);
-        const double fx = gx + bhx, fy = gy + bhy, fz = gz + bhz;
+        const double nx = fmax(0.0, __builtin_fma(gx, kNear, -bhx)),
+                     ny = fmax(0.0, __builtin_fma(gy, kNear, -bhy)),
+                     nz = fmax(0.0, __builtin_fma(gz, kNear, -bhz));
+        const double fx = __builtin_fma(gx, kFar, bhx), fy = __builtin_fma(gy, kFar, bhy),
+                     fz = __builtin_fma(gz, kFar, bhz);
         // (gx is NaN for a box that decides nothing, and nx then 0: hence the third test)
         const bool clear = leaf || (nx * nx + ny * ny + nz * nz > s2 * box_hi && gx == gx);
         const bool inside = fx * fx + fy * fy + fz * fz < s2 * box_lo;

@@ -555,3 +555,23 @@ def test_fp64_walk_massless(ctx, oracle, case, eps):
         np.testing.assert_allclose(got, want, rtol=1e-10, err_msg="theta=%g" % theta,
                                    atol=1e-10 * np.nanmax(np.abs(want), initial=0.0))
         assert np.array_equal(got, own, equal_nan=True), theta
+
+
+# 2, 16 and 64 targets per walk
+@pytest.mark.parametrize("side", [16, 32, 64])
+def test_fp64_walk_ties_far_from_the_origin(ctx, oracle, side):
+    """A lattice 8 kpc from the origin, and theta where targets lie on the threshold of the
+    nodes of eight: what a walk decides for all of its targets at once is what the reference
+    decides for each, to the last ulp of their coordinates."""
+    h = 1e-6
+    pos = np.array([8.1, -8.2, 0.3]) + h * np.indices((side,) * 3).reshape(3, -1).T
+    mass = np.random.default_rng(side).uniform(0.5, 2.0, len(pos))
+    some = np.random.default_rng(side).permutation(len(pos))[:3000]
+    for d2 in (0.5 ** 2 + 0.5 ** 2 + 3.5 ** 2, 0.5 ** 2 + 1.5 ** 2 + 2.5 ** 2, 3 * 2.5 ** 2):
+        theta = 2.0 / np.sqrt(d2)
+        _, want = oracle.tree(pos, mass, h, theta, force_pos=pos[some], count=True)
+        _, count = ctx.tree_interactions(pos, mass, h, theta)
+        own, alone = ctx.tree_interactions(pos, mass, h, theta, force_pos=pos[some])
+        assert np.array_equal(alone, want), d2
+        assert np.array_equal(count[some], want), d2
+        assert_bitwise(ctx.tree(pos, mass, h, theta, FP64)[some], own, "d2=%g" % d2)
