@@ -1,15 +1,16 @@
 """Differentiable leapfrog: gradients of a direct-sum N-body run with respect to the
 initial positions, velocities and masses, through a hand-written adjoint.
 
-    x, v = leapfrog(x0, v0, m, dt, eps, nsteps, checkpoint_every=20)
+    x, v = leapfrog(x0, v0, m, dt, eps, nsteps)
     loss = ((x - target) ** 2).sum(-1).mean(); loss.backward()
 
 x0, v0: (n,3) float64 CUDA tensors (kpc, km/s); m: (n,) float64 (Msun); dt in Myr,
 eps in kpc.  The forward is the drift-kick-drift of Simulation.run (gh_adjoint_forward,
-the same kernels as gh_run).  A run whose half-step positions take at most KEEP_BYTES keeps
-them (gh_adjoint_forward_kept); a longer one keeps (x, v) every `checkpoint_every` steps and
-backward re-runs each segment from its checkpoint.  Backward applies the reverse step with
-the vector-Jacobian products through the softened tidal tensor (gh_adjoint_backward).
+the same kernels as gh_run).  With `checkpoint_every` it keeps (x, v) that often, 48 bytes per
+particle, and backward re-runs each segment from its checkpoint.  Without, a run whose half-step
+positions take at most KEEP_BYTES keeps those (gh_adjoint_forward_kept) and nothing is re-run;
+a longer one has a checkpoint every 20 steps.  Backward applies the reverse step with the
+vector-Jacobian products through the softened tidal tensor (gh_adjoint_backward).
 Both are ordered with torch's current stream.
 """
 import ctypes
@@ -21,6 +22,7 @@ from . import _native
 
 # A thousandth of the card's memory per run in the graph: 28 bytes per particle and step.
 KEEP_BYTES = 256 << 20
+CHECKPOINT_EVERY = 20  # where the caller names no interval and the run is longer
 
 
 def _p(t):
@@ -56,10 +58,12 @@ class DirectLeapfrog(torch.autograd.Function):
         x = x0.detach().to(torch.float64).contiguous().clone()
         v = v0.detach().to(torch.float64).contiguous().clone()
         mm = m.detach().to(torch.float64).contiguous()
-        nseg = max(1, math.ceil(nsteps / every))
-        if n > 0 and nsteps >= 0 and every > 0 and 28 * n * nsteps <= KEEP_BYTES:
+        if every is None and n > 0 and nsteps >= 0 and 28 * n * nsteps <= KEEP_BYTES:
             return DirectLeapfrog._forward_kept(ctx, lib, x, v, mm, float(dt), float(eps),
                                                 int(precision), int(nsteps))
+        if every is None:
+            every = CHECKPOINT_EVERY
+        nseg = max(1, math.ceil(nsteps / every))
         ckpt = torch.empty((nseg, 2, n, 3), dtype=torch.float64, device=x.device)
         with _OnTorchStream(lib, x.device) as stream:
             lib.check(lib.lib.gh_adjoint_forward(lib.handle, _p(x), _p(v), _p(mm), n, float(dt),
@@ -112,7 +116,9 @@ class DirectLeapfrog(torch.autograd.Function):
         return lx, lv, lm, None, None, None, None, None
 
 
-def leapfrog(x0, v0, m, dt, eps, nsteps, checkpoint_every=20, precision="fp32"):
-    """Final (x, v) after nsteps drift-kick-drift steps, differentiable in x0, v0, m."""
-    return DirectLeapfrog.apply(x0, v0, m, dt, eps, int(nsteps), int(checkpoint_every),
+def leapfrog(x0, v0, m, dt, eps, nsteps, checkpoint_every=None, precision="fp32"):
+    """Final (x, v) after nsteps drift-kick-drift steps, differentiable in x0, v0, m.
+    checkpoint_every: the steps between checkpoints (None: KEEP_BYTES decides, see above)."""
+    every = None if checkpoint_every is None else int(checkpoint_every)
+    return DirectLeapfrog.apply(x0, v0, m, dt, eps, int(nsteps), every,
                                 _native.PRECISIONS[precision])

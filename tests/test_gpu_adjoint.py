@@ -155,3 +155,45 @@ def test_adjoint_kept_equals_checkpointed(ctx, monkeypatch, precision, n, steps)
                 grads(True, torch.autograd.graph.save_on_cpu())):
         for a, b in zip(got, want):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision,n,steps", [("fp32", 1, 3), ("fp32", 2, 4), ("fp32", 700, 0),
+                                               ("fp32", 700, 1), ("fp32", 3001, 7),
+                                               ("fp32", 17000, 5), ("fp64", 1, 2),
+                                               ("fp64", 300, 7), ("fp64", 7000, 3)])
+def test_adjoint_default_equals_checkpointed(ctx, precision, n, steps):
+    # without an interval a short run keeps its half-step positions: the bits of a run with
+    # checkpoints, also from a second backward pass and through hooks on the saved tensors
+    from gravhopper_amd import autograd
+    ic, _ = config(n, 700)
+    w = torch.tensor(np.random.default_rng(2).normal(size=(n, 3)), device="cuda")
+
+    def grads(passes=1, hooks=None, **kw):
+        s = [torch.tensor(ic[k], device="cuda", requires_grad=True) for k in ("pos", "vel", "mass")]
+        with hooks or torch.enable_grad():
+            x, v = autograd.leapfrog(*s, 0.005, 5e-5, steps, precision=precision, **kw)
+        loss = (x * w).sum() + 1e-3 * v.square().sum()
+        for k in range(passes):
+            g = torch.autograd.grad(loss, s, retain_graph=k + 1 < passes)
+        return [t.detach().cpu().numpy() for t in (x, v) + g]
+
+    want = grads(checkpoint_every=3)
+    for got in (grads(), grads(passes=3), grads(hooks=torch.autograd.graph.save_on_cpu()),
+                grads(checkpoint_every=1), grads(checkpoint_every=40)):
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("every", [None, 7, 20])
+def test_adjoint_memory_between_the_passes(ctx, every):
+    # a run with checkpoints holds them (and the masses) for backward and no more than them
+    from gravhopper_amd import autograd
+    n, steps = 20000, 40
+    ic, _ = config(n, 800)
+    s = [torch.tensor(ic[k], device="cuda", requires_grad=True) for k in ("pos", "vel", "mass")]
+    kw = {} if every is None else {"checkpoint_every": every}
+    before = torch.cuda.memory_allocated()
+    x, v = autograd.leapfrog(*s, 0.005, 5e-5, steps, **kw)
+    held = torch.cuda.memory_allocated() - before - 48 * n  # x and v
+    per_particle = 28 * steps if every is None else 48 * -(-steps // every)
+    assert per_particle * n <= held <= (per_particle + 8) * n + (1 << 16)
