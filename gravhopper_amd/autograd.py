@@ -29,6 +29,11 @@ def _p(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def _graph_is_kept():
+    """Whether the backward pass that is running leaves its graph for another one."""
+    return torch._C._autograd._get_current_graph_task_keep_graph()
+
+
 class _OnTorchStream:
     """Orders library work with torch's current stream.  A real stream is handed to the
     library; torch's legacy default stream (handle 0) cannot be, since 0 selects the
@@ -109,6 +114,8 @@ class DirectLeapfrog(torch.autograd.Function):
                 lib.check(lib.lib.gh_adjoint_backward_kept(lib.handle, _p(ckpt), order, _p(mm),
                                                            n, dt, eps, nsteps, _p(lx), _p(lv),
                                                            _p(lm), stream))
+                if not _graph_is_kept():
+                    ctx.order = None  # with the saved tensors
             else:
                 lib.check(lib.lib.gh_adjoint_backward(lib.handle, _p(ckpt), _p(mm), n, dt, eps,
                                                       precision, nsteps, every, _p(lx), _p(lv),

@@ -186,7 +186,8 @@ def test_adjoint_default_equals_checkpointed(ctx, precision, n, steps):
 
 @pytest.mark.parametrize("every", [None, 7, 20])
 def test_adjoint_memory_between_the_passes(ctx, every):
-    # a run with checkpoints holds them (and the masses) for backward and no more than them
+    # A run with checkpoints holds them (and the masses) for backward and no more than them;
+    # whatever a run holds is given back with the graph, also while its results live on.
     from gravhopper_amd import autograd
     n, steps = 20000, 40
     ic, _ = config(n, 800)
@@ -197,3 +198,9 @@ def test_adjoint_memory_between_the_passes(ctx, every):
     held = torch.cuda.memory_allocated() - before - 48 * n  # x and v
     per_particle = 28 * steps if every is None else 48 * -(-steps // every)
     assert per_particle * n <= held <= (per_particle + 8) * n + (1 << 16)
+    g = torch.autograd.grad(x.sum(), s, retain_graph=True)
+    del g
+    assert torch.cuda.memory_allocated() - before - 48 * n <= held + (1 << 16)
+    g = torch.autograd.grad(x.sum(), s)
+    del g
+    assert torch.cuda.memory_allocated() - before <= 48 * n + (1 << 16)
