@@ -1972,11 +1972,15 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
     };
     // (a separation of 0 counts as 0; only without softening is there one)
     auto evaluate = [&]() {
-        const bool none = !(isfinite(q0.x) && isfinite(q0.y) && isfinite(q1.x));
-        for (u64 left = __ballot(none && lane < have); left != 0; left &= left - 1)
-            hit |= lane_value(m_have, (int)__builtin_ctzll(left));
-        stage[lane] = none || lane >= have ? make_double4(0.0, 0.0, 0.0, 0.0)
-                                           : make_double4(q0.x, q0.y, q1.x, q1.y);
+        double4 record = make_double4(q0.x, q0.y, q1.x, q1.y);
+        // (a sum is finite if its terms are and do not overflow: few lists take the branch)
+        if (__ballot(lane >= have || !isfinite(q0.x + q0.y + q1.x)) != 0) {
+            const bool none = !(isfinite(q0.x) && isfinite(q0.y) && isfinite(q1.x));
+            for (u64 left = __ballot(none && lane < have); left != 0; left &= left - 1)
+                hit |= lane_value(m_have, (int)__builtin_ctzll(left));
+            if (none || lane >= have) record = make_double4(0.0, 0.0, 0.0, 0.0);
+        }
+        stage[lane] = record;
         wave_sync();
         if (eps2 > 0.0)
             evaluate_as(std::false_type());
