@@ -1780,6 +1780,7 @@ __device__ __forceinline__ double inv_d15(double d, double c15)
     return __builtin_fma(w, e * __builtin_fma(e, 1.875, c15), w);
 }
 
+constexpr int kDeepCap = 1536;  // stack entries of a walk that fills 1024
 constexpr int kWalkDone = (int)0x80000000;  // marks an accepted entry on the stack
 
 template <int T>
@@ -2018,6 +2019,9 @@ __global__ __launch_bounds__(64 * W) void k_walk_f64(const NodeD* __restrict__ n
             return;
         }
         int n_pop = top < 64 ? top : 64;
+        // Nearly full: as many as there is room for.  More would be tested for nothing, and with
+        // 64 targets a test that the box leaves open is a pass of its own.
+        if (T == 64) n_pop = min(n_pop, max(1, CAP - top));
         bool popped = lane < n_pop;
         const int entry = popped ? ids[top - 1 - lane] : kWalkDone;
         const Mask m = popped ? masks[top - 1 - lane] : (Mask)0;
@@ -2532,6 +2536,14 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
     // walk ms with 448 / 768 / 1024 entries: theta 0.7 1.88 / 2.17 / -, 0.5 5.74 / 4.60 /
     // 5.05, 0.3 - / 18.1 / 15.6 (one node at a time: 2.33, 5.63, 18.7).
     const int cap = theta >= 0.6 ? 448 : theta >= 0.45 ? 768 : 1024;
+    // Where walks are long and their targets far apart, 1024 entries stay full, and a step takes
+    // a node or two: the forces of more than 100000 particles at theta < 0.35, and 64 position
+    // targets a walk at theta < 0.4.  Ms with 1024 and with kDeepCap (and one node at a time):
+    // N = 130000 theta 0.2 11.9 / 8.5, 200000 0.3 8.2 / 4.6 (5.9), 0.2 16.1 / 13.6 (14.4),
+    // 500000 0.3 10.9 / 8.9 (10.3), 1500000 0.3 30.3 / 25.8 (26.5); 400001 targets among 10^6
+    // particles 0.3 26.8 / 14.4 (19.8), 10^6 on a line 11.5 / 12.3 (15.8); 2^20 0.3 16.9 / 17.6
+    // (18.9); not taken: N = 100000 0.3 2.30 / 2.42, 500000 0.4 4.43 / 4.72.
+    const bool deep = stgt ? theta < 0.35 && nt > 100000 : T == 64 && theta < 0.4;
     // One wavefront per workgroup where the 16 workgroups of a CU are as many walks as its
     // registers hold (64 targets, 448 entries), or where all walks are on the chip at once: a
     // workgroup of two holds the place of the one that ends first.  Us with two and with one:
@@ -2539,9 +2551,16 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
     // for places and two are dealt faster (150000: 426 and 436).
     constexpr int64_t kWalksResident = 3072;
     const bool alone = T == 64 || nt <= T * kWalksResident;
-    if (counts)
+    if (counts) {
         GH_WALK64(true, 1024, 2);
-    else if (cap == 448 && alone)
+        return;
+    }
+    if constexpr (T >= 16)
+        if (deep) {
+            GH_WALK64(false, kDeepCap, 1);
+            return;
+        }
+    if (cap == 448 && alone)
         GH_WALK64(false, 448, 1);
     else if (cap == 448)
         GH_WALK64(false, 448, 2);
@@ -2608,7 +2627,7 @@ static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps,
         int T = 1;
         if (self) {
             while (T < 16 && nt > T * kWalks64) T *= 2;
-            if (nt > 200000) T = 64;
+            if (nt > (theta < 0.35 ? 150000 : 200000)) T = 64;
         } else if (order) {
             while (T < 16 && nt > T * 20000) T *= 2;
             if (nt > 400000) T = 64;

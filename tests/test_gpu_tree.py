@@ -575,3 +575,18 @@ def test_fp64_walk_ties_far_from_the_origin(ctx, oracle, side):
         assert np.array_equal(alone, want), d2
         assert np.array_equal(count[some], want), d2
         assert_bitwise(ctx.tree(pos, mass, h, theta, FP64)[some], own, "d2=%g" % d2)
+
+
+# the deepest walks (16 and 64 targets, 1536 stack entries) and the sizes before them
+@pytest.mark.parametrize("n,nf,theta", [(100000, 0, 0.3), (100001, 0, 0.3), (150000, 0, 0.2),
+                                        (150001, 0, 0.2), (150001, 0, 0.349), (150001, 0, 0.35),
+                                        (3000, 400001, 0.3), (3000, 400001, 0.4)])
+def test_fp64_walk_deep_same_bits(ctx, n, nf, theta):
+    rng = np.random.default_rng(n)
+    pos = rng.standard_cauchy(size=(n, 3))
+    mass = rng.uniform(0.5, 2.0, size=n)
+    fpos = rng.standard_cauchy(size=(nf, 3)) if nf else None
+    tgt = pos if fpos is None else fpos
+    some = rng.permutation(len(tgt))[:400]
+    full = ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=fpos)
+    assert_bitwise(full[some], ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=tgt[some]))
