@@ -18,6 +18,7 @@
 //  spatially sorted particles (gh_frames.hip), so their accuracy does not depend on
 //  where the system sits; non-compact groups take double-single instances.
 #include <cmath>
+#include <type_traits>
 
 #include "gh_internal.h"
 #include "gh_pairf64.h"
@@ -333,6 +334,47 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
     }
 }
 
+// The field of few sources: one target per lane, the sources one after the other and four factors
+// at a time.
+__global__ __launch_bounds__(kBlock) void k_direct_f64_few(const double* __restrict__ pos,
+                                                           const double* __restrict__ mass, int np,
+                                                           const double* __restrict__ tgt,
+                                                           int64_t nt, double eps2,
+                                                           double* __restrict__ acc)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nt) return;
+    const double xi = tgt[3 * i], yi = tgt[3 * i + 1], zi = tgt[3 * i + 2];
+    double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+    auto add = [&](auto count, int j) {
+        constexpr int U = decltype(count)::value;
+        double dx[U], dy[U], dz[U], d[U], inv[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            dx[u] = pos[3 * (j + u)] - xi;
+            dy[u] = pos[3 * (j + u) + 1] - yi;
+            dz[u] = pos[3 * (j + u) + 2] - zi;
+            double d2 = dx[u] * dx[u];
+            d2 = d2 + dy[u] * dy[u];
+            d2 = d2 + dz[u] * dz[u];
+            d[u] = d2 + eps2;
+        }
+        pair_factors<false, U>(d, inv);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            f0 = f0 + mass[j + u] * dx[u] * inv[u];
+            f1 = f1 + mass[j + u] * dy[u] * inv[u];
+            f2 = f2 + mass[j + u] * dz[u] * inv[u];
+        }
+    };
+    int j = 0;
+    for (; j + 4 <= np; j += 4) add(std::integral_constant<int, 4>(), j);
+    for (; j < np; j++) add(std::integral_constant<int, 1>(), j);
+    acc[3 * i] = f0;
+    acc[3 * i + 1] = f1;
+    acc[3 * i + 2] = f2;
+}
+
 // Kernel shape for the FP64 sums.  Up to kF64RelayMax targets k_direct_f64_relay: the chain of
 // ordered additions is what bounds it, so the fewest wavefronts that keep up with it, and as many
 // targets per workgroup as give each CU one workgroup, or two of 6 or 9 where that is as many as
@@ -349,15 +391,19 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
 //   ring                      60.6  86.0 |  111    293    398    723   1509   5817   14040   90900
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
 // 3001 targets of 65536 sources: 455 (before 1300); 200 of 100000: 393 (1062).
+// Few sources are a chunk of the relay at most, whose many small workgroups then cost more than
+// the ring's: 50 sources at 3000 and 6500 targets 7.5 and 9.9 us, with the ring 7.1 and 7.1; 100
+// at 3000 7.5 and 7.8.
+constexpr int64_t kF64FewSources = 64;
 enum class F64Ring { none, w8_h2, w8_h1, w4_h2, w4_h1 };
 struct F64Shape {
     int targets;  // relay: per workgroup
     F64Ring ring;
 };
-static F64Shape f64_shape(const gh_ctx* c, int64_t nt)
+static F64Shape f64_shape(const gh_ctx* c, int64_t np, int64_t nt)
 {
     const int tune = c->tune[GH_TUNE_DIRECT_F64_TPW];
-    const bool relay = tune < 0 || (tune == 0 && nt <= kF64RelayMax);
+    const bool relay = tune < 0 || (tune == 0 && nt <= (np <= kF64FewSources ? 2048 : kF64RelayMax));
     if (relay) {
         int64_t t = tune < 0 ? -(int64_t)tune : 0;
         if (tune == 0)
@@ -389,6 +435,16 @@ static int64_t f64_whole_rounds(const gh_ctx* c, int64_t nt)
     return c->tune[GH_TUNE_DIRECT_F64_TPW] == 0 && nt > kF64Round && rest <= kF64Round / 2
                ? nt - rest
                : 0;
+}
+
+// The field of few sources at many targets, which k_direct_f64_few takes: there a workgroup of the
+// ring has hardly a turn for each of its wavefronts, and starting and ending it is what counts.
+// Us with the ring and with it: 1 source at 100000 targets 16.5 and 7.6, at 10^6 97 and 12; 16
+// at 20000 11.8 and 7.6; 64 at 50000 14.1 and 13.7; 200 at 200000 70.5 and 71.5, at 10^6 308 and
+// 263; 1000 at 10^6 1369 and 1311; not taken: 32 at 30000 8.4 and 9.3, 500 at 200000 153 and 175.
+static bool f64_few(const gh_ctx* c, int64_t np, int64_t nt)
+{
+    return c->tune[GH_TUNE_DIRECT_F64_TPW] == 0 && nt > kF64Round && np <= nt / 1000;
 }
 
 // ------------------------------------------------------------------------------
@@ -1292,8 +1348,13 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     if (precision == GH_FP64) {
         const double eps2 = eps * eps;
         F64Call q = {self, d_pos, d_mass, np, tgt, 0, nt, eps2, d_acc, StepUpdate(), s};
-        F64Shape sh = f64_shape(c, nt);
+        F64Shape sh = f64_shape(c, np, nt);
         TimedScope ts(c, s, GH_T_DIRECT_F64);
+        if (f64_few(c, np, nt)) {
+            hipLaunchKernelGGL(k_direct_f64_few, dim3(blocks_for(nt, kBlock)), dim3(kBlock), 0, s,
+                               d_pos, d_mass, (int)np, tgt, nt, eps2, d_acc);
+            return check_launch(c, "k_direct_f64_few");
+        }
         if (sh.ring == F64Ring::none) {
             if (up && up->xh_next != up->xh) {  // other workgroups read xh
                 q.up = *up;
@@ -1305,7 +1366,7 @@ int direct_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
             if (whole == nt) return 0;
             q.from = whole;
             q.nt = nt;
-            sh = f64_shape(c, nt - whole);
+            sh = f64_shape(c, np, nt - whole);
         }
         return launch_f64(c, sh, q);
     }

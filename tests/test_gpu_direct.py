@@ -368,3 +368,18 @@ def test_fp64_relay_shapes(ctx, oracle, n):
     ic = workloads.plummer(n, seed=n)
     own = ctx.direct(ic["pos"], ic["mass"], 2e-5, FP64)[-40:]
     assert_bitwise(own, oracle.direct(ic["pos"], ic["mass"], 2e-5)[-40:], "self field")
+
+
+# the field of few sources: the relay, the ring and one target per lane meet at these counts
+@pytest.mark.parametrize("n,nf", [(n, nf) for nf in (2048, 2049, 6500, 16384, 16385)
+                                  for n in (1, 3, 16, 17, 64, 65)] +
+                         [(n, 70001) for n in (1, 4, 5, 70, 71)] + [(1, 262144), (262, 262145)])
+def test_fp64_field_of_few_sources_bitwise(ctx, oracle, n, nf):
+    rng = np.random.default_rng(nf + n)
+    fpos = rng.standard_cauchy(size=(nf, 3))
+    pos = rng.standard_cauchy(size=(n, 3))
+    pos[:n // 2] = fpos[nf - n // 2:] if n > 1 else pos[:0]  # coincident pairs
+    mass = rng.uniform(0.1, 3.0, size=n)
+    for eps in (0.0, 1e-3):
+        assert_bitwise(ctx.direct(pos, mass, eps, FP64, force_pos=fpos),
+                       oracle.direct_position(pos, mass, fpos, eps), "eps=%g" % eps)
