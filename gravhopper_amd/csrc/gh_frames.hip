@@ -111,13 +111,14 @@ __device__ __forceinline__ void points_box(const double* __restrict__ pos, int n
 
 // Run b of RUN points (RUN of the kRunThreads threads hold one each; all of them form the box
 // of the run's segment): the keys in order, with the points they belong to.  Places behind the
-// segment's points are filled with the largest key.
+// segment's points are filled with the largest key.  single: no segment has more than one run,
+// whose order is then the segment's and goes to perm at once.
 template <int RUN>
 __global__ __launch_bounds__(kRunThreads) void k_rank_runs(
     const double* __restrict__ pos, int64_t n_all, const int* __restrict__ seg,
     const int64_t* __restrict__ seg_start, const int64_t* __restrict__ seg_count,
     u32* __restrict__ keys, u32* __restrict__ from, u32* __restrict__ perm,
-    int* __restrict__ nflag)
+    int* __restrict__ nflag, bool single)
 {
     const int t = threadIdx.x;
     const int g = seg ? seg[blockIdx.x] : 0;
@@ -140,27 +141,43 @@ __global__ __launch_bounds__(kRunThreads) void k_rank_runs(
         perm[base + t] = idx;
     }
     const int at = sort_run<RUN>(key, idx, act);
-    if (act) {
+    if (act && single) {
+        if ((int64_t)idx - first < n) perm[base + at] = idx;
+    } else if (act) {
         keys[base + at] = key;
         from[base + at] = idx;
     }
 }
 
 // The order of n points, or of segments of at most `most` points each (runs of `run` places,
-// seg[b] the segment of run b), as o.perm().  keys[0] and keys[1] hold n_pad 32-bit words.
+// seg[b] the segment of run b), as o.perm().  keys[0] and keys[1] hold n_pad 32-bit words.  The
+// merge has as many wavefronts as there are parts of 1024 keys to search, up to 16: more would
+// hold places that other workgroups wait for (4 steps of 2000 simulations of 500 with runs of 256,
+// us: radix passes 1525, 16 wavefronts 1589, one 1189).
 static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, int64_t n_pad,
                       int run, const int* seg, const int64_t* start, const int64_t* count,
-                      hipStream_t s)
+                      int64_t most, hipStream_t s)
 {
-    const dim3 runs((unsigned)(n_pad / run)), blocks((unsigned)(n_pad / 64)), threads(kRunThreads);
-    u32 *keys = o.keys[0].as<u32>(), *from = o.keys[1].as<u32>(), *perm = o.kept ? o.kept : o.idx[0].as<u32>();
-#define GH_RANK(RUN)                                                                          \
-    case RUN:                                                                                 \
-        hipLaunchKernelGGL(k_rank_runs<RUN>, runs, threads, 0, s, d_pos, n, seg, start, count, \
-                           keys, from, perm, o.nflag.as<int>());                              \
-        GH_TRY(check_launch(c, "k_rank_runs"));                                               \
-        hipLaunchKernelGGL((k_run_merge<RUN, kRunThreads / 64, 1, u32>), blocks, threads, 0,  \
-                           s, keys, from, n, seg, start, count, (u32*)nullptr, perm);         \
+    const dim3 runs((unsigned)(n_pad / run)), blocks((unsigned)(n_pad / 64));
+    u32 *keys = o.keys[0].as<u32>(), *from = o.keys[1].as<u32>();
+    u32* const perm = o.kept ? o.kept : o.idx[0].as<u32>();
+    const bool single = most <= run;
+#define GH_MERGE(RUN, WAVES)                                                                   \
+    hipLaunchKernelGGL((k_run_merge<RUN, WAVES, 1, u32>), blocks, dim3(64 * WAVES), 0, s, keys, \
+                       from, n, seg, start, count, (u32*)nullptr, perm)
+#define GH_RANK(RUN)                                                                           \
+    case RUN:                                                                                  \
+        hipLaunchKernelGGL(k_rank_runs<RUN>, runs, dim3(kRunThreads), 0, s, d_pos, n, seg,     \
+                           start, count, keys, from, perm, o.nflag.as<int>(), single);         \
+        GH_TRY(check_launch(c, "k_rank_runs"));                                                \
+        if (single)                                                                            \
+            break;                                                                             \
+        else if (most <= 1024)                                                                 \
+            GH_MERGE(RUN, 1);                                                                  \
+        else if (most <= 4096)                                                                 \
+            GH_MERGE(RUN, 4);                                                                  \
+        else                                                                                   \
+            GH_MERGE(RUN, 16);                                                                 \
         break;
     switch (run) {
         GH_RANK(256)
@@ -169,6 +186,7 @@ static int rank_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, i
     default: return fail(c, GH_EARG, "internal: runs of %d keys", run);
     }
 #undef GH_RANK
+#undef GH_MERGE
     o.sel = 0;
     return check_launch(c, "k_run_merge");
 }
@@ -181,10 +199,12 @@ __global__ __launch_bounds__(kBlock) void k_copy_order(const u32* __restrict__ a
 }
 
 // Every run forms the box of all its segment's points, and every 64 points search all its runs,
-// so the work grows as n^2.  Where this is the faster form, of n places in segments of at most `most` points: a
-// force of 65536 particles took 1058 us with it and 1080 with the radix passes, of 98304 2083
-// and 2089, of 131072 3158 and 3135; a step of 4 simulations of 32768 1.11 ms and 1.22, of 32
-// of 16384 2.19 and 2.20, of 128 of 16384 7.84 and 7.75.
+// so the work grows as n^2.  Where this is the faster form, of n places in segments of at most
+// `most` points: a force of 65536 particles took 1058 us with it and 1080 with the radix passes,
+// of 98304 2083 and 2089, of 131072 3158 and 3135; a step of 4 simulations of 32768 1.11 ms and
+// 1.22, of 32 of 16384 2.19 and 2.20, of 128 of 16384 7.84 and 7.75.  With the passes and with it,
+// four steps of many small ones: 20000 of 20 4.07 and 2.08 ms, 4096 of 250 1.23 and 0.86, 1000
+// of 1024 2.07 and 1.70, 300 of 2500 2.92 and 2.47.
 static bool rank_form(const gh_ctx* c, int64_t n, int64_t most)
 {
     return c->tune[GH_TUNE_SORT_DIRECT] >= 0 && n * most <= (int64_t)1 << 33;
@@ -203,7 +223,7 @@ int spatial_order(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n, hipSt
     GH_TRY(ensure(c, o.nflag, 256));
     if (rank_form(c, n, n)) {
         const int64_t n_pad = (int64_t)blocks_for(n, kRunThreads) * kRunThreads;
-        GH_TRY(rank_order(c, o, d_pos, n, n_pad, kRunThreads, nullptr, nullptr, nullptr, s));
+        GH_TRY(rank_order(c, o, d_pos, n, n_pad, kRunThreads, nullptr, nullptr, nullptr, n, s));
         o.sorted = d_pos;
         o.sorted_n = n;
         return 0;
@@ -315,7 +335,7 @@ int spatial_order_seg(gh_ctx* c, OrderBufs& o, const double* d_pos, int64_t n_pa
     GH_TRY(ensure(c, o.nflag, 256));
     GH_TRY(ensure(c, o.hist, sizeof(u32) * 256 * (size_t)(blocks_for(n_pad, kRsChunk) + 1)));
     if (rank_form(c, n_pad, most))
-        return rank_order(c, o, d_pos, 0, n_pad, blk, seg, start, count, s);
+        return rank_order(c, o, d_pos, 0, n_pad, blk, seg, start, count, most, s);
     hipLaunchKernelGGL(k_seg_box, dim3((unsigned)nseg), dim3(kBlock), 0, s, d_pos, start, count,
                        o.box.as<double>());
     GH_TRY(check_launch(c, "k_seg_box"));

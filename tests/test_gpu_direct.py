@@ -383,3 +383,30 @@ def test_fp64_field_of_few_sources_bitwise(ctx, oracle, n, nf):
     for eps in (0.0, 1e-3):
         assert_bitwise(ctx.direct(pos, mass, eps, FP64, force_pos=fpos),
                        oracle.direct_position(pos, mass, fpos, eps), "eps=%g" % eps)
+
+
+# one run per simulation, and parts of 1024 keys for 1, 4 and 16 wavefronts to search
+@pytest.mark.parametrize("ipt", [1, 2, 4])
+@pytest.mark.parametrize("most", [2, 256, 257, 1024, 1025, 4096, 4097])
+def test_fp32_run_sort_by_largest_segment(ctx, ipt, most):
+    rng = np.random.default_rng(most)
+    sims = []
+    for n in (1, most // 2 + 1, most, min(most, 100)):
+        # a coarse lattice, where many keys are equal, far from FP32 overflow when points coincide
+        sims.append({"pos": rng.integers(0, 9, size=(n, 3)).astype(np.float64),
+                     "vel": rng.normal(size=(n, 3)), "mass": rng.uniform(0.5, 1.0, size=n),
+                     "eps": 0.1, "dt": 1e-4})
+
+    def run(form):
+        ctx.set_tuning(_native.TUNE_SORT_DIRECT, form)
+        try:
+            ens = _native.Ensemble(ctx, sims, ipt=ipt)
+            ens.run(3)
+            state = [np.concatenate(a) for a in ens.state()]
+            ens.close()
+            return state + [ctx.direct(s["pos"], s["mass"], 0.1, FP32) for s in sims]
+        finally:
+            ctx.set_tuning(_native.TUNE_SORT_DIRECT, 0)
+
+    for k, (got, want) in enumerate(zip(run(0), run(-1))):
+        assert_bitwise(got, want, "array %d" % k)
