@@ -2518,9 +2518,10 @@ static int built_ahead(gh_ctx* c, int64_t n, hipStream_t s, bool* good)
 }
 
 template <int T>
-static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4* stgt,
-                            const u32* order, int64_t nt, double eps, double theta, double c_lo,
-                            double c_hi, double* acc, int* counts, hipStream_t s)
+static void launch_walk_f64(const TreeBufs* tb, int64_t np, const double* tgt,
+                            const double4* stgt, const u32* order, int64_t nt, double eps,
+                            double theta, double c_lo, double c_hi, double* acc, int* counts,
+                            hipStream_t s)
 {
 #define GH_WALK64(COUNT, CAP, W)                                                              \
     do {                                                                                      \
@@ -2535,7 +2536,11 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
     // makes steps small, while LDS for it takes walks off the CU.  N = 2^20, 64 targets,
     // walk ms with 448 / 768 / 1024 entries: theta 0.7 1.88 / 2.17 / -, 0.5 5.74 / 4.60 /
     // 5.05, 0.3 - / 18.1 / 15.6 (one node at a time: 2.33, 5.63, 18.7).
-    const int cap = theta >= 0.6 ? 448 : theta >= 0.45 ? 768 : 1024;
+    // The tree of few particles fills less at any theta: 10^6 targets among 300 of them, theta 0.3,
+    // us with 448 / 768 / 1024 / 1536: 436 / 458 / 494 / 535, 100000 among 5000 566 / 582 / 623 /
+    // 628, among 10000 1037 / 804 / 826 / 827, 10^6 among 20000 3780 / 3725 / 3983 / 4381.
+    const int most = stgt || np > 20000 ? 1024 : np > 5000 ? 768 : 448;
+    const int cap = std::min(most, theta >= 0.6 ? 448 : theta >= 0.45 ? 768 : 1024);
     // Where walks are long and their targets far apart, 1024 entries stay full, and a step takes
     // a node or two: the forces of more than 100000 particles at theta < 0.35, and 64 position
     // targets a walk at theta < 0.4.  Ms with 1024 and with kDeepCap (and one node at a time):
@@ -2543,7 +2548,8 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
     // 500000 0.3 10.9 / 8.9 (10.3), 1500000 0.3 30.3 / 25.8 (26.5); 400001 targets among 10^6
     // particles 0.3 26.8 / 14.4 (19.8), 10^6 on a line 11.5 / 12.3 (15.8); 2^20 0.3 16.9 / 17.6
     // (18.9); not taken: N = 100000 0.3 2.30 / 2.42, 500000 0.4 4.43 / 4.72.
-    const bool deep = stgt ? theta < 0.35 && nt > 100000 : T == 64 && theta < 0.4;
+    const bool deep = stgt ? theta < 0.35 && nt > 100000
+                           : T == 64 && theta < 0.4 && np > 20000;
     // One wavefront per workgroup where the 16 workgroups of a CU are as many walks as its
     // registers hold (64 targets, 448 entries), or where all walks are on the chip at once: a
     // workgroup of two holds the place of the one that ends first.  Us with two and with one:
@@ -2571,15 +2577,15 @@ static void launch_walk_f64(const TreeBufs* tb, const double* tgt, const double4
 #undef GH_WALK64
 }
 
-// Walks nt targets through the tree built last: the particles themselves (self) or the
-// positions tgt.  Targets are walked in octant-path (Morton) order, so that neighbouring
+// Walks nt targets through the tree of np particles built last: the particles themselves (self) or
+// the positions tgt.  Targets are walked in octant-path (Morton) order, so that neighbouring
 // lanes take neighbouring targets and a wavefront's paths through the tree nearly
 // coincide: self targets in the particles' sorted order, kSortTargetsMin or more
 // position targets in an order sorted here by the top 40 key bits (13 levels of the
 // particles' root box; targets outside the box fall in its edge cells).  Results are
 // written in the caller's order.
-static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps, double theta,
-                int precision, double* d_acc, int* counts, hipStream_t s)
+static int walk(gh_ctx* c, int64_t np, const double* tgt, bool self, int64_t nt, double eps,
+                double theta, int precision, double* d_acc, int* counts, hipStream_t s)
 {
     TreeBufs* tb = c->tree;
     if (nt <= 0) return 0;
@@ -2630,14 +2636,18 @@ static int walk(gh_ctx* c, const double* tgt, bool self, int64_t nt, double eps,
             if (nt > (theta < 0.35 ? 150000 : 200000)) T = 64;
         } else if (order) {
             while (T < 16 && nt > T * 20000) T *= 2;
-            if (nt > 400000) T = 64;
+            // (among few particles the walks of 64 are short: 300000 targets among 300, theta
+            // 0.3 and 0.7, 16 and 64 to a walk: 327 and 258, 264 and 218 us; 200000 among 700 317
+            // and 317, 242 and 242; 300000 among 3000 777 and 845, 379 and 377)
+            if (nt > (np <= 2000 ? 200000 : 400000)) T = 64;
         }
         const double inf = __builtin_huge_val();
         const double c_lo = theta > 0.0 ? (1.0 - 1e-13) / (theta * theta) : inf;
         const double c_hi = theta > 0.0 ? (1.0 + 1e-13) / (theta * theta) : inf;
 #define GH_WALK64(T)                                                                           \
     case T:                                                                                    \
-        launch_walk_f64<T>(tb, tgt, stgt, order, nt, eps, theta, c_lo, c_hi, d_acc, counts, s); \
+        launch_walk_f64<T>(tb, np, tgt, stgt, order, nt, eps, theta, c_lo, c_hi, d_acc, counts, \
+                           s);                                                                 \
         break
         switch (T) {
             GH_WALK64(1);
@@ -2705,13 +2715,13 @@ int tree_dev(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
     const double* tgt = self ? d_pos : d_fpos;
     bool pending = false, good = false;
     int rc = build_tree(c, d_pos, d_mass, np, eps, theta, what, s, &pending);
-    if (!rc) rc = walk(c, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
+    if (!rc) rc = walk(c, np, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
     if (!pending) return rc;
     const int seen = built_ahead(c, np, s, &good);  // also after an error: its words are written
     if (rc || seen) return rc ? rc : seen;
     if (good) return 0;
     GH_TRY(build_tree(c, d_pos, d_mass, np, eps, theta, what, s));
-    return walk(c, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
+    return walk(c, np, tgt, self, nt, eps, theta, precision, d_acc, nullptr, s);
 }
 
 void tree_free(gh_ctx* c)
@@ -2812,7 +2822,7 @@ static int tree_counts(gh_ctx* c, const double* pos, const double* mass, int64_t
     }
     GH_TRY(build_tree(c, c->pos64.as<double>(), c->mass64.as<double>(), np, eps, theta,
                       kFillKids | (precision == GH_FP64 ? kFillF64 : kFillW), s));
-    GH_TRY(walk(c, tgt, self, nt, eps, theta, precision, c->acc64.as<double>(),
+    GH_TRY(walk(c, np, tgt, self, nt, eps, theta, precision, c->acc64.as<double>(),
                 c->scratch.as<int>(), s));
     std::vector<int> cnt((size_t)(nt > 0 ? nt : 1));
     GH_HIP(c, hipMemcpyAsync(acc, c->acc64.p, sizeof(double) * 3 * (size_t)nt,

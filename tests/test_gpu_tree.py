@@ -590,3 +590,19 @@ def test_fp64_walk_deep_same_bits(ctx, n, nf, theta):
     some = rng.permutation(len(tgt))[:400]
     full = ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=fpos)
     assert_bitwise(full[some], ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=tgt[some]))
+
+
+# fields of few particles: targets per walk and stack entries go by their number
+@pytest.mark.parametrize("n,nf", [(2, 200001), (2000, 200000), (2000, 200001), (2001, 200001),
+                                  (5000, 30000), (5001, 30000), (20000, 400001), (20001, 400001)])
+def test_fp64_walk_few_particles_same_bits(ctx, n, nf):
+    rng = np.random.default_rng(n + nf)
+    pos = rng.normal(size=(n, 3)) * np.exp(rng.normal(size=(n, 1)))
+    mass = rng.uniform(0.5, 2.0, size=n)
+    fpos = rng.normal(size=(nf, 3))
+    fpos[::40] = pos[rng.integers(0, n, size=len(fpos[::40]))]
+    some = rng.permutation(nf)[:400]
+    for theta in (0.7, 0.3, 0.0 if n <= 2001 else 0.1):
+        full = ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=fpos)
+        assert_bitwise(full[some], ctx.tree(pos, mass, 0.01, theta, FP64, force_pos=fpos[some]),
+                       "theta=%g" % theta)
