@@ -327,3 +327,44 @@ def test_ensemble_state_without_padding(ctx, counts):
     for k, s in enumerate(sims):
         assert_bitwise(pos[k], s["pos"], "positions of %d" % k)
         assert_bitwise(vel[k], s["vel"], "velocities of %d" % k)
+
+
+# FP64 on both sides of the last size whose force kernel applies the update (two buffers of
+# half-step positions in turn); 101 steps are 13 slices of the history, the last of five
+@pytest.mark.parametrize("prec,n,nsteps", [(_native.GH_FP64, 1500, 8), (_native.GH_FP64, 3000, 101),
+                                           (_native.GH_FP64, 6500, 17), (_native.GH_FP64, 6501, 17),
+                                           (_native.GH_FP32, 3000, 101), (_native.GH_FP32, 20000, 9)])
+def test_direct_run_equals_chained_steps(ctx, prec, n, nsteps):
+    # every snapshot and the final state are those of runs of one step, each from the last's
+    ic = workloads.plummer(n, seed=n + nsteps)
+    args = (ic["mass"], 0.002, 2e-5)
+    x, v, hp, hv = ctx.run(ic["pos"], ic["vel"], *args, nsteps, precision=prec, history=True)
+    xc, vc = ic["pos"], ic["vel"]
+    for k in range(nsteps):
+        xc, vc = ctx.run(xc, vc, *args, 1, precision=prec)
+        assert_bitwise(hp[k], xc, "position of step %d" % k)
+        assert_bitwise(hv[k], vc, "velocity of step %d" % k)
+    assert_bitwise(x, xc)
+    assert_bitwise(v, vc)
+
+
+@pytest.mark.parametrize("drained", [0, -1])
+@pytest.mark.parametrize("prec,n", [(_native.GH_FP64, 700), (_native.GH_FP32, 5000)])
+def test_run_dev_drained_or_queued(ctx, prec, n, drained):
+    # whether the call waits for its steps or returns once they are queued: the same run,
+    # ordered before what the caller queues behind it
+    torch = pytest.importorskip("torch")
+    ic = workloads.plummer(n, seed=n)
+    want = ctx.run(ic["pos"], ic["vel"], ic["mass"], 0.002, 2e-5, 6, precision=prec)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        x, v, m = (torch.tensor(ic[k], device="cuda") for k in ("pos", "vel", "mass"))
+        ctx.set_tuning(_native.TUNE_RUN_GRAPH, drained)
+        try:
+            ctx.run_dev(x.data_ptr(), v.data_ptr(), m.data_ptr(), n, 0.002, 2e-5, 6,
+                        precision=prec, stream=stream.cuda_stream)
+        finally:
+            ctx.set_tuning(_native.TUNE_RUN_GRAPH, 0)
+        got = torch.stack([x, v])
+    stream.synchronize()
+    assert_bitwise(got.cpu().numpy(), np.stack(want))
