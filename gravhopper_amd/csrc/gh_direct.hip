@@ -16,7 +16,7 @@
 //  k_direct_sym_f32  the self field with each unordered pair computed once.
 //  Both FP32 kernels form coordinates only relative to FP64 origins of groups of
 //  spatially sorted particles (gh_frames.hip), so their accuracy does not depend on
-//  where the system sits; non-compact groups take double-single instances.
+//  where the system sits; non-compact groups take double-single forms.
 #include <cmath>
 #include <type_traits>
 
@@ -454,7 +454,7 @@ static bool f64_few(const gh_ctx* c, int64_t np, int64_t nt)
 // along a Morton curve, each block of consecutive sorted particles has an FP64 origin,
 // and a kernel forms its FP32 coordinates relative to one block's origin from FP64
 // values.  Blocks whose flag is set (not compact) are handled by the double-single
-// (DS) instances, which carry every coordinate as hi + lo FP32 words of an FP64
+// (DS) forms, which carry every coordinate as hi + lo FP32 words of an FP64
 // difference and form separations as (hi_j - hi_i) + (lo_j - lo_i).
 __device__ __forceinline__ void two_sum_into(float& hi, float& lo, float t)
 {
@@ -622,9 +622,8 @@ __global__ __launch_bounds__(kBlock) void k_direct_f32(const double4* __restrict
 // after 64 steps lane l holds the whole wavefront's force on j = l.  The four
 // wavefronts' j-partials are added in LDS.  A diagonal pair I = J is done one-sided.
 // The workgroup works in block I's frame: i-particles are block I's local coordinates,
-// block J's enter as fl(loc_J + fl(o_J - o_I)).  Pairs with a flagged block are left to
-// the DS instance, which stages both sides as hi + lo words of the FP64 differences
-// from o_I.
+// block J's enter as fl(loc_J + fl(o_J - o_I)).  Pairs with a flagged block take the DS form in
+// the same launch, which stages both sides as hi + lo words of the FP64 differences from o_I.
 //
 // Results are partial fields part[K][p] (FP32, 3 per particle): particle p of block B
 // receives one partial from every block K (K = B for its diagonal); k_reduce_sym adds
@@ -828,10 +827,11 @@ __device__ __forceinline__ void sym_item(const float4* __restrict__ src,
 //    blocks are flagged, and 4.6 us where no block is.)
 //  - Items whose blocks each have one mass (umass, not NaN) take the UNI form in simulations
 //    of at least kUniMin particles (nb_blk[b] or, where it is null, nb blocks), unless the
-//    guard is needed, which bounds the factors with their masses.  Measured (N = 262144,
-//    equal masses, per launch): 13.33 -> 11.98 ms.  Below kUniMin the sort, the reduction
-//    and the launches are a growing share of a step (N = 16384: 2 % of a gradient gained),
-//    and results keep the bits of the general form.
+//    guard is needed, which bounds the factors with their masses.  Systems of unequal masses
+//    gain nothing.  Measured (N = 262144, equal masses, per launch): 13.33 -> 11.98 ms.  Below
+//    kUniMin results keep the bits of the general form, though there is as much to gain (us a
+//    force: N = 16384 109 -> 104, 32768 319 -> 288, 65536 1029 -> 931, 98304 2083 -> 1874): the
+//    sums are rounded elsewhere, and four steps move the velocities by up to 1e-7.
 //  - Registers for six wavefronts per SIMD where a lane has one particle and five otherwise,
 //    as LDS allows: N = 16384 118 -> 113 us a call, 32768 334 -> 319 (four lose 3 % at 65536
 //    and beyond).  Padding left out: 128 spheres of 1024 to 65536 15.0 -> 14.6 ms a step.

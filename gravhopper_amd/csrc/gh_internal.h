@@ -234,8 +234,10 @@ int direct_sym(gh_ctx* c, const double* d_pos, const double* d_mass, int64_t np,
                double eps, double* d_acc, hipStream_t s, const StepUpdate* up = nullptr,
                bool* updated = nullptr);
 // The pair-once kernel over a block-pair list (src: local FP32 coordinates per sorted
-// particle, s64: the same particles in FP64, frame/flag/umass/used: per block), followed by its
-// double-single instance for the items with a flagged block.
+// particle, s64: the same particles in FP64, frame/flag/umass/used: per block), the items with
+// a flagged block in their double-single form.  nflag (read with a queue only): whether a
+// persistent launch takes those items first; 0 or not, every item is evaluated once, but with
+// flags set a 0 leaves them in the order of the list, and it may be nonzero without any.
 // jpart (nullable): the j-side partials go to jpart[slot_j][p - joff] with a stride of
 // jstride particles instead of part.
 int launch_sym(gh_ctx* c, int ipt, bool guard, const float4* src, const double4* s64,

@@ -865,7 +865,7 @@ struct FillArgs {
 };
 
 constexpr int kFillF64 = 1;   // NodeD + leaf flags (FP64 walk, dump)
-constexpr int kFillKids = 2;  // children lists (FP32 group walk)
+constexpr int kFillKids = 2;  // children lists (both walks)
 constexpr int kFillDump = 4;  // levels and branches (canonical dump)
 constexpr int kFillW = 8;     // NodeW records (FP32 group walk)
 
@@ -2198,8 +2198,7 @@ int radix_sort(gh_ctx* c, DevBuf* keys, DevBuf* idx, DevBuf& hist, int64_t n, in
     return 0;
 }
 
-// Root box of the reference (centre box[0..2], size box[3], gravhopper/_jbgrav.c:747-772)
-// of n points, written to the device array box; part holds the partial extents.
+// Extents of n points per workgroup into part, *nparts of them.
 static int bbox_parts_dev(gh_ctx* c, const double* d_pos, int64_t n, DevBuf& part, hipStream_t s,
                           int* nparts)
 {
@@ -2210,6 +2209,8 @@ static int bbox_parts_dev(gh_ctx* c, const double* d_pos, int64_t n, DevBuf& par
     return check_launch(c, "k_bbox_partial");
 }
 
+// Root box of the reference (centre box[0..2], size box[3], gravhopper/_jbgrav.c:747-772)
+// of n points, written to the device array box; part holds the partial extents.
 int bbox_dev(gh_ctx* c, const double* d_pos, int64_t n, double eps, DevBuf& part, double* box,
              hipStream_t s)
 {
@@ -2628,8 +2629,17 @@ static int walk(gh_ctx* c, int64_t np, const double* tgt, bool self, int64_t nt,
         //   16            69    86    116    135     406     750   2665
         //   64           166   214    325    301     456     687   1883
         //   before       144   233    408    448     682     894   2331
-        // and of 20011 targets among 300007 particles with T = 1, 4, 16, 64: 227, 205, 413
-        // and 1426 us (before 772).
+        // Position targets among 10^6 particles (force, us, theta = 0.7), in the volume of the
+        // galaxy and on a plane through it:
+        //   targets    20000       40000       100000       200000       400000       10^6
+        //   T = 1     490   563   647  791   1101  1439
+        //   2         461   503   582  651    889  1045   1375  1682   2211  2815
+        //   4         462   486   554  584    786   869   1110  1274   1719  2055   3475  4322
+        //   8         555   511   601  570    718   733    934   984   1313  1432   2460  2794
+        //   16        657   703   718  673    818   729    967   889   1274  1192   2023  2124
+        //   64       2591  4485  3466 3119   2855  2273   3291  1464   2971  1311   2958  1601
+        // On a line, whose neighbours are closest, 64 lead from 100000 on (606 and 531 us with
+        // 16 and 64, 400000 1167 and 800, 10^6 2313 and 1304): 64 from between the two on.
         int T = 1;
         if (self) {
             while (T < 16 && nt > T * kWalks64) T *= 2;
@@ -2644,20 +2654,20 @@ static int walk(gh_ctx* c, int64_t np, const double* tgt, bool self, int64_t nt,
         const double inf = __builtin_huge_val();
         const double c_lo = theta > 0.0 ? (1.0 - 1e-13) / (theta * theta) : inf;
         const double c_hi = theta > 0.0 ? (1.0 + 1e-13) / (theta * theta) : inf;
-#define GH_WALK64(T)                                                                           \
+#define GH_WALK64_T(T)                                                                         \
     case T:                                                                                    \
         launch_walk_f64<T>(tb, np, tgt, stgt, order, nt, eps, theta, c_lo, c_hi, d_acc, counts, \
                            s);                                                                 \
         break
         switch (T) {
-            GH_WALK64(1);
-            GH_WALK64(2);
-            GH_WALK64(4);
-            GH_WALK64(8);
-            GH_WALK64(16);
-            GH_WALK64(64);
+            GH_WALK64_T(1);
+            GH_WALK64_T(2);
+            GH_WALK64_T(4);
+            GH_WALK64_T(8);
+            GH_WALK64_T(16);
+            GH_WALK64_T(64);
         }
-#undef GH_WALK64
+#undef GH_WALK64_T
         return check_launch(c, "k_walk_f64");
     }
     // FP32: the group walk, 16 targets per wavefront, or one target per wavefront when
