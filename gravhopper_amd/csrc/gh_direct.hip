@@ -7,7 +7,8 @@
 //                 gh_pairf64.h, correctly rounded like the compiler's division and square
 //                 root.  The terms are computed by many wavefronts and added in order by
 //                 one: a wavefront of its own (relay, few targets) or each in its turn
-//                 (ring).
+//                 (ring).  k_direct_f64_few, the fields of few sources: the same sums, one
+//                 target per lane.
 //  k_direct_f32   FP32 pair forces with v_rsq_f32, IPT targets per lane, 256-source
 //                 tiles staged in LDS as float4 (x, y, z, m) and read as wave-wide
 //                 broadcasts, FP32 sums per tile and an FP32 two-sum (hi, lo) across
@@ -334,8 +335,10 @@ __global__ __launch_bounds__(W * 64) void k_direct_f64_ring(const double* __rest
     }
 }
 
-// The field of few sources: one target per lane, the sources one after the other and four factors
-// at a time.
+// The field of few sources: one target per lane, the sources one after the other, whose records
+// are the same for all and arrive through scalar loads, and four factors at a time.  Nothing is
+// shared, so a workgroup is as long as its sums: bound by HBM for up to 4 sources (10^6 targets in
+// 12 us, 48 MB), by the FP64 issue rate beyond (50 sources 71 us).
 __global__ __launch_bounds__(kBlock) void k_direct_f64_few(const double* __restrict__ pos,
                                                            const double* __restrict__ mass, int np,
                                                            const double* __restrict__ tgt,
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(kBlock) void k_direct_f64_few(const double* __restr
 // division and square root):
 //   N        500  1000  2000  4000  6000 | 8000  12000  16384  20000  32768  65536  100003  262144
 //   relay    7.3  10.0  17.9  41.2  80.7 |  141    289    529    817   2063
-//   ring                      60.6  86.0 |  111    293    398    723   1509   5817   14040   90900
+//   ring                      60.6  86.0 |  110    287    389    656   1518   6000   14460   91900
 //   before   9.2  14.7  29.7  78.5   169 |  241    483   1017   1399   3589  13545   30155  142460
 // 3001 targets of 65536 sources: 455 (before 1300); 200 of 100000: 393 (1062).
 // Few sources are a chunk of the relay at most, whose many small workgroups then cost more than
